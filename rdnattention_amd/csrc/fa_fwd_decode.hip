@@ -9,11 +9,16 @@
 //   * grid = (splits, B * Hkv); a workgroup owns one contiguous key range of
 //     one kv head and all M = (Hq/Hkv) * Sq query rows of that head group,
 //     packed as the 32 columns of one MFMA block (M <= 32)
-//   * its 4 waves work independently on interleaved 32-key tiles: each wave
-//     streams K and V with buffer_load ... lds (HBM -> LDS, no VGPR staging),
-//     non-temporal since every byte is read once, into its own
-//     double-buffered LDS slice, two tiles in flight, no workgroup barriers in
-//     the loop
+//   * its waves (eight up to D = 160) work independently on interleaved
+//     32-key tiles: each streams K and V with buffer_load ... lds (HBM -> LDS,
+//     no VGPR staging), non-temporal since every byte is read once, into its
+//     own K and V slots; K(j + 1) leaves as soon as S(j) has read K(j), V(j +
+//     1) after P V(j), so one of the two is always in flight; no workgroup
+//     barriers in the loop
+//     (B = 8 Hq = 16 Hkv = 8 Sk = 6001 D = 256, 393 MB: 65 us, 6.1 TB/s; the
+//     prefill kernel, one row of 128 in use, 183 us; two waves with two slots
+//     each of K and V, 111 us: a wave spends ~80 cycles issuing each 1 KB DMA,
+//     so more waves, not deeper slots, keep the bytes coming)
 //   * LDS rows are stored with an XOR swizzle of their 16-byte chunks so the
 //     ds_read_b128 of K (16 rows) and the ds_read_b64_tr_b16 of V (4 rows x
 //     32 B) both hit distinct banks although the DMA writes rows unpadded
@@ -23,9 +28,11 @@
 #include "fa_common.hpp"
 #include "fa_host.hpp"
 #include "fa_internal.hpp"
+#include "fa_splitk.hpp"
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace rdna_amd {
 
@@ -33,23 +40,24 @@ float softmax_log2_scale(float scale);
 
 namespace {
 
-constexpr int kDecWaves = 4;
-constexpr int kDecThreads = 64 * kDecWaves;
-constexpr int kDecTile = 32;              // keys per wave tile
+constexpr int kDecTile = 32; // keys per wave tile
 constexpr float kDecRescaleThreshold = 8.0f;
 
 struct DecodeParams {
     const _Float16* q;
     const _Float16* k;
     const _Float16* v;
+    _Float16* o;
     const float* rot_cos;
     const float* rot_sin;
     int64_t q_sb, q_sh, q_ss;
     int64_t k_sb, k_sh, k_ss;
     int64_t v_sb, v_sh, v_ss;
-    float* part_o;  // [B*Hkv][splits][M][D] unnormalised O
+    int64_t o_sb, o_sh, o_ss;
+    float* part_o;  // [B*Hkv][splits][M][D] unnormalised O (splits > 1)
     float* part_ml; // [B*Hkv][splits][M][2]  (m in log2 units, l)
     int32_t Sq, Hkv, ratio, M, splits, keys_per_split;
+    int32_t key0; // first key of split 0
     float c;
     float q_sign;
     MaskSpec mask;
@@ -58,23 +66,34 @@ struct DecodeParams {
 
 template <int D>
 struct DecCfg {
+    // LDS holds one K and one V tile per wave, 128 D bytes: eight waves up to
+    // D = 160 (160 KB there), six at 192 (144 KB), four above (128 KB at 256;
+    // one wave per SIMD, whose O alone takes 128 registers)
+    static constexpr int WAVES = D <= 160 ? 8 : (D <= 192 ? 6 : 4);
+    static constexpr int THREADS = 64 * WAVES;
     static constexpr int RB = 2 * D;                 // row bytes (unpadded)
     static constexpr int KCH = D / 8;                // 16-byte chunks per row
     static constexpr int TILE_BYTES = kDecTile * RB; // one K (or V) tile
-    static constexpr int SLOT_BYTES = 2 * TILE_BYTES;
-    static constexpr int WAVE_BYTES = 2 * SLOT_BYTES; // double-buffered
+    static constexpr int WAVE_BYTES = 2 * TILE_BYTES;
     static constexpr int NS = D / 16;
     static constexpr int NDT = D / 32;
     static constexpr int DMA_PER_TILE = TILE_BYTES / 1024; // 1 KB per wave-wide DMA
-    static constexpr int ROWS_PER_DMA = 1024 / RB;
+    static constexpr int LDM = D + 4;                      // floats per merged row (conflict-free b128)
+    static_assert(WAVES * WAVE_BYTES <= 160 * 1024, "K/V tiles fit the LDS");
+    static constexpr int MERGE = WAVES / 2; // waves whose O is in LDS at once
+    static_assert((MERGE * 32 * LDM + WAVES * 32 * 2) * 4 <= WAVES * WAVE_BYTES, "the merge reuses the tile area");
 };
 
 // XOR swizzle of the 16-byte chunk index of row r (see the file comment).
+// Rows are 2 D bytes and the 64 banks 256 B: rows r and r + 4 (D % 64 = 32),
+// r + 2 (D % 128 = 64) or r + 1 (D % 128 = 0) start in the same bank, so that
+// many chunk positions spread them: XOR within groups of 4, 8 or 16 chunks
+// (each divides D / 8).
 template <int D>
 __device__ __forceinline__ int dec_swz(int r) {
-    if constexpr (D == 32) {
+    if constexpr (D % 64 == 32) {
         return (r >> 2) & 3;
-    } else if constexpr (D == 64) {
+    } else if constexpr (D % 128 == 64) {
         return (((r >> 1) & 3) << 1) | ((r >> 3) & 1);
     } else {
         return ((r & 7) << 1) | ((r >> 3) & 1);
@@ -82,9 +101,9 @@ __device__ __forceinline__ int dec_swz(int r) {
 }
 
 template <int D>
-__global__ __launch_bounds__(kDecThreads, 1) void fa_fwd_f16_decode(DecodeParams p) {
+__global__ __launch_bounds__(DecCfg<D>::THREADS, 1) void fa_fwd_f16_decode(DecodeParams p) {
     using C = DecCfg<D>;
-    __shared__ __attribute__((aligned(16))) char dsm[kDecWaves * C::WAVE_BYTES];
+    __shared__ __attribute__((aligned(16))) char dsm[C::WAVES * C::WAVE_BYTES];
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6); // wave-uniform
@@ -102,6 +121,64 @@ __global__ __launch_bounds__(kDecThreads, 1) void fa_fwd_f16_decode(DecodeParams
     const int q = col_valid ? l32 - hoff * p.Sq : 0;
     const int h = kvh * p.ratio + hoff;
 
+    // this split's key range, restricted to what any of the M rows can see
+    const int k_begin = p.key0 + split * p.keys_per_split;
+    const int k_end = min(k_begin + p.keys_per_split, p.mask.sk);
+    int vis_lo, vis_hi;
+    visible_key_range(p.mask, 0, p.Sq - 1, vis_lo, vis_hi);
+    const int lo = max(k_begin, vis_lo);
+    const int hi = min(k_end - 1, vis_hi);
+    int t0 = 0, nt = 0; // tiles of this wave: kt = t0 + wave + WAVES * j
+    if (hi >= lo) {
+        t0 = lo / kDecTile;
+        nt = hi / kDecTile + 1 - t0;
+    }
+    const int my_tiles = nt > wave ? (nt - wave + C::WAVES - 1) / C::WAVES : 0;
+
+    const _Float16* kbase = p.k + b * p.k_sb + kvh * p.k_sh;
+    const _Float16* vbase = p.v + b * p.v_sb + kvh * p.v_sh;
+    char* wsm = dsm + wave * C::WAVE_BYTES;
+
+    // DMA source offsets: lane i of DMA j writes LDS bytes 1024 j + 16 i of the
+    // tile, i.e. stored chunk n % KCH of row r = n / KCH with n = 64 j + i,
+    // which holds logical chunk (n % KCH) ^ swz(r)
+    uint32_t kdo[C::DMA_PER_TILE], vdo[C::DMA_PER_TILE];
+#pragma unroll
+    for (int j = 0; j < C::DMA_PER_TILE; j++) {
+        const int n = 64 * j + lane;
+        const int r = n / C::KCH;
+        const int cl = (n - r * C::KCH) ^ dec_swz<D>(r);
+        kdo[j] = (uint32_t)(((int64_t)r * p.k_ss + 8 * cl) * 2);
+        vdo[j] = (uint32_t)(((int64_t)r * p.v_ss + 8 * cl) * 2);
+    }
+    const uint32_t lds_k = (uint32_t)reinterpret_cast<uintptr_t>(wsm);
+    const uint32_t lds_v = lds_k + C::TILE_BYTES;
+    auto issue_k = [&](int j_tile) {
+        const int kt0 = (t0 + wave + C::WAVES * j_tile) * kDecTile;
+        const i32x4_t r = make_rsrc_v(kbase + (int64_t)kt0 * p.k_ss,
+                                      tile_bytes<kDecTile>(p.mask.sk - kt0, (uint32_t)(p.k_ss * 2), D * 2));
+#pragma unroll
+        for (int j = 0; j < C::DMA_PER_TILE; j++) {
+            dma_load16_nt(r, kdo[j], lds_k + 1024 * j);
+        }
+    };
+    auto issue_v = [&](int j_tile) {
+        const int kt0 = (t0 + wave + C::WAVES * j_tile) * kDecTile;
+        const i32x4_t r = make_rsrc_v(vbase + (int64_t)kt0 * p.v_ss,
+                                      tile_bytes<kDecTile>(p.mask.sk - kt0, (uint32_t)(p.v_ss * 2), D * 2));
+#pragma unroll
+        for (int j = 0; j < C::DMA_PER_TILE; j++) {
+            dma_load16_nt(r, vdo[j], lds_v + 1024 * j);
+        }
+    };
+
+    // The first tiles leave before the Q loads, so that a short key range
+    // costs one memory round trip and not two; the wait for Q drains them too
+    // (the compiler's vmcnt waits do not count the DMAs), once.
+    if (my_tiles > 0) {
+        issue_k(0);
+        issue_v(0);
+    }
     h8 qreg[C::NS];
     {
         const int qr = q; // 0 for an unused column
@@ -109,8 +186,6 @@ __global__ __launch_bounds__(kDecThreads, 1) void fa_fwd_f16_decode(DecodeParams
         load_q_operand(qreg, qrow, p.rot_cos + (int64_t)qr * (D / 2), p.rot_sin + (int64_t)qr * (D / 2), g, col_valid,
                        p.rope_q != 0, p.q_sign < 0.0f);
     }
-    // Q is in registers before any DMA is issued, so no later wait for it can
-    // drain the DMA queue (the compiler does not see the DMAs)
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     int row_lo, row_hi;
     row_key_bounds(p.mask, q, row_lo, row_hi);
@@ -119,52 +194,6 @@ __global__ __launch_bounds__(kDecThreads, 1) void fa_fwd_f16_decode(DecodeParams
         row_hi = 0; // sees nothing
     }
 
-    // this split's key range, restricted to what any of the M rows can see
-    const int k_begin = split * p.keys_per_split;
-    const int k_end = min(k_begin + p.keys_per_split, p.mask.sk);
-    int vis_lo, vis_hi;
-    visible_key_range(p.mask, 0, p.Sq - 1, vis_lo, vis_hi);
-    const int lo = max(k_begin, vis_lo);
-    const int hi = min(k_end - 1, vis_hi);
-    int t0 = 0, nt = 0; // tiles of this wave: kt = t0 + wave + 4 * j
-    if (hi >= lo) {
-        t0 = lo / kDecTile;
-        nt = hi / kDecTile + 1 - t0;
-    }
-    const int my_tiles = nt > wave ? (nt - wave + kDecWaves - 1) / kDecWaves : 0;
-
-    const _Float16* kbase = p.k + b * p.k_sb + kvh * p.k_sh;
-    const _Float16* vbase = p.v + b * p.v_sb + kvh * p.v_sh;
-    char* wsm = dsm + wave * C::WAVE_BYTES;
-
-    // DMA source offsets: lane i of DMA j writes LDS bytes 1024 j + 16 i of the
-    // tile, i.e. row r = j * ROWS_PER_DMA + i / KCH, stored chunk i % KCH,
-    // which holds logical chunk (i % KCH) ^ swz(r)
-    uint32_t kdo[C::DMA_PER_TILE], vdo[C::DMA_PER_TILE];
-#pragma unroll
-    for (int j = 0; j < C::DMA_PER_TILE; j++) {
-        const int r = j * C::ROWS_PER_DMA + lane / C::KCH;
-        const int cs = lane % C::KCH;
-        const int cl = cs ^ dec_swz<D>(r);
-        kdo[j] = (uint32_t)(((int64_t)r * p.k_ss + 8 * cl) * 2);
-        vdo[j] = (uint32_t)(((int64_t)r * p.v_ss + 8 * cl) * 2);
-    }
-    auto issue_tile = [&](int j_tile, int slot) {
-        const int kt0 = (t0 + wave + kDecWaves * j_tile) * kDecTile;
-        const i32x4_t rk = make_rsrc_v(kbase + (int64_t)kt0 * p.k_ss, tile_bytes<kDecTile>(p.mask.sk - kt0, (uint32_t)(p.k_ss * 2), D * 2));
-        const i32x4_t rv = make_rsrc_v(vbase + (int64_t)kt0 * p.v_ss, tile_bytes<kDecTile>(p.mask.sk - kt0, (uint32_t)(p.v_ss * 2), D * 2));
-        const uint32_t sk = (uint32_t)reinterpret_cast<uintptr_t>(wsm + slot * C::SLOT_BYTES);
-        const uint32_t sv = sk + C::TILE_BYTES;
-#pragma unroll
-        for (int j = 0; j < C::DMA_PER_TILE; j++) {
-            dma_load16_nt(rk, kdo[j], sk + 1024 * j);
-        }
-#pragma unroll
-        for (int j = 0; j < C::DMA_PER_TILE; j++) {
-            dma_load16_nt(rv, vdo[j], sv + 1024 * j);
-        }
-    };
-
     f16x oacc[C::NDT];
 #pragma unroll
     for (int dt = 0; dt < C::NDT; dt++) {
@@ -172,23 +201,13 @@ __global__ __launch_bounds__(kDecThreads, 1) void fa_fwd_f16_decode(DecodeParams
     }
     float m_run = -INFINITY, l_run = 0.0f;
 
-    if (my_tiles > 0) {
-        issue_tile(0, 0);
-    }
-    if (my_tiles > 1) {
-        issue_tile(1, 1);
-    }
     for (int j = 0; j < my_tiles; j++) {
-        const int slot = j & 1;
-        // tile j landed: at most one tile's DMAs (tile j+1) still outstanding
-        if (j + 1 < my_tiles) {
-            __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * C::DMA_PER_TILE));
-        } else {
-            __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-        }
-        const int kt0 = (t0 + wave + kDecWaves * j) * kDecTile;
-        const char* sk = wsm + slot * C::SLOT_BYTES;
-        const char* sv = sk + C::TILE_BYTES;
+        // K(j) landed: only V(j)'s DMAs, issued after it, may be outstanding
+        // (the first two tiles were awaited with Q)
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(C::DMA_PER_TILE));
+        const int kt0 = (t0 + wave + C::WAVES * j) * kDecTile;
+        const char* sk = wsm;
+        const char* sv = wsm + C::TILE_BYTES;
 
         // S^T[key][col] = K Q^T over one 32-key tile
         f16x sacc = {};
@@ -202,6 +221,11 @@ __global__ __launch_bounds__(kDecThreads, 1) void fa_fwd_f16_decode(DecodeParams
                 h8 a = *reinterpret_cast<const h8*>(krow + ((cl ^ sw) << 4));
                 sacc = mfma_32x32x16_f16(a, qreg[s], sacc);
             }
+        }
+        const bool more = j + 1 < my_tiles;
+        if (more) {
+            __builtin_amdgcn_s_waitcnt(waitcnt_lgkm(0)); // every read of K(j) has returned
+            issue_k(j + 1);
         }
         // mask (only where a tile crosses a row's visible range; cheap anyway)
         {
@@ -239,6 +263,12 @@ __global__ __launch_bounds__(kDecThreads, 1) void fa_fwd_f16_decode(DecodeParams
         }
         l_run += (ps[0] + ps[1]) + (ps[2] + ps[3]);
 
+        // V(j) landed: only K(j + 1)'s DMAs are younger
+        if (more) {
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(C::DMA_PER_TILE));
+        } else {
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        }
         // O^T += V^T P^T; V^T operand through transpose reads
         {
             const int j16 = lane & 15;
@@ -260,70 +290,104 @@ __global__ __launch_bounds__(kDecThreads, 1) void fa_fwd_f16_decode(DecodeParams
                 }
             }
         }
-        // every LDS read of this slot has returned before the next DMA lands in it
-        if (j + 2 < my_tiles) {
-            __builtin_amdgcn_s_waitcnt(waitcnt_lgkm(0));
-            issue_tile(j + 2, slot);
+        if (more) {
+            __builtin_amdgcn_s_waitcnt(waitcnt_lgkm(0)); // every read of V(j) has returned
+            issue_v(j + 1);
         }
     }
     __builtin_amdgcn_s_waitcnt(0); // all DMAs and LDS traffic of this wave done
     __syncthreads();
 
-    // ---- merge the 4 waves in LDS (reusing the tile buffers)
-    float* sm_ml = reinterpret_cast<float*>(dsm);                 // [4][32][2]
-    float* sm_o = reinterpret_cast<float*>(dsm + 4 * 32 * 2 * 4); // [4][D][32]
+    // ---- merge the waves in LDS (reusing the tile buffers)
+    float* sm_o = reinterpret_cast<float*>(dsm);            // [MERGE][32][LDM]
+    float* sm_ml = sm_o + C::MERGE * 32 * C::LDM;           // [WAVES][32][2]
     const float l_tot = pair_sum(l_run);
     if (g == 0) {
         sm_ml[(wave * 32 + l32) * 2 + 0] = m_run;
         sm_ml[(wave * 32 + l32) * 2 + 1] = l_tot;
     }
     __syncthreads();
-    float mref = -INFINITY;
+    float mref = -INFINITY, lsum = 0.0f; // of column l32 over the waves
 #pragma unroll
-    for (int w = 0; w < kDecWaves; w++) {
-        const float mw = sm_ml[(w * 32 + l32) * 2 + 0];
+    for (int w = 0; w < C::WAVES; w++) {
         if (sm_ml[(w * 32 + l32) * 2 + 1] > 0.0f) {
-            mref = fmaxf(mref, mw);
+            mref = fmaxf(mref, sm_ml[(w * 32 + l32) * 2 + 0]);
         }
     }
-    const float scale_w = (l_tot > 0.0f) ? fast_exp2(m_run - mref) : 0.0f;
+#pragma unroll
+    for (int w = 0; w < C::WAVES; w++) {
+        const float lw = sm_ml[(w * 32 + l32) * 2 + 1];
+        if (lw > 0.0f) {
+            lsum += lw * fast_exp2(sm_ml[(w * 32 + l32) * 2 + 0] - mref);
+        }
+    }
+    const bool whole = p.splits == 1;
+    float scale_w = (l_tot > 0.0f) ? fast_exp2(m_run - mref) : 0.0f;
+    if (whole) {
+        scale_w *= lsum > 0.0f ? 1.0f / lsum : 0.0f;
+    }
 #pragma unroll
     for (int dt = 0; dt < C::NDT; dt++) {
+        oacc[dt] *= scale_w;
+    }
+    // the upper half of the waves through LDS into the lower half, then those
+    // through LDS into whole rows
+    float* const my_o = &sm_o[((wave % C::MERGE) * 32 + l32) * C::LDM + 4 * g];
+    auto put_o = [&]() {
+        if (col_valid) {
 #pragma unroll
-        for (int e = 0; e < 16; e++) {
-            const int d = 32 * dt + 8 * (e >> 2) + 4 * g + (e & 3);
-            sm_o[(wave * D + d) * 32 + l32] = oacc[dt][e] * scale_w;
+            for (int dt = 0; dt < C::NDT; dt++) {
+#pragma unroll
+                for (int e4 = 0; e4 < 4; e4++) {
+                    *reinterpret_cast<f4*>(my_o + 32 * dt + 8 * e4) =
+                        f4{oacc[dt][4 * e4], oacc[dt][4 * e4 + 1], oacc[dt][4 * e4 + 2], oacc[dt][4 * e4 + 3]};
+                }
+            }
         }
+    };
+    if (wave >= C::MERGE) {
+        put_o();
     }
     __syncthreads();
-    const int64_t part = (int64_t)bkv * p.splits + split;
-    for (int e = tid; e < p.M * D; e += kDecThreads) {
-        const int col = e / D;
-        const int d = e - col * D;
-        float acc = 0.0f;
+    if (wave < C::MERGE && col_valid) {
 #pragma unroll
-        for (int w = 0; w < kDecWaves; w++) {
-            acc += sm_o[(w * D + d) * 32 + col];
+        for (int dt = 0; dt < C::NDT; dt++) {
+#pragma unroll
+            for (int e4 = 0; e4 < 4; e4++) {
+                const f4 x = *reinterpret_cast<const f4*>(my_o + 32 * dt + 8 * e4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    oacc[dt][4 * e4 + e] += x[e];
+                }
+            }
         }
-        p.part_o[(part * p.M + col) * D + d] = acc;
     }
-    if (tid < p.M) {
-        float mr = -INFINITY, lsum = 0.0f;
+    if (wave < C::MERGE) {
+        put_o(); // its own slot, read above by the same lanes
+    }
+    const int64_t part = ((int64_t)bkv * p.splits + split) * p.M;
+    if (!whole && tid < p.M) { // M <= 32: the threads that hold mref, lsum of column tid
+        p.part_ml[(part + tid) * 2 + 0] = mref;
+        p.part_ml[(part + tid) * 2 + 1] = lsum;
+    }
+    __syncthreads();
+    auto out_row = [&](int col) {
+        const int ho = col / p.Sq;
+        return p.o + b * p.o_sb + (kvh * p.ratio + ho) * p.o_sh + (int64_t)(col - ho * p.Sq) * p.o_ss;
+    };
+    for (int e = tid; e < p.M * (D / 4); e += C::THREADS) {
+        const int col = e / (D / 4);
+        const int d = 4 * (e - col * (D / 4));
+        f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int w = 0; w < kDecWaves; w++) {
-            if (sm_ml[(w * 32 + tid) * 2 + 1] > 0.0f) {
-                mr = fmaxf(mr, sm_ml[(w * 32 + tid) * 2 + 0]);
-            }
+        for (int w = 0; w < C::MERGE; w++) {
+            acc += *reinterpret_cast<const f4*>(&sm_o[(w * 32 + col) * C::LDM + d]);
         }
-#pragma unroll
-        for (int w = 0; w < kDecWaves; w++) {
-            const float lw = sm_ml[(w * 32 + tid) * 2 + 1];
-            if (lw > 0.0f) {
-                lsum += lw * fast_exp2(sm_ml[(w * 32 + tid) * 2 + 0] - mr);
-            }
+        if (whole) {
+            *reinterpret_cast<h4*>(out_row(col) + d) = __builtin_convertvector(acc, h4);
+        } else {
+            *reinterpret_cast<f4*>(&p.part_o[(part + col) * D + d]) = acc;
         }
-        p.part_ml[(part * p.M + tid) * 2 + 0] = mr;
-        p.part_ml[(part * p.M + tid) * 2 + 1] = lsum;
     }
 }
 
@@ -336,8 +400,15 @@ struct CombineParams {
 };
 
 // One workgroup per output row (b, kv head, column): log-sum-exp merge of the
-// splits, normalise once in fp32, round once to fp16.
-__global__ __launch_bounds__(128) void fa_decode_combine(CombineParams p) {
+// splits, normalised in fp32, rounded once to fp16.  Merging inside the split
+// kernel instead, by the last workgroup of each group to arrive, measured
+// slower although it saves this launch (B = 4 Hq = 32 Hkv = 8 Sk = 4096 D =
+// 128: 31.6 against 19.2 us a call; B = 16 Sk = 32768: 330 against 317): the
+// device-scope release and acquire it needs write back and invalidate whole
+// L2s.
+template <int T>
+__global__ __launch_bounds__(T) void fa_decode_combine(CombineParams p) {
+    __shared__ __attribute__((aligned(16))) float lds[merge_lds_floats(kMaxSplits, T)];
     const int row = blockIdx.x; // (b * Hkv + kvh) * M + col
     const int col = row % p.M;
     const int bkv = row / p.M;
@@ -345,39 +416,18 @@ __global__ __launch_bounds__(128) void fa_decode_combine(CombineParams p) {
     const int kvh = bkv - b * p.Hkv;
     const int h = kvh * p.ratio + col / p.Sq;
     const int q = col % p.Sq;
-    float mref = -INFINITY;
-    for (int s = 0; s < p.splits; s++) {
-        const float* ml = p.part_ml + (((int64_t)bkv * p.splits + s) * p.M + col) * 2;
-        if (ml[1] > 0.0f) {
-            mref = fmaxf(mref, ml[0]);
-        }
-    }
-    float lsum = 0.0f;
-    for (int s = 0; s < p.splits; s++) {
-        const float* ml = p.part_ml + (((int64_t)bkv * p.splits + s) * p.M + col) * 2;
-        if (ml[1] > 0.0f) {
-            lsum += ml[1] * fast_exp2(ml[0] - mref);
-        }
-    }
-    const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
     _Float16* orow = p.o + b * p.o_sb + h * p.o_sh + (int64_t)q * p.o_ss;
-    for (int d = threadIdx.x; d < p.D; d += blockDim.x) {
-        float acc = 0.0f;
-        for (int s = 0; s < p.splits; s++) {
-            const int64_t part = (int64_t)bkv * p.splits + s;
-            const float* ml = p.part_ml + (part * p.M + col) * 2;
-            if (ml[1] > 0.0f) {
-                acc += p.part_o[(part * p.M + col) * p.D + d] * fast_exp2(ml[0] - mref);
-            }
-        }
-        orow[d] = (_Float16)(acc * inv);
-    }
+    const int64_t first = (int64_t)bkv * p.splits * p.M + col;
+    const SplitParts parts{p.part_o + first * p.D, p.part_ml + first * 2, (int64_t)p.M * p.D, 2 * p.M, p.splits, p.D};
+    merge_splits<T>(parts, lds, [&](int d, f4 x) {
+        *reinterpret_cast<h4*>(orow + d) = __builtin_convertvector(x, h4);
+    });
 }
 
 template <int D>
 int launch_decode(const DecodeParams& p, int n_bkv, hipStream_t stream, std::string& err) {
     KernelTimerGuard timer(stream);
-    hipLaunchKernelGGL(fa_fwd_f16_decode<D>, dim3(p.splits, n_bkv), dim3(kDecThreads), 0, stream, p);
+    hipLaunchKernelGGL(fa_fwd_f16_decode<D>, dim3(p.splits, n_bkv), dim3(DecCfg<D>::THREADS), 0, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         err = hipGetErrorString(e);
@@ -386,9 +436,19 @@ int launch_decode(const DecodeParams& p, int n_bkv, hipStream_t stream, std::str
     return 0;
 }
 
-template <int D>
-int64_t decode_resident(std::string& err) {
-    return resident_workgroups(reinterpret_cast<const void*>(&fa_fwd_f16_decode<D>), kDecThreads, err);
+// f(std::integral_constant<int, D>) for the head dims the kernel is built for
+template <class F>
+auto for_dim(int d, F&& f) -> decltype(f(std::integral_constant<int, 32>{})) {
+    switch (d) {
+    case 32: return f(std::integral_constant<int, 32>{});
+    case 64: return f(std::integral_constant<int, 64>{});
+    case 96: return f(std::integral_constant<int, 96>{});
+    case 128: return f(std::integral_constant<int, 128>{});
+    case 160: return f(std::integral_constant<int, 160>{});
+    case 192: return f(std::integral_constant<int, 192>{});
+    case 224: return f(std::integral_constant<int, 224>{});
+    default: return f(std::integral_constant<int, 256>{});
+    }
 }
 
 } // namespace
@@ -398,35 +458,75 @@ bool splitk_supported(const AttnArgs& a) {
     return (a.D == 32 || a.D == 64 || a.D == 128) && M <= 32;
 }
 
-int splitk_plan(const AttnArgs& a, int& splits, int& keys_per_split, std::string& err) {
-    // splits: one round of workgroups over the device (as many as it holds at
-    // once: one per CU at D = 128, where the LDS ring is 128 KB), each split a
-    // whole number of 4-wave tile rounds. Measured on the B=16 Hkv=8
-    // Sk=32768 cache: 256 workgroups stream 1-4 % faster than 512 and
-    // 4-14 % faster than 1024 or 2048; uneven counts (384, 768) are slower.
-    const int n_bkv = a.B * a.Hkv;
-    const int round = kDecWaves * kDecTile;
-    const int max_splits = std::max(1, (a.Sk + round - 1) / round);
-    const int64_t resident = a.D == 32 ? decode_resident<32>(err)
-                                       : (a.D == 64 ? decode_resident<64>(err) : decode_resident<128>(err));
+bool splitk_built(const AttnArgs& a) {
+    return a.D <= 256 && (int64_t)(a.Hq / a.Hkv) * a.Sq <= 32;
+}
+
+int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::string& err) {
+    // The keys that some row sees, from a tile boundary on, are dealt to the
+    // splits in whole rounds of tiles (one tile per wave).
+    const MaskSpec mask{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
+    int lo, hi;
+    visible_key_range(mask, 0, a.Sq - 1, lo, hi);
+    plan = SplitKPlan{};
+    if (hi < lo) {
+        plan.keys_per_split = kDecTile;
+        return 0; // one split, which writes zeros
+    }
+    plan.key0 = lo / kDecTile * kDecTile;
+    const int64_t keys = (int64_t)hi + 1 - plan.key0;
+    const int64_t n_bkv = (int64_t)a.B * a.Hkv;
+    int64_t round = 0, resident = 0;
+    for_dim(a.D, [&](auto d) {
+        constexpr int D = decltype(d)::value;
+        round = DecCfg<D>::WAVES * kDecTile;
+        resident = resident_workgroups(reinterpret_cast<const void*>(&fa_fwd_f16_decode<D>), DecCfg<D>::THREADS, err);
+    });
     if (resident <= 0) {
         return -1;
     }
-    const int n = (int)std::max<int64_t>(1, std::min<int64_t>(max_splits, (resident + n_bkv - 1) / n_bkv));
-    int kps = (a.Sk + n - 1) / n;
-    kps = std::max(round, (kps + round - 1) / round * round);
-    splits = std::max(1, (a.Sk + kps - 1) / kps);
-    keys_per_split = kps;
+    // Splits: the least modelled time over 1 .. 256.  A launch runs in rounds
+    // of `resident` workgroups (one per CU at D = 128); a workgroup takes
+    // about 2 us beside its keys and streams at most 40 KB/us (measured: 40
+    // with 128 workgroups, 48 to 50 with 8 to 64, D = 128 to 256), all
+    // together 6.8 TB/s; merging takes about 2 us.  So a count just above a
+    // whole round (264 workgroups for 24 kv heads) is never taken, which
+    // rounding resident / n_bkv up did.  Measured, us a call, against the
+    // count chosen: n_bkv 128, Sk 32768: 420 (1), 317 (2, chosen), 349 (3);
+    // 32, 4096: 23 (4), 19.2 (8, chosen), 25.7 (16); 8, 32768: 37 (16),
+    // 29.7 (32, chosen), 33.7 (64); D = 64, 256, 2048: 27.6 (1, chosen), 33 (2).
+    const int64_t key_bytes = 4 * (int64_t)a.D;
+    const int64_t rounds_of_keys = (keys + round - 1) / round;
+    double best = 0.0;
+    for (int64_t s = 1; s <= std::min<int64_t>(rounds_of_keys, kMaxSplits); s++) {
+        const int64_t kps = (rounds_of_keys + s - 1) / s * round;
+        if (kps * (s - 1) >= keys || region_bytes(splitk_partial_bytes(a, (int)s)) > max_partials) {
+            continue; // the last split would be empty, or the partials too large
+        }
+        const int64_t wgs = n_bkv * s;
+        const int64_t waves_of_wgs = (wgs + resident - 1) / resident;
+        const double rate = std::min(40e3, 6.8e6 / (double)std::min(wgs, resident)); // bytes per us
+        const double t = (double)waves_of_wgs * (2.0 + (double)(std::min(kps, keys) * key_bytes) / rate) +
+                         (s > 1 ? 2.0 : 0.0);
+        if (s == 1 || t < best) {
+            best = t;
+            plan.splits = (int)s;
+            plan.keys_per_split = (int)kps;
+        }
+    }
     return 0;
 }
 
 size_t splitk_partial_bytes(const AttnArgs& a, int splits) {
+    if (splits <= 1) {
+        return 0;
+    }
     const size_t n_part = (size_t)a.B * a.Hkv * splits * ((a.Hq / a.Hkv) * a.Sq);
     return n_part * (a.D + 2) * sizeof(float);
 }
 
 int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err, ScratchRegion* region) {
-    if (!splitk_supported(a)) {
+    if (!splitk_built(a)) {
         err = "split-K path needs head_dim in {32, 64, 128} and (num_heads / num_kv_heads) * seq_len <= 32";
         return -1;
     }
@@ -434,6 +534,7 @@ int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::stri
     p.q = static_cast<const _Float16*>(a.q);
     p.k = static_cast<const _Float16*>(a.k);
     p.v = static_cast<const _Float16*>(a.v);
+    p.o = static_cast<_Float16*>(a.o);
     p.rot_cos = a.rot_cos;
     p.rot_sin = a.rot_sin;
     p.q_sb = a.qs[0];
@@ -445,6 +546,9 @@ int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::stri
     p.v_sb = a.vs[0];
     p.v_sh = a.vs[1];
     p.v_ss = a.vs[2];
+    p.o_sb = a.os[0];
+    p.o_sh = a.os[1];
+    p.o_ss = a.os[2];
     p.Sq = a.Sq;
     p.Hkv = a.Hkv;
     p.ratio = a.Hq / a.Hkv;
@@ -455,37 +559,34 @@ int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::stri
     p.rope_q = rope_q ? 1 : 0;
 
     const int n_bkv = a.B * a.Hkv;
-    int splits = 0, kps = 0;
-    if (splitk_plan(a, splits, kps, err) != 0) {
+    SplitKPlan plan;
+    const size_t room = region != nullptr ? region->bytes - region->used : SIZE_MAX;
+    if (splitk_plan(a, room, plan, err) != 0) {
         return -1;
     }
-    p.splits = splits;
-    p.keys_per_split = kps;
+    p.splits = plan.splits;
+    p.keys_per_split = plan.keys_per_split;
+    p.key0 = plan.key0;
 
     // every partial is written by its split's workgroup before the combine
     // reads it, so the buffer needs no clearing
     StreamScratch ws(ScratchUse::SplitKPartials, region);
-    const size_t n_part = (size_t)n_bkv * splits * p.M;
-    if (ws.alloc(splitk_partial_bytes(a, splits), stream, err) != 0) {
+    const size_t n_part = (size_t)n_bkv * p.splits * p.M;
+    if (ws.alloc(splitk_partial_bytes(a, p.splits), stream, err) != 0) {
         return -1;
     }
     p.part_o = static_cast<float*>(ws.ptr);
-    p.part_ml = p.part_o + n_part * a.D;
-
-    int rc = -1;
-    switch (a.D) {
-    case 32: rc = launch_decode<32>(p, n_bkv, stream, err); break;
-    case 64: rc = launch_decode<64>(p, n_bkv, stream, err); break;
-    case 128: rc = launch_decode<128>(p, n_bkv, stream, err); break;
-    default: err = "unsupported head_dim"; return -1;
+    p.part_ml = p.splits > 1 ? p.part_o + n_part * a.D : nullptr;
+    if (for_dim(a.D, [&](auto d) { return launch_decode<decltype(d)::value>(p, n_bkv, stream, err); }) != 0) {
+        return -1;
     }
-    if (rc != 0) {
-        return rc;
+    if (p.splits == 1) {
+        return 0;
     }
     CombineParams cp{};
     cp.part_o = p.part_o;
     cp.part_ml = p.part_ml;
-    cp.o = static_cast<_Float16*>(a.o);
+    cp.o = p.o;
     cp.o_sb = a.os[0];
     cp.o_sh = a.os[1];
     cp.o_ss = a.os[2];
@@ -493,9 +594,14 @@ int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::stri
     cp.ratio = p.ratio;
     cp.Sq = a.Sq;
     cp.M = p.M;
-    cp.splits = splits;
+    cp.splits = p.splits;
     cp.D = a.D;
-    hipLaunchKernelGGL(fa_decode_combine, dim3((uint32_t)(n_bkv * p.M)), dim3(128), 0, stream, cp);
+    const dim3 grid((uint32_t)(n_bkv * p.M));
+    if (p.splits >= 8) {
+        hipLaunchKernelGGL(fa_decode_combine<256>, grid, dim3(256), 0, stream, cp);
+    } else {
+        hipLaunchKernelGGL(fa_decode_combine<64>, grid, dim3(64), 0, stream, cp);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         err = hipGetErrorString(e);

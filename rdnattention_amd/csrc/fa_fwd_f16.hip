@@ -795,11 +795,12 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
 }
 
 bool splitk_supported(const AttnArgs& a);
+bool splitk_built(const AttnArgs& a);
 
 // Auto: few query rows per kv head against a long key sequence -> split-K
 // (HBM-bound, parallel over the key axis); everything else -> prefill tiles.
 bool prefer_splitk(const AttnArgs& a) {
-    return splitk_supported(a) && a.Sk >= 512;
+    return splitk_built(a) && a.Sk >= 512;
 }
 
 int64_t fwd_f16_scratch_bytes(const AttnArgs& a, F16Path path, std::string& err) {
@@ -808,12 +809,13 @@ int64_t fwd_f16_scratch_bytes(const AttnArgs& a, F16Path path, std::string& err)
     if (a.has_rope && a.Sk > 0) {
         bytes += region_bytes((size_t)a.B * a.Hkv * a.Sk * a.D * sizeof(_Float16));
     }
-    if (splitk && splitk_supported(a)) {
-        int splits = 0, kps = 0;
-        if (splitk_plan(a, splits, kps, err) != 0) {
+    if (splitk && splitk_built(a)) {
+        // fewer splits where the partials would not fit beside the K copy
+        SplitKPlan plan;
+        if (splitk_plan(a, kNoAllocBytes - std::min(bytes, kNoAllocBytes), plan, err) != 0) {
             return -1;
         }
-        bytes += region_bytes(splitk_partial_bytes(a, splits));
+        bytes += region_bytes(splitk_partial_bytes(a, plan.splits));
     }
     return (int64_t)bytes;
 }
@@ -826,6 +828,10 @@ int fwd_f16(const AttnArgs& in, F16Path path, hipStream_t stream, std::string& e
         return -1;
     }
     const bool splitk = path == F16Path::SplitK || (path == F16Path::Auto && prefer_splitk(a));
+    if (path == F16Path::SplitK && !splitk_supported(a)) {
+        err = "split-K path needs head_dim in {32, 64, 128} and (num_heads / num_kv_heads) * seq_len <= 32";
+        return -1;
+    }
     StreamScratch krot(ScratchUse::RotatedK, region);
     if (a.has_rope && a.Sk > 0) {
         const size_t bytes = (size_t)a.B * a.Hkv * a.Sk * a.D * sizeof(_Float16);

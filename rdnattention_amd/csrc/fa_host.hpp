@@ -65,8 +65,8 @@ struct ScratchRegion;
 // checks fwd_f16_scratch_bytes against its size.
 int fwd_f16(const AttnArgs& a, F16Path path, hipStream_t stream, std::string& err, ScratchRegion* region = nullptr);
 
-// Scratch bytes fwd_f16 takes for these arguments (each buffer 256-byte
-// aligned), or -1 with `err`.
+// Scratch bytes fwd_f16 takes from a region of kNoAllocBytes for these arguments
+// (each buffer 256-byte aligned), or -1 with `err`.
 int64_t fwd_f16_scratch_bytes(const AttnArgs& a, F16Path path, std::string& err);
 
 // INT8 forward (Q K^T on int8 MFMA, P V on fp16 MFMA).  Returns 0 or sets `err`.

@@ -106,11 +106,18 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
 int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err,
                    ScratchRegion* region = nullptr);
 
-// Split-K plan of a decode launch: key splits and keys per split.  0, or -1
-// with `err` (occupancy query failed).
-int splitk_plan(const AttnArgs& a, int& splits, int& keys_per_split, std::string& err);
+// Split-K plan of a decode launch: split s of `splits` covers keys_per_split
+// keys from key0 + s * keys_per_split on, with at most max_partials bytes of
+// partials.  0, or -1 with `err` (occupancy query failed).
+struct SplitKPlan {
+    int splits = 1;
+    int keys_per_split = 0;
+    int key0 = 0;
+};
+int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::string& err);
 
-// Bytes of the split-K partials (per split and query row: O in fp32 plus m, l).
+// Bytes of the split-K partials (per split and query row: O in fp32 plus m, l;
+// none for a single split).
 size_t splitk_partial_bytes(const AttnArgs& a, int splits);
 
 } // namespace rdna_amd

@@ -97,3 +97,53 @@ def test_splitk_unsupported_shape_is_rejected(gpu):
     assert forward_raw(q, k, k, out, path=PATH_SPLITK) == -3
     assert "split-K" in rdnattention.last_error()
     assert forward_raw(q, k, k, out, path=0) == 0  # auto falls back to the prefill kernel
+
+
+# d, b, hq, hkv, sq, sk, causal, window: every head dim the automatic choice
+# sends to split-K, at the edges of its tiles (32 keys), rounds (32 keys per
+# wave) and columns (1 .. 32 rows per kv head); merged by the last workgroup
+# (few splits or rows), by the combine kernel (MQA with many), or not at all
+AUTO_CASES = [(d, 1, 8, 2, 1, 513, False, -1) for d in range(32, 257, 32)] + [
+    (256, 2, 4, 4, 1, 2049, False, -1),
+    (256, 1, 32, 1, 1, 4100, False, -1),
+    (224, 1, 8, 8, 5, 1023, True, -1),
+    (192, 2, 8, 2, 8, 3000, True, -1),
+    (160, 1, 6, 2, 3, 1500, True, 600),
+    (96, 3, 5, 1, 4, 777, True, -1),
+    (96, 1, 8, 2, 2, 4000, False, 900),
+    (128, 1, 32, 1, 1, 30000, False, -1),
+    (128, 33, 8, 8, 1, 520, False, -1),
+]
+
+
+@pytest.mark.parametrize("case", AUTO_CASES, ids=["d{}b{}h{}kv{}q{}k{}c{:d}w{}".format(*c) for c in AUTO_CASES])
+def test_auto_decode_vs_oracle(gpu, oracle_lib, case):
+    """FP16 bar against the oracle; a second call (the arrival counters of the
+    first must have returned to zero), the no-allocation entry point's two
+    launches and a captured graph's give the same bits."""
+    from tests.gpu_util import lib
+
+    d, b, hq, hkv, sq, sk, causal, window = case
+    log(f"[auto decode] {case}")
+    q, k, v = seeded_inputs(31, b, hq, hkv, sq, sk, d)
+    ref = reference_f16(q, k, v, causal, window)
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    outs = [torch.full_like(qd, float("nan")) for _ in range(4)]
+    for o in outs[:2]:
+        assert forward_raw(qd, kd, vd, o, causal, window) == 0
+    o = outs[2]
+    qs, ks, vs, os_ = qd.stride(), kd.stride(), vd.stride(), o.stride()
+    assert lib().rdna_attention_forward_noalloc(
+        qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), o.data_ptr(), None, None, *qs[:3], *ks[:3], *vs[:3], *os_[:3],
+        b, hq, hkv, sq, sk, d, d ** -0.5, int(causal), 0, window, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert forward_raw(qd, kd, vd, outs[3], causal, window) == 0
+    for _ in range(3):
+        outs[3].fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(outs[3], outs[0])
+    assert torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
+    assert_f16_parity(outs[0].float().cpu().numpy(), ref, "auto decode")
