@@ -47,16 +47,13 @@ struct DecodeParams {
     const _Float16* q;
     const _Float16* k;
     const _Float16* v;
-    _Float16* o;
     const float* rot_cos;
     const float* rot_sin;
     int64_t q_sb, q_sh, q_ss;
     int64_t k_sb, k_sh, k_ss;
     int64_t v_sb, v_sh, v_ss;
-    int64_t o_sb, o_sh, o_ss;
-    float* part_o;  // [B*Hkv][splits][M][D] unnormalised O (splits > 1)
-    float* part_ml; // [B*Hkv][splits][M][2]  (m in log2 units, l)
-    int32_t Sq, Hkv, ratio, M, splits, keys_per_split;
+    SplitRows out;
+    int32_t Hkv, keys_per_split;
     int32_t key0; // first key of split 0
     float c;
     float q_sign;
@@ -71,6 +68,8 @@ struct DecCfg {
     // one wave per SIMD, whose O alone takes 128 registers)
     static constexpr int WAVES = D <= 160 ? 8 : (D <= 192 ? 6 : 4);
     static constexpr int THREADS = 64 * WAVES;
+    // waves per SIMD: two workgroups share a CU's LDS at D = 64, four at 32
+    static constexpr int WAVES_PER_SIMD = D <= 32 ? 7 : (D <= 64 ? 4 : 1);
     static constexpr int RB = 2 * D;                 // row bytes (unpadded)
     static constexpr int KCH = D / 8;                // 16-byte chunks per row
     static constexpr int TILE_BYTES = kDecTile * RB; // one K (or V) tile
@@ -78,10 +77,8 @@ struct DecCfg {
     static constexpr int NS = D / 16;
     static constexpr int NDT = D / 32;
     static constexpr int DMA_PER_TILE = TILE_BYTES / 1024; // 1 KB per wave-wide DMA
-    static constexpr int LDM = D + 4;                      // floats per merged row (conflict-free b128)
     static_assert(WAVES * WAVE_BYTES <= 160 * 1024, "K/V tiles fit the LDS");
-    static constexpr int MERGE = WAVES / 2; // waves whose O is in LDS at once
-    static_assert((MERGE * 32 * LDM + WAVES * 32 * 2) * 4 <= WAVES * WAVE_BYTES, "the merge reuses the tile area");
+    static_assert(finish_lds_bytes(D, WAVES) <= WAVES * WAVE_BYTES, "the merge reuses the tile area");
 };
 
 // XOR swizzle of the 16-byte chunk index of row r (see the file comment).
@@ -101,7 +98,7 @@ __device__ __forceinline__ int dec_swz(int r) {
 }
 
 template <int D>
-__global__ __launch_bounds__(DecCfg<D>::THREADS, 1) void fa_fwd_f16_decode(DecodeParams p) {
+__global__ __launch_bounds__(DecCfg<D>::THREADS, DecCfg<D>::WAVES_PER_SIMD) void fa_fwd_f16_decode(DecodeParams p) {
     using C = DecCfg<D>;
     __shared__ __attribute__((aligned(16))) char dsm[C::WAVES * C::WAVE_BYTES];
 
@@ -116,16 +113,16 @@ __global__ __launch_bounds__(DecCfg<D>::THREADS, 1) void fa_fwd_f16_decode(Decod
     const int kvh = bkv - b * p.Hkv;
 
     // column l32 <-> (query head, query row)
-    const bool col_valid = l32 < p.M;
-    const int hoff = col_valid ? l32 / p.Sq : 0;
-    const int q = col_valid ? l32 - hoff * p.Sq : 0;
-    const int h = kvh * p.ratio + hoff;
+    const bool col_valid = l32 < p.out.M;
+    const int hoff = col_valid ? l32 / p.out.Sq : 0;
+    const int q = col_valid ? l32 - hoff * p.out.Sq : 0;
+    const int h = kvh * p.out.ratio + hoff;
 
     // this split's key range, restricted to what any of the M rows can see
     const int k_begin = p.key0 + split * p.keys_per_split;
     const int k_end = min(k_begin + p.keys_per_split, p.mask.sk);
     int vis_lo, vis_hi;
-    visible_key_range(p.mask, 0, p.Sq - 1, vis_lo, vis_hi);
+    visible_key_range(p.mask, 0, p.out.Sq - 1, vis_lo, vis_hi);
     const int lo = max(k_begin, vis_lo);
     const int hi = min(k_end - 1, vis_hi);
     int t0 = 0, nt = 0; // tiles of this wave: kt = t0 + wave + WAVES * j
@@ -296,108 +293,8 @@ __global__ __launch_bounds__(DecCfg<D>::THREADS, 1) void fa_fwd_f16_decode(Decod
         }
     }
     __builtin_amdgcn_s_waitcnt(0); // all DMAs and LDS traffic of this wave done
-    __syncthreads();
-
-    // ---- merge the waves in LDS (reusing the tile buffers)
-    float* sm_o = reinterpret_cast<float*>(dsm);            // [MERGE][32][LDM]
-    float* sm_ml = sm_o + C::MERGE * 32 * C::LDM;           // [WAVES][32][2]
-    const float l_tot = pair_sum(l_run);
-    if (g == 0) {
-        sm_ml[(wave * 32 + l32) * 2 + 0] = m_run;
-        sm_ml[(wave * 32 + l32) * 2 + 1] = l_tot;
-    }
-    __syncthreads();
-    float mref = -INFINITY, lsum = 0.0f; // of column l32 over the waves
-#pragma unroll
-    for (int w = 0; w < C::WAVES; w++) {
-        if (sm_ml[(w * 32 + l32) * 2 + 1] > 0.0f) {
-            mref = fmaxf(mref, sm_ml[(w * 32 + l32) * 2 + 0]);
-        }
-    }
-#pragma unroll
-    for (int w = 0; w < C::WAVES; w++) {
-        const float lw = sm_ml[(w * 32 + l32) * 2 + 1];
-        if (lw > 0.0f) {
-            lsum += lw * fast_exp2(sm_ml[(w * 32 + l32) * 2 + 0] - mref);
-        }
-    }
-    const bool whole = p.splits == 1;
-    float scale_w = (l_tot > 0.0f) ? fast_exp2(m_run - mref) : 0.0f;
-    if (whole) {
-        scale_w *= lsum > 0.0f ? 1.0f / lsum : 0.0f;
-    }
-#pragma unroll
-    for (int dt = 0; dt < C::NDT; dt++) {
-        oacc[dt] *= scale_w;
-    }
-    // the upper half of the waves through LDS into the lower half, then those
-    // through LDS into whole rows
-    float* const my_o = &sm_o[((wave % C::MERGE) * 32 + l32) * C::LDM + 4 * g];
-    auto put_o = [&]() {
-        if (col_valid) {
-#pragma unroll
-            for (int dt = 0; dt < C::NDT; dt++) {
-#pragma unroll
-                for (int e4 = 0; e4 < 4; e4++) {
-                    *reinterpret_cast<f4*>(my_o + 32 * dt + 8 * e4) =
-                        f4{oacc[dt][4 * e4], oacc[dt][4 * e4 + 1], oacc[dt][4 * e4 + 2], oacc[dt][4 * e4 + 3]};
-                }
-            }
-        }
-    };
-    if (wave >= C::MERGE) {
-        put_o();
-    }
-    __syncthreads();
-    if (wave < C::MERGE && col_valid) {
-#pragma unroll
-        for (int dt = 0; dt < C::NDT; dt++) {
-#pragma unroll
-            for (int e4 = 0; e4 < 4; e4++) {
-                const f4 x = *reinterpret_cast<const f4*>(my_o + 32 * dt + 8 * e4);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    oacc[dt][4 * e4 + e] += x[e];
-                }
-            }
-        }
-    }
-    if (wave < C::MERGE) {
-        put_o(); // its own slot, read above by the same lanes
-    }
-    const int64_t part = ((int64_t)bkv * p.splits + split) * p.M;
-    if (!whole && tid < p.M) { // M <= 32: the threads that hold mref, lsum of column tid
-        p.part_ml[(part + tid) * 2 + 0] = mref;
-        p.part_ml[(part + tid) * 2 + 1] = lsum;
-    }
-    __syncthreads();
-    auto out_row = [&](int col) {
-        const int ho = col / p.Sq;
-        return p.o + b * p.o_sb + (kvh * p.ratio + ho) * p.o_sh + (int64_t)(col - ho * p.Sq) * p.o_ss;
-    };
-    for (int e = tid; e < p.M * (D / 4); e += C::THREADS) {
-        const int col = e / (D / 4);
-        const int d = 4 * (e - col * (D / 4));
-        f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int w = 0; w < C::MERGE; w++) {
-            acc += *reinterpret_cast<const f4*>(&sm_o[(w * 32 + col) * C::LDM + d]);
-        }
-        if (whole) {
-            *reinterpret_cast<h4*>(out_row(col) + d) = __builtin_convertvector(acc, h4);
-        } else {
-            *reinterpret_cast<f4*>(&p.part_o[(part + col) * D + d]) = acc;
-        }
-    }
+    finish_rows<D, C::WAVES>(oacc, m_run, l_run, dsm, p.out, b, kvh, bkv, split, [](f4 x, int) { return x; });
 }
-
-struct CombineParams {
-    const float* part_o;
-    const float* part_ml;
-    _Float16* o;
-    int64_t o_sb, o_sh, o_ss;
-    int32_t Hkv, ratio, Sq, M, splits, D;
-};
 
 // One workgroup per output row (b, kv head, column): log-sum-exp merge of the
 // splits, normalised in fp32, rounded once to fp16.  Merging inside the split
@@ -407,18 +304,16 @@ struct CombineParams {
 // device-scope release and acquire it needs write back and invalidate whole
 // L2s.
 template <int T>
-__global__ __launch_bounds__(T) void fa_decode_combine(CombineParams p) {
+__global__ __launch_bounds__(T) void fa_decode_combine(SplitRows r, int32_t Hkv, int32_t D) {
     __shared__ __attribute__((aligned(16))) float lds[merge_lds_floats(kMaxSplits, T)];
     const int row = blockIdx.x; // (b * Hkv + kvh) * M + col
-    const int col = row % p.M;
-    const int bkv = row / p.M;
-    const int b = bkv / p.Hkv;
-    const int kvh = bkv - b * p.Hkv;
-    const int h = kvh * p.ratio + col / p.Sq;
-    const int q = col % p.Sq;
-    _Float16* orow = p.o + b * p.o_sb + h * p.o_sh + (int64_t)q * p.o_ss;
-    const int64_t first = (int64_t)bkv * p.splits * p.M + col;
-    const SplitParts parts{p.part_o + first * p.D, p.part_ml + first * 2, (int64_t)p.M * p.D, 2 * p.M, p.splits, p.D};
+    const int col = row % r.M;
+    const int bkv = row / r.M;
+    const int b = bkv / Hkv;
+    const int kvh = bkv - b * Hkv;
+    _Float16* orow = r.row(b, kvh, col);
+    const int64_t first = (int64_t)bkv * r.splits * r.M + col;
+    const SplitParts parts{r.part_o + first * D, r.part_ml + first * 2, (int64_t)r.M * D, 2 * r.M, r.splits, D};
     merge_splits<T>(parts, lds, [&](int d, f4 x) {
         *reinterpret_cast<h4*>(orow + d) = __builtin_convertvector(x, h4);
     });
@@ -427,7 +322,7 @@ __global__ __launch_bounds__(T) void fa_decode_combine(CombineParams p) {
 template <int D>
 int launch_decode(const DecodeParams& p, int n_bkv, hipStream_t stream, std::string& err) {
     KernelTimerGuard timer(stream);
-    hipLaunchKernelGGL(fa_fwd_f16_decode<D>, dim3(p.splits, n_bkv), dim3(DecCfg<D>::THREADS), 0, stream, p);
+    hipLaunchKernelGGL(fa_fwd_f16_decode<D>, dim3(p.out.splits, n_bkv), dim3(DecCfg<D>::THREADS), 0, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         err = hipGetErrorString(e);
@@ -462,29 +357,29 @@ bool splitk_built(const AttnArgs& a) {
     return a.D <= 256 && (int64_t)(a.Hq / a.Hkv) * a.Sq <= 32;
 }
 
-int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::string& err) {
+size_t splitk_partial_bytes(const AttnArgs& a, int splits) {
+    if (splits <= 1) {
+        return 0;
+    }
+    const size_t n_part = (size_t)a.B * a.Hkv * splits * ((a.Hq / a.Hkv) * a.Sq);
+    return n_part * (a.D + 2) * sizeof(float);
+}
+
+SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
+                           size_t max_partials) {
     // The keys that some row sees, from a tile boundary on, are dealt to the
     // splits in whole rounds of tiles (one tile per wave).
     const MaskSpec mask{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
     int lo, hi;
     visible_key_range(mask, 0, a.Sq - 1, lo, hi);
-    plan = SplitKPlan{};
+    SplitKPlan plan;
     if (hi < lo) {
-        plan.keys_per_split = kDecTile;
-        return 0; // one split, which writes zeros
+        plan.keys_per_split = tile;
+        return plan; // one split, which writes zeros
     }
-    plan.key0 = lo / kDecTile * kDecTile;
+    plan.key0 = lo / tile * tile;
     const int64_t keys = (int64_t)hi + 1 - plan.key0;
     const int64_t n_bkv = (int64_t)a.B * a.Hkv;
-    int64_t round = 0, resident = 0;
-    for_dim(a.D, [&](auto d) {
-        constexpr int D = decltype(d)::value;
-        round = DecCfg<D>::WAVES * kDecTile;
-        resident = resident_workgroups(reinterpret_cast<const void*>(&fa_fwd_f16_decode<D>), DecCfg<D>::THREADS, err);
-    });
-    if (resident <= 0) {
-        return -1;
-    }
     // Splits: the least modelled time over 1 .. 256.  A launch runs in rounds
     // of `resident` workgroups (one per CU at D = 128); a workgroup takes
     // about 2 us beside its keys and streams at most 40 KB/us (measured: 40
@@ -495,7 +390,6 @@ int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::s
     // count chosen: n_bkv 128, Sk 32768: 420 (1), 317 (2, chosen), 349 (3);
     // 32, 4096: 23 (4), 19.2 (8, chosen), 25.7 (16); 8, 32768: 37 (16),
     // 29.7 (32, chosen), 33.7 (64); D = 64, 256, 2048: 27.6 (1, chosen), 33 (2).
-    const int64_t key_bytes = 4 * (int64_t)a.D;
     const int64_t rounds_of_keys = (keys + round - 1) / round;
     double best = 0.0;
     for (int64_t s = 1; s <= std::min<int64_t>(rounds_of_keys, kMaxSplits); s++) {
@@ -514,15 +408,58 @@ int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::s
             plan.keys_per_split = (int)kps;
         }
     }
+    return plan;
+}
+
+int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::string& err) {
+    return for_dim(a.D, [&](auto d) {
+        using C = DecCfg<decltype(d)::value>;
+        const int64_t resident = resident_workgroups(
+            reinterpret_cast<const void*>(&fa_fwd_f16_decode<decltype(d)::value>), C::THREADS, err);
+        if (resident <= 0) {
+            return -1;
+        }
+        plan = splitk_plan_for(a, kDecTile, C::WAVES * kDecTile, 2 * C::RB, resident, max_partials);
+        return 0;
+    });
+}
+
+int splitk_begin(const AttnArgs& a, const SplitKPlan& plan, StreamScratch& ws, hipStream_t stream, SplitRows& r,
+                 std::string& err) {
+    r.o = static_cast<_Float16*>(a.o);
+    r.o_sb = a.os[0];
+    r.o_sh = a.os[1];
+    r.o_ss = a.os[2];
+    r.Sq = a.Sq;
+    r.ratio = a.Hq / a.Hkv;
+    r.M = r.ratio * a.Sq;
+    r.splits = plan.splits;
+    // every partial is written by its split's workgroup before the combine
+    // reads it, so the buffer needs no clearing
+    if (ws.alloc(splitk_partial_bytes(a, plan.splits), stream, err) != 0) {
+        return -1;
+    }
+    r.part_o = static_cast<float*>(ws.ptr);
+    r.part_ml = plan.splits > 1 ? r.part_o + (size_t)a.B * a.Hkv * r.splits * r.M * a.D : nullptr;
     return 0;
 }
 
-size_t splitk_partial_bytes(const AttnArgs& a, int splits) {
-    if (splits <= 1) {
+int splitk_finish(const AttnArgs& a, const SplitRows& r, hipStream_t stream, std::string& err) {
+    if (r.splits == 1) {
         return 0;
     }
-    const size_t n_part = (size_t)a.B * a.Hkv * splits * ((a.Hq / a.Hkv) * a.Sq);
-    return n_part * (a.D + 2) * sizeof(float);
+    const dim3 grid((uint32_t)(a.B * a.Hkv * r.M));
+    if (r.splits >= 8) {
+        hipLaunchKernelGGL(fa_decode_combine<256>, grid, dim3(256), 0, stream, r, a.Hkv, a.D);
+    } else {
+        hipLaunchKernelGGL(fa_decode_combine<64>, grid, dim3(64), 0, stream, r, a.Hkv, a.D);
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        err = hipGetErrorString(e);
+        return -1;
+    }
+    return 0;
 }
 
 int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err, ScratchRegion* region) {
@@ -534,7 +471,6 @@ int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::stri
     p.q = static_cast<const _Float16*>(a.q);
     p.k = static_cast<const _Float16*>(a.k);
     p.v = static_cast<const _Float16*>(a.v);
-    p.o = static_cast<_Float16*>(a.o);
     p.rot_cos = a.rot_cos;
     p.rot_sin = a.rot_sin;
     p.q_sb = a.qs[0];
@@ -546,68 +482,25 @@ int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::stri
     p.v_sb = a.vs[0];
     p.v_sh = a.vs[1];
     p.v_ss = a.vs[2];
-    p.o_sb = a.os[0];
-    p.o_sh = a.os[1];
-    p.o_ss = a.os[2];
-    p.Sq = a.Sq;
     p.Hkv = a.Hkv;
-    p.ratio = a.Hq / a.Hkv;
-    p.M = p.ratio * a.Sq;
     p.c = softmax_log2_scale(a.scale);
     p.q_sign = a.scale < 0.0f ? -1.0f : 1.0f;
     p.mask = MaskSpec{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
     p.rope_q = rope_q ? 1 : 0;
 
-    const int n_bkv = a.B * a.Hkv;
     SplitKPlan plan;
     const size_t room = region != nullptr ? region->bytes - region->used : SIZE_MAX;
     if (splitk_plan(a, room, plan, err) != 0) {
         return -1;
     }
-    p.splits = plan.splits;
     p.keys_per_split = plan.keys_per_split;
     p.key0 = plan.key0;
-
-    // every partial is written by its split's workgroup before the combine
-    // reads it, so the buffer needs no clearing
     StreamScratch ws(ScratchUse::SplitKPartials, region);
-    const size_t n_part = (size_t)n_bkv * p.splits * p.M;
-    if (ws.alloc(splitk_partial_bytes(a, p.splits), stream, err) != 0) {
+    if (splitk_begin(a, plan, ws, stream, p.out, err) != 0 ||
+        for_dim(a.D, [&](auto d) { return launch_decode<decltype(d)::value>(p, a.B * a.Hkv, stream, err); }) != 0) {
         return -1;
     }
-    p.part_o = static_cast<float*>(ws.ptr);
-    p.part_ml = p.splits > 1 ? p.part_o + n_part * a.D : nullptr;
-    if (for_dim(a.D, [&](auto d) { return launch_decode<decltype(d)::value>(p, n_bkv, stream, err); }) != 0) {
-        return -1;
-    }
-    if (p.splits == 1) {
-        return 0;
-    }
-    CombineParams cp{};
-    cp.part_o = p.part_o;
-    cp.part_ml = p.part_ml;
-    cp.o = p.o;
-    cp.o_sb = a.os[0];
-    cp.o_sh = a.os[1];
-    cp.o_ss = a.os[2];
-    cp.Hkv = a.Hkv;
-    cp.ratio = p.ratio;
-    cp.Sq = a.Sq;
-    cp.M = p.M;
-    cp.splits = p.splits;
-    cp.D = a.D;
-    const dim3 grid((uint32_t)(n_bkv * p.M));
-    if (p.splits >= 8) {
-        hipLaunchKernelGGL(fa_decode_combine<256>, grid, dim3(256), 0, stream, cp);
-    } else {
-        hipLaunchKernelGGL(fa_decode_combine<64>, grid, dim3(64), 0, stream, cp);
-    }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        err = hipGetErrorString(e);
-        return -1;
-    }
-    return 0;
+    return splitk_finish(a, p.out, stream, err);
 }
 
 } // namespace rdna_amd

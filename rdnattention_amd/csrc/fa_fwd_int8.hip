@@ -699,6 +699,12 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
     if (n_wg < 0) {
         return -1;
     }
+    // few query rows per kv head (one MFMA column block): split-K, at every key
+    // count; the prefill kernels put 256 rows in a workgroup (B8 Hq32 Hkv8
+    // Sq1 Sk8192 D128: 32 us a call against 206)
+    if ((a.D == 64 || a.D == 128) && (int64_t)p.ratio * a.Sq <= 32) {
+        return fwd_int8_splitk(a, p, stream, err);
+    }
     if (a.D == 64 && p.vtok == nullptr) {
         return p.ksv != nullptr ? launch_int8<64, true, false>(p, n_wg, stream, err)
                                 : launch_int8<64, false, false>(p, n_wg, stream, err);

@@ -68,4 +68,8 @@ int64_t int8_params(const AttnArgs& a, Int8Params& p, std::string& err);
 int launch_int8_f16pv(const Int8Params& p, int head_dim, bool scores, int64_t n_wg, hipStream_t stream,
                       std::string& err);
 
+// Split-K decode (fa_fwd_int8_decode.hip): (Hq / Hkv) * Sq <= 32, head_dim 64
+// or 128.
+int fwd_int8_splitk(const AttnArgs& a, const Int8Params& p, hipStream_t stream, std::string& err);
+
 } // namespace rdna_amd

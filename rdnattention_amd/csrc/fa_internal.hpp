@@ -116,6 +116,19 @@ struct SplitKPlan {
 };
 int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::string& err);
 
+// The same for any split-K kernel: `tile` keys per wave tile, `round` per
+// workgroup round of them, key_bytes of K and V per key, `resident` workgroups
+// on the device.
+SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
+                           size_t max_partials);
+
+// Before and after a split-K launch: `r` from the arguments, with the partials
+// taken from `ws`; and the combine launch.  0, or -1 with `err`.
+struct SplitRows;
+int splitk_begin(const AttnArgs& a, const SplitKPlan& plan, StreamScratch& ws, hipStream_t stream, SplitRows& r,
+                 std::string& err);
+int splitk_finish(const AttnArgs& a, const SplitRows& r, hipStream_t stream, std::string& err);
+
 // Bytes of the split-K partials (per split and query row: O in fp32 plus m, l;
 // none for a single split).
 size_t splitk_partial_bytes(const AttnArgs& a, int splits);

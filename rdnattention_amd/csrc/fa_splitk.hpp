@@ -1,4 +1,5 @@
-// Merge of key splits, shared by the split-K kernels (device code).
+// Merges shared by the split-K kernels (device code): of a workgroup's waves,
+// and of the key splits.
 //
 // A split leaves, per query row, O unnormalised in fp32 and (m, l): its
 // reference maximum in log2 units and its row sum relative to it.  The merged
@@ -11,6 +12,134 @@
 namespace rdna_amd {
 
 constexpr int kMaxSplits = 256; // weights of one row in the merge's LDS
+
+// Where the M = ratio * Sq rows of a (b, kv head) go: column c is query row
+// c % Sq of query head c / Sq of the group.
+struct SplitRows {
+    _Float16* o;
+    int64_t o_sb, o_sh, o_ss;
+    float* part_o;  // [B*Hkv][splits][M][D] unnormalised O (splits > 1)
+    float* part_ml; // [B*Hkv][splits][M][2] (m in log2 units, l)
+    int32_t Sq, ratio, M, splits;
+
+    __device__ __forceinline__ _Float16* row(int b, int kvh, int col) const {
+        const int ho = col / Sq;
+        return o + b * o_sb + (kvh * ratio + ho) * o_sh + (int64_t)(col - ho * Sq) * o_ss;
+    }
+};
+
+// LDS of finish_rows: half of the waves' O (rows of D + 4 floats, conflict-free
+// 16-byte accesses) and every wave's (m, l).
+constexpr int finish_lds_bytes(int D, int waves) {
+    return (waves / 2 * 32 * (D + 4) + waves * 32 * 2) * 4;
+}
+
+// Merges the O^T accumulators (32 columns, unnormalised, relative to m_run,
+// with row sums l_run per half-wave) of a workgroup's WAVES waves through
+// `lds` and writes split `split` of the group's rows: the partial, or, of one
+// split, the output.  The values go through scaled(f4, d) last (d the first of
+// the four columns).  Every wave's own use of `lds` is over on entry.
+template <int D, int WAVES, class Scaled>
+__device__ __forceinline__ void finish_rows(f16x (&oacc)[D / 32], float m_run, float l_run, char* lds,
+                                            const SplitRows& r, int b, int kvh, int bkv, int split, Scaled&& scaled) {
+    static_assert(WAVES % 2 == 0, "halves of the waves");
+    constexpr int NDT = D / 32;
+    constexpr int LDM = D + 4;
+    constexpr int MERGE = WAVES / 2; // waves whose O is in LDS at once
+    const int tid = threadIdx.x;
+    const int wave = tid >> 6;
+    const int l32 = tid & 31;
+    const int g = (tid >> 5) & 1;
+    const bool col_valid = l32 < r.M;
+    float* const sm_o = reinterpret_cast<float*>(lds); // [MERGE][32][LDM]
+    float* const sm_ml = sm_o + MERGE * 32 * LDM;      // [WAVES][32][2]
+    __syncthreads();
+    const float l_tot = pair_sum(l_run);
+    if (g == 0) {
+        sm_ml[(wave * 32 + l32) * 2 + 0] = m_run;
+        sm_ml[(wave * 32 + l32) * 2 + 1] = l_tot;
+    }
+    __syncthreads();
+    float mref = -INFINITY, lsum = 0.0f; // of column l32 over the waves
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+        if (sm_ml[(w * 32 + l32) * 2 + 1] > 0.0f) {
+            mref = fmaxf(mref, sm_ml[(w * 32 + l32) * 2 + 0]);
+        }
+    }
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+        const float lw = sm_ml[(w * 32 + l32) * 2 + 1];
+        if (lw > 0.0f) {
+            lsum += lw * fast_exp2(sm_ml[(w * 32 + l32) * 2 + 0] - mref);
+        }
+    }
+    const bool whole = r.splits == 1;
+    float scale_w = (l_tot > 0.0f) ? fast_exp2(m_run - mref) : 0.0f;
+    if (whole) {
+        scale_w *= lsum > 0.0f ? 1.0f / lsum : 0.0f;
+    }
+#pragma unroll
+    for (int dt = 0; dt < NDT; dt++) {
+        oacc[dt] *= scale_w;
+    }
+    // the upper half of the waves through LDS into the lower half, then those
+    // through LDS into whole rows
+    float* const my_o = &sm_o[((wave % MERGE) * 32 + l32) * LDM + 4 * g];
+    auto put_o = [&]() {
+        if (col_valid) {
+#pragma unroll
+            for (int dt = 0; dt < NDT; dt++) {
+#pragma unroll
+                for (int e4 = 0; e4 < 4; e4++) {
+                    *reinterpret_cast<f4*>(my_o + 32 * dt + 8 * e4) =
+                        f4{oacc[dt][4 * e4], oacc[dt][4 * e4 + 1], oacc[dt][4 * e4 + 2], oacc[dt][4 * e4 + 3]};
+                }
+            }
+        }
+    };
+    if (wave >= MERGE) {
+        put_o();
+    }
+    __syncthreads();
+    if (wave < MERGE && col_valid) {
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++) {
+#pragma unroll
+            for (int e4 = 0; e4 < 4; e4++) {
+                const f4 x = *reinterpret_cast<const f4*>(my_o + 32 * dt + 8 * e4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    oacc[dt][4 * e4 + e] += x[e];
+                }
+            }
+        }
+    }
+    if (wave < MERGE) {
+        put_o(); // its own slot, read above by the same lanes
+    }
+    const int64_t part = ((int64_t)bkv * r.splits + split) * r.M;
+    if (!whole && tid < r.M) { // M <= 32: the threads that hold mref, lsum of column tid
+        r.part_ml[(part + tid) * 2 + 0] = mref;
+        r.part_ml[(part + tid) * 2 + 1] = lsum;
+    }
+    __syncthreads();
+    for (int e = tid; e < r.M * (D / 4); e += 64 * WAVES) {
+        const int col = e / (D / 4);
+        const int d = 4 * (e - col * (D / 4));
+        f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < MERGE; w++) {
+            acc += *reinterpret_cast<const f4*>(&sm_o[(w * 32 + col) * LDM + d]);
+        }
+        acc = scaled(acc, d);
+        if (whole) {
+            *reinterpret_cast<h4*>(r.row(b, kvh, col) + d) = __builtin_convertvector(acc, h4);
+        } else {
+            *reinterpret_cast<f4*>(&r.part_o[(part + col) * D + d]) = acc;
+        }
+    }
+}
 
 // Partials of one row: split s has its O at part_o[s * so] and its (m, l) at
 // part_ml[s * sml].

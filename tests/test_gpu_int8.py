@@ -421,3 +421,64 @@ def test_int8_quantised_p_against_oracle_integers(gpu, oracle_lib, d, per_token)
     # within 9.2e-5 of a tie
     assert worst <= 5e-4
     assert n_diff <= 2e-5 * diff.size
+
+
+# b, hq, hkv, sq, sk, d, causal, window, scales: the split-K decode kernel at
+# the edges of its 64-key tiles, its rounds of eight of them and its 32 columns
+DECODE_CASES = [(1, 8, 2, 1, sk, d, False, -1, sc) for d in (64, 128)
+                for sk, sc in ((1, "tensor"), (63, "token"), (65, "channel"), (512, "vtoken"), (513, "token"))] + [
+    (2, 8, 8, 1, 3000, 128, False, -1, "channel"),
+    (1, 32, 1, 1, 9001, 128, False, -1, "token"),
+    (2, 16, 4, 8, 2049, 64, True, -1, "vtoken"),
+    (1, 6, 2, 5, 1500, 128, True, 700, "channel"),
+    (1, 4, 2, 3, 4000, 64, False, 500, "tensor"),
+    (1, 2, 2, 9, 4, 128, True, -1, "token"),  # rows without keys
+]
+
+
+@pytest.mark.parametrize("case", DECODE_CASES, ids=["b{}h{}kv{}q{}k{}d{}c{:d}w{}{}".format(*c) for c in DECODE_CASES])
+def test_int8_decode_vs_emulation(gpu, oracle_lib, case):
+    """INT8 bar against the kernel-exact emulation, whose running maximum goes
+    through the keys in order: a wave of the split-K kernel takes every eighth
+    block, so its P may be rounded to a finer step (never a coarser one), which
+    the bar for a rounding of 1/127 covers.  K and V are views into one cache
+    with a row stride of 2 Hkv D; a second call gives the same bits."""
+    import rdnattention as ra
+
+    b, hq, hkv, sq, sk, d, causal, window, scales = case
+    log(f"[int8 decode] {case}")
+    rng = np.random.default_rng(41)
+    f = rng.standard_normal
+    qi, qs = oracle.quant_pertoken(f((b, hq, sq, d)).astype(np.float32))
+    ki, ks = oracle.quant_pertoken(f((b, hkv, sk, d)).astype(np.float32))
+    vi = rng.integers(-127, 128, (b, hkv, sk, d), dtype=np.int8)
+    vs = 1.0 / 127.0
+    if scales == "tensor":
+        qs, ks = float(qs.mean()), float(ks.mean())
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    cache = torch.empty(b, sk, 2, hkv, d, dtype=torch.int8, device=gpu)
+    kd, vd = cache[:, :, 0].transpose(1, 2), cache[:, :, 1].transpose(1, 2)
+    kd.copy_(t(ki))
+    vd.copy_(t(vi))
+    extra = {}
+    if scales == "channel":
+        vch = rng.uniform(0.2, 1.0, (b, hkv, d)).astype(np.float32)
+        extra["v_channel"] = t(vch)
+    elif scales == "vtoken":
+        vtok = rng.uniform(0.2, 1.0, (b, hkv, sk)).astype(np.float32)
+        extra["v_token"] = t(vtok)
+    scale = lambda x: x if isinstance(x, float) else t(x)  # noqa: E731
+    outs = [torch.full((b, hq, sq, d), float("nan"), dtype=torch.float16, device=gpu) for _ in range(2)]
+    for o in outs:
+        ra.attention_int8_forward_into(t(qi), kd, vd, o, scale(qs), scale(ks), vs, is_causal=causal,
+                                       window_size=window, **extra)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    got = outs[0].float().cpu().numpy()
+    emu = oracle.attention_int8(qi, ki, vi, qs, ks, vs, causal=causal, window=window,
+                                v_token=vtok if scales == "vtoken" else None)
+    if scales == "channel":
+        emu = emu * np.repeat(vch, hq // hkv, axis=1)[:, :, None, :]
+    assert np.isfinite(got).all()
+    mx, _, _ = errors(got, emu)
+    assert mx <= I8_MAX_ABS, f"max_abs {mx:.3e}"
