@@ -113,7 +113,7 @@ __global__ __launch_bounds__(DecCfg<D>::THREADS, DecCfg<D>::WAVES_PER_SIMD) void
     const int kvh = bkv - b * p.Hkv;
 
     // column l32 <-> (query head, query row)
-    const bool col_valid = l32 < p.out.M;
+    const bool col_valid = l32 < p.out.ratio * p.out.Sq;
     const int hoff = col_valid ? l32 / p.out.Sq : 0;
     const int q = col_valid ? l32 - hoff * p.out.Sq : 0;
     const int h = kvh * p.out.ratio + hoff;
@@ -293,10 +293,10 @@ __global__ __launch_bounds__(DecCfg<D>::THREADS, DecCfg<D>::WAVES_PER_SIMD) void
         }
     }
     __builtin_amdgcn_s_waitcnt(0); // all DMAs and LDS traffic of this wave done
-    finish_rows<D, C::WAVES>(oacc, m_run, l_run, dsm, p.out, b, kvh, bkv, split, [](f4 x, int) { return x; });
+    finish_rows<D, C::WAVES>(oacc, m_run, l_run, dsm, p.out, b, kvh, split, [](f4 x, int) { return x; });
 }
 
-// One workgroup per output row (b, kv head, column): log-sum-exp merge of the
+// One workgroup per output row: log-sum-exp merge of the
 // splits, normalised in fp32, rounded once to fp16.  Merging inside the split
 // kernel instead, by the last workgroup of each group to arrive, measured
 // slower although it saves this launch (B = 4 Hq = 32 Hkv = 8 Sk = 4096 D =
@@ -304,16 +304,14 @@ __global__ __launch_bounds__(DecCfg<D>::THREADS, DecCfg<D>::WAVES_PER_SIMD) void
 // device-scope release and acquire it needs write back and invalidate whole
 // L2s.
 template <int T>
-__global__ __launch_bounds__(T) void fa_decode_combine(SplitRows r, int32_t Hkv, int32_t D) {
+__global__ __launch_bounds__(T) void fa_decode_combine(SplitRows r, int32_t D) {
     __shared__ __attribute__((aligned(16))) float lds[merge_lds_floats(kMaxSplits, T)];
-    const int row = blockIdx.x; // (b * Hkv + kvh) * M + col
-    const int col = row % r.M;
-    const int bkv = row / r.M;
-    const int b = bkv / Hkv;
-    const int kvh = bkv - b * Hkv;
-    _Float16* orow = r.row(b, kvh, col);
-    const int64_t first = (int64_t)bkv * r.splits * r.M + col;
-    const SplitParts parts{r.part_o + first * D, r.part_ml + first * 2, (int64_t)r.M * D, 2 * r.M, r.splits, D};
+    const int row = blockIdx.x; // (b * Hq + h) * Sq + q
+    const int bh = row / r.Sq;
+    const int b = bh / r.Hq;
+    _Float16* orow = r.row(b, bh - b * r.Hq, row - bh * r.Sq);
+    const SplitParts parts{r.part_o + (int64_t)row * D, r.part_ml + (int64_t)row * 2, r.n_rows * D, 2 * r.n_rows,
+                           r.splits, D};
     merge_splits<T>(parts, lds, [&](int d, f4 x) {
         *reinterpret_cast<h4*>(orow + d) = __builtin_convertvector(x, h4);
     });
@@ -358,11 +356,7 @@ bool splitk_built(const AttnArgs& a) {
 }
 
 size_t splitk_partial_bytes(const AttnArgs& a, int splits) {
-    if (splits <= 1) {
-        return 0;
-    }
-    const size_t n_part = (size_t)a.B * a.Hkv * splits * ((a.Hq / a.Hkv) * a.Sq);
-    return n_part * (a.D + 2) * sizeof(float);
+    return splits <= 1 ? 0 : (size_t)a.B * a.Hq * a.Sq * splits * (a.D + 2) * sizeof(float);
 }
 
 SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
@@ -424,23 +418,24 @@ int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::s
     });
 }
 
-int splitk_begin(const AttnArgs& a, const SplitKPlan& plan, StreamScratch& ws, hipStream_t stream, SplitRows& r,
+int splitk_begin(const AttnArgs& a, int splits, StreamScratch& ws, hipStream_t stream, SplitRows& r,
                  std::string& err) {
     r.o = static_cast<_Float16*>(a.o);
     r.o_sb = a.os[0];
     r.o_sh = a.os[1];
     r.o_ss = a.os[2];
+    r.n_rows = (int64_t)a.B * a.Hq * a.Sq;
     r.Sq = a.Sq;
+    r.Hq = a.Hq;
     r.ratio = a.Hq / a.Hkv;
-    r.M = r.ratio * a.Sq;
-    r.splits = plan.splits;
+    r.splits = splits;
     // every partial is written by its split's workgroup before the combine
     // reads it, so the buffer needs no clearing
-    if (ws.alloc(splitk_partial_bytes(a, plan.splits), stream, err) != 0) {
+    if (ws.alloc(splitk_partial_bytes(a, splits), stream, err) != 0) {
         return -1;
     }
     r.part_o = static_cast<float*>(ws.ptr);
-    r.part_ml = plan.splits > 1 ? r.part_o + (size_t)a.B * a.Hkv * r.splits * r.M * a.D : nullptr;
+    r.part_ml = splits > 1 ? r.part_o + (size_t)splits * r.n_rows * a.D : nullptr;
     return 0;
 }
 
@@ -448,11 +443,12 @@ int splitk_finish(const AttnArgs& a, const SplitRows& r, hipStream_t stream, std
     if (r.splits == 1) {
         return 0;
     }
-    const dim3 grid((uint32_t)(a.B * a.Hkv * r.M));
-    if (r.splits >= 8) {
-        hipLaunchKernelGGL(fa_decode_combine<256>, grid, dim3(256), 0, stream, r, a.Hkv, a.D);
+    // four waves per row where few rows have many splits
+    const dim3 grid((uint32_t)r.n_rows);
+    if (r.splits >= 8 && r.n_rows < 2048) {
+        hipLaunchKernelGGL(fa_decode_combine<256>, grid, dim3(256), 0, stream, r, a.D);
     } else {
-        hipLaunchKernelGGL(fa_decode_combine<64>, grid, dim3(64), 0, stream, r, a.Hkv, a.D);
+        hipLaunchKernelGGL(fa_decode_combine<64>, grid, dim3(64), 0, stream, r, a.D);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -496,7 +492,7 @@ int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::stri
     p.keys_per_split = plan.keys_per_split;
     p.key0 = plan.key0;
     StreamScratch ws(ScratchUse::SplitKPartials, region);
-    if (splitk_begin(a, plan, ws, stream, p.out, err) != 0 ||
+    if (splitk_begin(a, plan.splits, ws, stream, p.out, err) != 0 ||
         for_dim(a.D, [&](auto d) { return launch_decode<decltype(d)::value>(p, a.B * a.Hkv, stream, err); }) != 0) {
         return -1;
     }

@@ -28,6 +28,7 @@
 #include "fa_host.hpp"
 #include "fa_internal.hpp"
 #include "fa_prefill.hpp"
+#include "fa_splitk.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -112,8 +113,11 @@ struct PPCfg {
 // the MFMA output is the exponent itself: p = 2^acc with no per-score
 // multiply-add.  The accumulators are shifted only when the running max
 // moves.  Without PRE, Q carries only the sign and p = 2^(acc c - m).
-template <int D, bool PRE>
-__global__ __launch_bounds__(kPPThreads, 1) void fa_fwd_f16_pp(PrefillParams p) {
+//
+// SPLIT: every row tile's key tiles are dealt to p.splits workgroups, which
+// write partials for the combine kernel.
+template <int D, bool PRE, bool SPLIT>
+__device__ __forceinline__ void pp_body(PrefillParams p) {
     using C = PPCfg<D>;
     // sK[slot], sV[slot], sQ
     __shared__ __attribute__((aligned(16))) _Float16 smem[2 * C::TILE_K + 2 * C::TILE_V + C::TILE_Q];
@@ -160,8 +164,11 @@ __global__ __launch_bounds__(kPPThreads, 1) void fa_fwd_f16_pp(PrefillParams p) 
     // prologue may overwrite LDS. Otherwise the grid has one workgroup per
     // row tile.
     auto run_tile = [&](const int wg) {
-        int hg, rt;
-        wg_tile(wg, p.n_head_groups, p.n_row_tiles, p.hg_chunk, hg, rt);
+        int hg, rt, split = 0;
+        wg_tile(wg, p.n_head_groups, SPLIT ? p.n_row_tiles * p.splits : p.n_row_tiles, p.hg_chunk, hg, rt);
+        if constexpr (SPLIT) {
+            split_row_tile(p, rt, split);
+        }
         const int per_b = p.Hkv * p.groups_per_kv;
         const int b = hg / per_b;
         const int rem = hg - b * per_b;
@@ -264,6 +271,9 @@ __global__ __launch_bounds__(kPPThreads, 1) void fa_fwd_f16_pp(PrefillParams p) 
         if (khi >= klo) {
             t_begin = klo / kBN;
             n = khi / kBN + 1 - t_begin;
+        }
+        if constexpr (SPLIT) {
+            split_key_tiles(p.splits, split, t_begin, n);
         }
         const int Sk = p.mask.sk;
         const uint32_t k_row_b = (uint32_t)(p.k_ss * 2), v_row_b = (uint32_t)(p.v_ss * 2);
@@ -646,8 +656,14 @@ __global__ __launch_bounds__(kPPThreads, 1) void fa_fwd_f16_pp(PrefillParams p) 
             }
         }
 
-        // O = O^T / l, through this wave's sQ slot (free since read_q)
-        if (wave_active) {
+        if constexpr (SPLIT) {
+            const float l = pair_sum(l_run);
+            if (wave_active && q < p.Sq) {
+                const int64_t row = split * p.n_rows + ((int64_t)b * p.Hkv * p.ratio + h) * p.Sq + q;
+                store_partial(oacc, m_run, l, g == 0, p.part_o, p.part_ml, row, D, 0, g);
+            }
+        } else if (wave_active) {
+            // O = O^T / l, through this wave's sQ slot (free since read_q)
             const float l = pair_sum(l_run);
             const float inv = l > 0.0f ? 1.0f / l : 0.0f;
             store_o_tile<D, C::LDQ>(oacc, [&](int) { return f4{inv, inv, inv, inv}; }, sQ + wave * 32 * C::LDQ,
@@ -671,20 +687,30 @@ __global__ __launch_bounds__(kPPThreads, 1) void fa_fwd_f16_pp(PrefillParams p) 
 }
 
 template <int D, bool PRE>
+__global__ __launch_bounds__(kPPThreads, 1) void fa_fwd_f16_pp(PrefillParams p) {
+    pp_body<D, PRE, false>(p);
+}
+
+template <int D, bool PRE>
+__global__ __launch_bounds__(kPPThreads, 1) void fa_fwd_f16_pp_split(PrefillParams p) {
+    pp_body<D, PRE, true>(p);
+}
+
+template <int D, bool PRE>
 int launch_pp_as(const PrefillParams& p, int64_t n_wg, hipStream_t stream, std::string& err) {
     // persistent: as many workgroups as the device holds at once, each
     // walking its share of the n_wg row tiles
+    auto* const kernel = p.splits > 1 ? &fa_fwd_f16_pp_split<D, PRE> : &fa_fwd_f16_pp<D, PRE>;
     int64_t grid = n_wg;
     if (PPCfg<D>::PERSIST) {
-        const int64_t resident =
-            resident_workgroups(reinterpret_cast<const void*>(&fa_fwd_f16_pp<D, PRE>), kPPThreads, err);
+        const int64_t resident = resident_workgroups(reinterpret_cast<const void*>(kernel), kPPThreads, err);
         if (resident <= 0) {
             return -1;
         }
         grid = std::min(n_wg, resident);
     }
     KernelTimerGuard timer(stream);
-    hipLaunchKernelGGL((fa_fwd_f16_pp<D, PRE>), dim3((uint32_t)grid), dim3(kPPThreads), 0, stream, p);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(kPPThreads), 0, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         err = hipGetErrorString(e);
@@ -727,7 +753,65 @@ float softmax_log2_scale(float scale) {
     return std::max(std::fabs(scale) * kLog2e, 1e-30f);
 }
 
-int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err) {
+// Query heads per prefill workgroup (G | Hq/Hkv, G <= 4).
+static int prefill_group(const AttnArgs& a) {
+    const int ratio = a.Hq / a.Hkv;
+    return ratio % 4 == 0 ? 4 : (ratio % 2 == 0 ? 2 : 1);
+}
+
+int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, size_t max_partials) {
+    // Too few workgroups for the CUs and many key tiles for each: split the
+    // keys, by the least modelled time.  A workgroup takes about 5 us beside
+    // its key tiles; the partials are written and read at about 2.5 MB/us, and
+    // the combine launch adds about 5 us.  Measured, us a call, unsplit against
+    // split: B1 Hq32 Hkv8 Sq256 Sk16640 D128 355 / 80 (8 splits, 79 of them
+    // the 33.5 MB launch); Sq64 Sk4096 92 / 27; B2 Sq256 Sk8192 183 / 85; B1
+    // Hq16 Hkv4 Sq128 Sk2000 D64 37 / 19.  Whole prompts this small stay
+    // unsplit (1 x 8 heads, S 512, D64: 13.9 / 18.3; S 1024 causal 22.8 /
+    // 23.2).  With more workgroups than CUs the persistent grid balances them.
+    const int G = prefill_group(a);
+    const int rows = wg_rows / G;
+    const int64_t row_tiles = (a.Sq + rows - 1) / rows;
+    const int64_t n_wg = row_tiles * a.B * (a.Hq / G);
+    if (n_wg > 256) {
+        return 1;
+    }
+    const MaskSpec mask{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
+    int64_t tiles = 0; // of the longest row tile: the last one, or one from the middle under a window
+    for (int64_t rt : {row_tiles - 1, row_tiles / 2, int64_t{0}}) {
+        int lo, hi;
+        visible_key_range(mask, (int)(rt * rows), (int)std::min<int64_t>((rt + 1) * rows, a.Sq) - 1, lo, hi);
+        tiles = std::max<int64_t>(tiles, hi >= lo ? hi / kBN + 1 - lo / kBN : 0);
+    }
+    int best_s = 1;
+    double best = 0.0;
+    for (int64_t s = 1; s <= std::min<int64_t>(tiles / 2, kMaxSplits); s++) {
+        const size_t partials = splitk_partial_bytes(a, (int)s);
+        if (region_bytes(partials) > max_partials) {
+            break;
+        }
+        const double rounds = (double)((n_wg * s + 255) / 256);
+        const double t = rounds * (5.0 + (double)((tiles + s - 1) / s) * tile_us) +
+                         (s > 1 ? 5.0 + 2.0 * (double)partials / 2.5e6 : 0.0);
+        if (s == 1 || t < best) {
+            best = t;
+            best_s = (int)s;
+        }
+    }
+    return best_s;
+}
+
+// Splits of an FP16 prefill call.  Up to D = 256; a 64-key tile takes about
+// 1.4 us at D = 128 with 256 rows, or at D = 256 with 128.
+static int f16_prefill_splits(const AttnArgs& a, size_t max_partials) {
+    if (a.D > 256) {
+        return 1;
+    }
+    return a.D > 128 ? prefill_splits(a, kKPairRows, 0.4 + 1.0 * a.D / 256, max_partials)
+                     : prefill_splits(a, 32 * kPPWaves, 0.4 + 1.0 * a.D / 128, max_partials);
+}
+
+int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err, ScratchRegion* region) {
     PrefillParams p{};
     p.q = static_cast<const _Float16*>(a.q);
     p.k = static_cast<const _Float16*>(a.k);
@@ -755,7 +839,7 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
     // every kernel holds G query heads of one kv head (G | Hq/Hkv, G <= 4)
     // and 128 (query, head) rows per workgroup: 8 waves of 32 rows (D <= 128)
     // or 4 pairs of waves of 32 rows (D > 128)
-    p.G = (p.ratio % 4 == 0) ? 4 : ((p.ratio % 2 == 0) ? 2 : 1);
+    p.G = prefill_group(a);
     p.rows_per_wg = (kpair ? kKPairRows : dpair ? kDPairRows : 32 * kPPWaves) / p.G;
     p.n_row_tiles = (a.Sq + p.rows_per_wg - 1) / p.rows_per_wg;
     p.groups_per_kv = p.ratio / p.G;
@@ -767,7 +851,8 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
     p.mask = MaskSpec{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
     p.rope_q = rope_q ? 1 : 0;
 
-    const int64_t n_wg = (int64_t)p.n_row_tiles * p.n_head_groups;
+    p.splits = f16_prefill_splits(a, region != nullptr ? region->bytes - region->used : SIZE_MAX);
+    const int64_t n_wg = (int64_t)p.n_row_tiles * p.n_head_groups * p.splits;
     p.n_items = (int32_t)std::min<int64_t>(n_wg, INT32_MAX);
     if (n_wg <= 0) {
         err = "empty launch grid";
@@ -777,21 +862,31 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
         err = "launch grid too large";
         return -1;
     }
+    SplitRows out{};
+    StreamScratch ws(ScratchUse::SplitKPartials, region);
+    if (splitk_begin(a, p.splits, ws, stream, out, err) != 0) {
+        return -1;
+    }
+    p.part_o = out.part_o;
+    p.part_ml = out.part_ml;
+    p.n_rows = out.n_rows;
+    int rc = -1;
     switch (a.D) {
-    case 32: return launch_pp<32>(p, n_wg, stream, err);
-    case 64: return launch_pp<64>(p, n_wg, stream, err);
-    case 96: return launch_pp<96>(p, n_wg, stream, err);
-    case 128: return launch_pp<128>(p, n_wg, stream, err);
-    default: break;
+    case 32: rc = launch_pp<32>(p, n_wg, stream, err); break;
+    case 64: rc = launch_pp<64>(p, n_wg, stream, err); break;
+    case 96: rc = launch_pp<96>(p, n_wg, stream, err); break;
+    case 128: rc = launch_pp<128>(p, n_wg, stream, err); break;
+    default:
+        if (kpair) {
+            rc = launch_kpair(p, (int)a.D, n_wg, stream, err);
+        } else if (dpair) {
+            rc = launch_dpair(p, (int)a.D, n_wg, stream, err);
+        } else {
+            err = "unsupported head_dim (multiples of 32 from 32 to 512)";
+        }
+        break;
     }
-    if (kpair) {
-        return launch_kpair(p, (int)a.D, n_wg, stream, err);
-    }
-    if (dpair) {
-        return launch_dpair(p, (int)a.D, n_wg, stream, err);
-    }
-    err = "unsupported head_dim (multiples of 32 from 32 to 512)";
-    return -1;
+    return rc != 0 ? rc : splitk_finish(a, out, stream, err);
 }
 
 bool splitk_supported(const AttnArgs& a);
@@ -806,13 +901,16 @@ bool prefer_splitk(const AttnArgs& a) {
 int64_t fwd_f16_scratch_bytes(const AttnArgs& a, F16Path path, std::string& err) {
     const bool splitk = path == F16Path::SplitK || (path == F16Path::Auto && prefer_splitk(a));
     size_t bytes = 0;
+    auto left = [&]() { return kNoAllocBytes - std::min(bytes, kNoAllocBytes); };
     if (a.has_rope && a.Sk > 0) {
         bytes += region_bytes((size_t)a.B * a.Hkv * a.Sk * a.D * sizeof(_Float16));
     }
-    if (splitk && splitk_built(a)) {
-        // fewer splits where the partials would not fit beside the K copy
+    // fewer splits where the partials would not fit beside the K copy
+    if (!splitk) {
+        bytes += region_bytes(splitk_partial_bytes(a, f16_prefill_splits(a, left())));
+    } else if (splitk_built(a)) {
         SplitKPlan plan;
-        if (splitk_plan(a, kNoAllocBytes - std::min(bytes, kNoAllocBytes), plan, err) != 0) {
+        if (splitk_plan(a, left(), plan, err) != 0) {
             return -1;
         }
         bytes += region_bytes(splitk_partial_bytes(a, plan.splits));
@@ -844,7 +942,7 @@ int fwd_f16(const AttnArgs& in, F16Path path, hipStream_t stream, std::string& e
         a.ks[2] = a.D;
     }
     return splitk ? fwd_f16_splitk(a, a.has_rope != 0, stream, err, region)
-                  : fwd_f16_prefill(a, a.has_rope != 0, stream, err);
+                  : fwd_f16_prefill(a, a.has_rope != 0, stream, err, region);
 }
 
 } // namespace rdna_amd

@@ -121,7 +121,8 @@ struct DmaPair {
 
 // The work of one half (C0, W) of every pair, over the persistent grid's
 // row tiles.  Both halves of a group pass the same barriers.
-template <int D, bool PRE, int C0, int W>
+// SPLIT: see fa_fwd_f16_pp_split.
+template <int D, bool PRE, bool SPLIT, int C0, int W>
 __device__ __forceinline__ void kpair_half(const PrefillParams& p, char* smem, const int wave) {
     using C = KPCfg<D>;
     constexpr int HALF = C0 == 0 ? 0 : 1;
@@ -173,8 +174,11 @@ __device__ __forceinline__ void kpair_half(const PrefillParams& p, char* smem, c
     auto stages = [&](int it) { return stager && (32 % C::RPI == 0 || srow + C::RPI * it < 32); };
 
     auto run_tile = [&](const int wg) {
-        int hg, rt;
-        wg_tile(wg, p.n_head_groups, p.n_row_tiles, p.hg_chunk, hg, rt);
+        int hg, rt, split = 0;
+        wg_tile(wg, p.n_head_groups, SPLIT ? p.n_row_tiles * p.splits : p.n_row_tiles, p.hg_chunk, hg, rt);
+        if constexpr (SPLIT) {
+            split_row_tile(p, rt, split);
+        }
         const int per_b = p.Hkv * p.groups_per_kv;
         const int b = hg / per_b;
         const int rem = hg - b * per_b;
@@ -198,6 +202,9 @@ __device__ __forceinline__ void kpair_half(const PrefillParams& p, char* smem, c
         if (khi >= klo) {
             t_begin = klo / kKPBN;
             n = khi / kKPBN + 1 - t_begin;
+        }
+        if constexpr (SPLIT) {
+            split_key_tiles(p.splits, split, t_begin, n);
         }
         // Key-tile walk: step x visits tile T(x) = t_begin + (x + off) mod n.
         // Under a sliding window the bands of consecutive row tiles start at
@@ -672,6 +679,17 @@ __device__ __forceinline__ void kpair_half(const PrefillParams& p, char* smem, c
         // half stores 16 of those rows whole, 16 bytes per lane, non-temporal
         // (O is not read again; streaming it past the L2 keeps the K/V tiles
         // that other row tiles reuse resident).
+        if constexpr (SPLIT) {
+            const float l = pair_sum(l_run);
+            if (wave_active && q < p.Sq) {
+                const int64_t row = split * p.n_rows + ((int64_t)b * p.Hkv * p.ratio + h) * p.Sq + q;
+                store_partial(oacc, m_run, l, HALF == 0 && g == 0, p.part_o, p.part_ml, row, D, C0, g);
+            }
+            if constexpr (C::PERSIST) {
+                __syncthreads(); // the next row tile's prologue writes the K/V area
+            }
+            return;
+        }
         _Float16* const oslot = sKs + pair * 32 * C::LDO;
         if (wave_active) {
             const float l = pair_sum(l_run);
@@ -722,8 +740,8 @@ __device__ __forceinline__ void kpair_half(const PrefillParams& p, char* smem, c
     }
 }
 
-template <int D, bool PRE>
-__global__ __launch_bounds__(kKPThreads, 1) void fa_fwd_f16_kpair(PrefillParams p) {
+template <int D, bool PRE, bool SPLIT>
+__device__ __forceinline__ void kpair_body(PrefillParams p) {
     using C = KPCfg<D>;
     __shared__ __attribute__((aligned(16))) char smem[C::SMEM_BYTES];
     // The branch between the halves must be wave-uniform (both sides pass
@@ -732,26 +750,36 @@ __global__ __launch_bounds__(kKPThreads, 1) void fa_fwd_f16_kpair(PrefillParams 
     // moves to scalar registers and the kernel spills).
     const int wave = threadIdx.x >> 6;
     if (__builtin_amdgcn_readfirstlane(wave & 1) == 0) {
-        kpair_half<D, PRE, 0, C::DA>(p, smem, wave);
+        kpair_half<D, PRE, SPLIT, 0, C::DA>(p, smem, wave);
     } else {
-        kpair_half<D, PRE, C::DA, C::DB>(p, smem, wave);
+        kpair_half<D, PRE, SPLIT, C::DA, C::DB>(p, smem, wave);
     }
+}
+
+template <int D, bool PRE>
+__global__ __launch_bounds__(kKPThreads, 1) void fa_fwd_f16_kpair(PrefillParams p) {
+    kpair_body<D, PRE, false>(p);
+}
+
+template <int D, bool PRE>
+__global__ __launch_bounds__(kKPThreads, 1) void fa_fwd_f16_kpair_split(PrefillParams p) {
+    kpair_body<D, PRE, true>(p);
 }
 
 template <int D, bool PRE>
 int launch_kpair_as(const PrefillParams& p, int64_t n_wg, hipStream_t stream, std::string& err) {
     // persistent: as many workgroups as the device holds at once
+    auto* const kernel = p.splits > 1 ? &fa_fwd_f16_kpair_split<D, PRE> : &fa_fwd_f16_kpair<D, PRE>;
     int64_t grid = n_wg;
     if (KPCfg<D>::PERSIST) {
-        const int64_t resident =
-            resident_workgroups(reinterpret_cast<const void*>(&fa_fwd_f16_kpair<D, PRE>), kKPThreads, err);
+        const int64_t resident = resident_workgroups(reinterpret_cast<const void*>(kernel), kKPThreads, err);
         if (resident <= 0) {
             return -1;
         }
         grid = std::min(n_wg, resident);
     }
     KernelTimerGuard timer(stream);
-    hipLaunchKernelGGL((fa_fwd_f16_kpair<D, PRE>), dim3((uint32_t)grid), dim3(kKPThreads), 0, stream, p);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(kKPThreads), 0, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         err = hipGetErrorString(e);

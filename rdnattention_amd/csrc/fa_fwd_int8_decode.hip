@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kI8DecThreads, D == 64 && !VTOK ? 4 : 2) void fa_fw
     const int kvh = bkv - b * p.Hkv;
 
     // column l32 <-> (query head, query row)
-    const bool col_valid = l32 < pp.out.M;
+    const bool col_valid = l32 < p.ratio * p.Sq;
     const int hoff = col_valid ? l32 / p.Sq : 0;
     const int q = col_valid ? l32 - hoff * p.Sq : 0;
     const int h = kvh * p.ratio + hoff;
@@ -355,7 +355,7 @@ __global__ __launch_bounds__(kI8DecThreads, D == 64 && !VTOK ? 4 : 2) void fa_fw
     __builtin_amdgcn_s_waitcnt(0); // all DMAs and LDS traffic of this wave done
     // O in units of pq v, l in units of 1/127
     const float* vch = p.vch != nullptr ? p.vch + ((int64_t)b * p.Hkv + kvh) * D : nullptr;
-    finish_rows<D, kI8DecWaves>(oacc, m_run, l_run, dsm, pp.out, b, kvh, bkv, split, [&](f4 x, int d) {
+    finish_rows<D, kI8DecWaves>(oacc, m_run, l_run, dsm, pp.out, b, kvh, split, [&](f4 x, int d) {
         x *= p.v_scale;
         return vch != nullptr ? x * *reinterpret_cast<const f4*>(vch + d) : x;
     });
@@ -374,7 +374,7 @@ int launch_int8_decode_as(const AttnArgs& a, const Int8Params& ip, hipStream_t s
     p.keys_per_split = plan.keys_per_split;
     p.key0 = plan.key0;
     StreamScratch ws(ScratchUse::SplitKPartials);
-    if (splitk_begin(a, plan, ws, stream, p.out, err) != 0) {
+    if (splitk_begin(a, plan.splits, ws, stream, p.out, err) != 0) {
         return -1;
     }
     {

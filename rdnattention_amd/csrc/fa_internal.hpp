@@ -102,7 +102,8 @@ class KernelTimerGuard {
 int64_t resident_workgroups(const void* kernel, int threads, std::string& err);
 
 // Launchers.  `region`, when given, supplies every scratch buffer.
-int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err);
+int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err,
+                    ScratchRegion* region = nullptr);
 int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err,
                    ScratchRegion* region = nullptr);
 
@@ -122,10 +123,15 @@ int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::s
 SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
                            size_t max_partials);
 
-// Before and after a split-K launch: `r` from the arguments, with the partials
-// taken from `ws`; and the combine launch.  0, or -1 with `err`.
+// Key splits of a prefill launch whose workgroups hold wg_rows rows (of G
+// heads) and take tile_us per 64-key tile, with at most max_partials bytes of
+// partials; 1 where splitting does not pay.
+int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, size_t max_partials);
+
+// Before and after a launch of `splits` key splits: `r` from the arguments, with
+// the partials taken from `ws`; and the combine launch.  0, or -1 with `err`.
 struct SplitRows;
-int splitk_begin(const AttnArgs& a, const SplitKPlan& plan, StreamScratch& ws, hipStream_t stream, SplitRows& r,
+int splitk_begin(const AttnArgs& a, int splits, StreamScratch& ws, hipStream_t stream, SplitRows& r,
                  std::string& err);
 int splitk_finish(const AttnArgs& a, const SplitRows& r, hipStream_t stream, std::string& err);
 

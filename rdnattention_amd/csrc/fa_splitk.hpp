@@ -13,18 +13,18 @@ namespace rdna_amd {
 
 constexpr int kMaxSplits = 256; // weights of one row in the merge's LDS
 
-// Where the M = ratio * Sq rows of a (b, kv head) go: column c is query row
-// c % Sq of query head c / Sq of the group.
+// The output rows of a launch and the partials of their splits.  Row
+// (b * Hq + h) * Sq + q of split s is partial s * n_rows + row.
 struct SplitRows {
     _Float16* o;
     int64_t o_sb, o_sh, o_ss;
-    float* part_o;  // [B*Hkv][splits][M][D] unnormalised O (splits > 1)
-    float* part_ml; // [B*Hkv][splits][M][2] (m in log2 units, l)
-    int32_t Sq, ratio, M, splits;
+    float* part_o;  // [splits][n_rows][D] unnormalised O (splits > 1)
+    float* part_ml; // [splits][n_rows][2] (m in log2 units, l)
+    int64_t n_rows; // B * Hq * Sq
+    int32_t Sq, Hq, ratio, splits;
 
-    __device__ __forceinline__ _Float16* row(int b, int kvh, int col) const {
-        const int ho = col / Sq;
-        return o + b * o_sb + (kvh * ratio + ho) * o_sh + (int64_t)(col - ho * Sq) * o_ss;
+    __device__ __forceinline__ _Float16* row(int b, int h, int q) const {
+        return o + b * o_sb + h * o_sh + (int64_t)q * o_ss;
     }
 };
 
@@ -36,12 +36,13 @@ constexpr int finish_lds_bytes(int D, int waves) {
 
 // Merges the O^T accumulators (32 columns, unnormalised, relative to m_run,
 // with row sums l_run per half-wave) of a workgroup's WAVES waves through
-// `lds` and writes split `split` of the group's rows: the partial, or, of one
-// split, the output.  The values go through scaled(f4, d) last (d the first of
+// `lds` and writes split `split` of the rows of kv head `kvh` (column c is
+// query row c % Sq of head kvh * ratio + c / Sq): the partial, or, of one split,
+// the output.  The values go through scaled(f4, d) last (d the first of
 // the four columns).  Every wave's own use of `lds` is over on entry.
 template <int D, int WAVES, class Scaled>
 __device__ __forceinline__ void finish_rows(f16x (&oacc)[D / 32], float m_run, float l_run, char* lds,
-                                            const SplitRows& r, int b, int kvh, int bkv, int split, Scaled&& scaled) {
+                                            const SplitRows& r, int b, int kvh, int split, Scaled&& scaled) {
     static_assert(WAVES % 2 == 0, "halves of the waves");
     constexpr int NDT = D / 32;
     constexpr int LDM = D + 4;
@@ -50,7 +51,8 @@ __device__ __forceinline__ void finish_rows(f16x (&oacc)[D / 32], float m_run, f
     const int wave = tid >> 6;
     const int l32 = tid & 31;
     const int g = (tid >> 5) & 1;
-    const bool col_valid = l32 < r.M;
+    const int M = r.ratio * r.Sq;
+    const bool col_valid = l32 < M;
     float* const sm_o = reinterpret_cast<float*>(lds); // [MERGE][32][LDM]
     float* const sm_ml = sm_o + MERGE * 32 * LDM;      // [WAVES][32][2]
     __syncthreads();
@@ -118,13 +120,14 @@ __device__ __forceinline__ void finish_rows(f16x (&oacc)[D / 32], float m_run, f
     if (wave < MERGE) {
         put_o(); // its own slot, read above by the same lanes
     }
-    const int64_t part = ((int64_t)bkv * r.splits + split) * r.M;
-    if (!whole && tid < r.M) { // M <= 32: the threads that hold mref, lsum of column tid
+    // the group's rows are consecutive
+    const int64_t part = split * r.n_rows + ((int64_t)b * r.Hq + kvh * r.ratio) * r.Sq;
+    if (!whole && tid < M) { // M <= 32: the threads that hold mref, lsum of column tid
         r.part_ml[(part + tid) * 2 + 0] = mref;
         r.part_ml[(part + tid) * 2 + 1] = lsum;
     }
     __syncthreads();
-    for (int e = tid; e < r.M * (D / 4); e += 64 * WAVES) {
+    for (int e = tid; e < M * (D / 4); e += 64 * WAVES) {
         const int col = e / (D / 4);
         const int d = 4 * (e - col * (D / 4));
         f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -134,7 +137,8 @@ __device__ __forceinline__ void finish_rows(f16x (&oacc)[D / 32], float m_run, f
         }
         acc = scaled(acc, d);
         if (whole) {
-            *reinterpret_cast<h4*>(r.row(b, kvh, col) + d) = __builtin_convertvector(acc, h4);
+            const int ho = col / r.Sq;
+            *reinterpret_cast<h4*>(r.row(b, kvh * r.ratio + ho, col - ho * r.Sq) + d) = __builtin_convertvector(acc, h4);
         } else {
             *reinterpret_cast<f4*>(&r.part_o[(part + col) * D + d]) = acc;
         }

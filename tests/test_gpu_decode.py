@@ -147,3 +147,37 @@ def test_auto_decode_vs_oracle(gpu, oracle_lib, case):
         assert torch.equal(outs[3], outs[0])
     assert torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
     assert_f16_parity(outs[0].float().cpu().numpy(), ref, "auto decode")
+
+
+# d, b, hq, hkv, sq, sk, causal, window, rope: prefill launches too small for
+# the CUs, whose keys are split (every head dim; one and several row tiles,
+# rows without keys, splits that end short or empty, a window)
+SPLIT_PREFILL_CASES = [(d, 1, 8, 2, 70, 1500, True, -1, False) for d in range(32, 257, 32)] + [
+    (128, 1, 8, 2, 257, 5000, True, -1, True),
+    (128, 1, 4, 4, 33, 2049, False, -1, False),
+    (64, 2, 4, 2, 300, 1111, True, 500, False),
+    (256, 1, 4, 2, 129, 2600, True, -1, True),
+    (192, 1, 4, 1, 200, 1900, False, 1000, False),
+    (96, 1, 5, 1, 1500, 900, True, -1, False),
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_PREFILL_CASES,
+                         ids=["d{}b{}h{}kv{}q{}k{}c{:d}w{}r{:d}".format(*c) for c in SPLIT_PREFILL_CASES])
+def test_split_prefill_vs_oracle(gpu, oracle_lib, case):
+    """FP16 bar against the oracle; a second call gives the same bits."""
+    d, b, hq, hkv, sq, sk, causal, window, rope = case
+    log(f"[split prefill] {case}")
+    q, k, v = seeded_inputs(51, b, hq, hkv, sq, sk, d)
+    cos = sin = cd = sd = None
+    if rope:
+        cos, sin = oracle.rope_tables(max(sq, sk), d)
+        cd, sd = torch.from_numpy(cos).to(gpu), torch.from_numpy(sin).to(gpu)
+    ref = reference_f16(q, k, v, causal, window, cos, sin)
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    outs = [torch.full_like(qd, float("nan")) for _ in range(2)]
+    for o in outs:
+        assert forward_raw(qd, kd, vd, o, causal, window, cd, sd) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    assert_f16_parity(outs[0].float().cpu().numpy(), ref, "split prefill")
