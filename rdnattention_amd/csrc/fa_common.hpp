@@ -301,6 +301,14 @@ __device__ __forceinline__ void dma_load16_nt(i32x4_t rsrc, uint32_t voff, uint3
                  : "memory", "m0");
 }
 
+// dma_load16_nt with a wave-uniform byte offset (see dma_load16_s)
+__device__ __forceinline__ void dma_load16_nt_s(i32x4_t rsrc, uint32_t voff, uint32_t soff, uint32_t lds_byte_addr) {
+    asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds"
+                 :
+                 : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_byte_addr)
+                 : "memory", "m0");
+}
+
 // Bytes of one key tile: min(rows_left, TILE_ROWS) rows of row_bytes at a
 // stride of stride_bytes (<= 2^25 and TILE_ROWS <= 64, so the result fits 32
 // bits), 0 when rows_left <= 0.

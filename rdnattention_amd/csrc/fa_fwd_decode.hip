@@ -360,7 +360,7 @@ size_t splitk_partial_bytes(const AttnArgs& a, int splits) {
 }
 
 SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
-                           size_t max_partials) {
+                           size_t max_partials, int64_t max_keys) {
     // The keys that some row sees, from a tile boundary on, are dealt to the
     // splits in whole rounds of tiles (one tile per wave).
     const MaskSpec mask{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
@@ -385,18 +385,18 @@ SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_b
     // 32, 4096: 23 (4), 19.2 (8, chosen), 25.7 (16); 8, 32768: 37 (16),
     // 29.7 (32, chosen), 33.7 (64); D = 64, 256, 2048: 27.6 (1, chosen), 33 (2).
     const int64_t rounds_of_keys = (keys + round - 1) / round;
-    double best = 0.0;
+    double best = INFINITY;
     for (int64_t s = 1; s <= std::min<int64_t>(rounds_of_keys, kMaxSplits); s++) {
         const int64_t kps = (rounds_of_keys + s - 1) / s * round;
-        if (kps * (s - 1) >= keys || region_bytes(splitk_partial_bytes(a, (int)s)) > max_partials) {
-            continue; // the last split would be empty, or the partials too large
+        if (kps > max_keys || kps * (s - 1) >= keys || region_bytes(splitk_partial_bytes(a, (int)s)) > max_partials) {
+            continue; // too many keys for a split, the last one empty, or the partials too large
         }
         const int64_t wgs = n_bkv * s;
         const int64_t waves_of_wgs = (wgs + resident - 1) / resident;
         const double rate = std::min(40e3, 6.8e6 / (double)std::min(wgs, resident)); // bytes per us
         const double t = (double)waves_of_wgs * (2.0 + (double)(std::min(kps, keys) * key_bytes) / rate) +
                          (s > 1 ? 2.0 : 0.0);
-        if (s == 1 || t < best) {
+        if (t < best) {
             best = t;
             plan.splits = (int)s;
             plan.keys_per_split = (int)kps;

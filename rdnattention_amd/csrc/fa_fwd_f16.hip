@@ -167,7 +167,7 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
         int hg, rt, split = 0;
         wg_tile(wg, p.n_head_groups, SPLIT ? p.n_row_tiles * p.splits : p.n_row_tiles, p.hg_chunk, hg, rt);
         if constexpr (SPLIT) {
-            split_row_tile(p, rt, split);
+            split_row_tile(p.n_row_tiles, rt, split);
         }
         const int per_b = p.Hkv * p.groups_per_kv;
         const int b = hg / per_b;
@@ -660,7 +660,8 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
             const float l = pair_sum(l_run);
             if (wave_active && q < p.Sq) {
                 const int64_t row = split * p.n_rows + ((int64_t)b * p.Hkv * p.ratio + h) * p.Sq + q;
-                store_partial(oacc, m_run, l, g == 0, p.part_o, p.part_ml, row, D, 0, g);
+                store_partial(oacc, m_run, l, g == 0, p.part_o, p.part_ml, row, D, 0, g,
+                              [](int) { return 1.0f; });
             }
         } else if (wave_active) {
             // O = O^T / l, through this wave's sQ slot (free since read_q)

@@ -41,6 +41,7 @@
 #include "fa_host.hpp"
 #include "fa_internal.hpp"
 #include "fa_prefill.hpp"
+#include "fa_splitk.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -177,7 +178,7 @@ __device__ __forceinline__ void kpair_half(const PrefillParams& p, char* smem, c
         int hg, rt, split = 0;
         wg_tile(wg, p.n_head_groups, SPLIT ? p.n_row_tiles * p.splits : p.n_row_tiles, p.hg_chunk, hg, rt);
         if constexpr (SPLIT) {
-            split_row_tile(p, rt, split);
+            split_row_tile(p.n_row_tiles, rt, split);
         }
         const int per_b = p.Hkv * p.groups_per_kv;
         const int b = hg / per_b;
@@ -683,7 +684,8 @@ __device__ __forceinline__ void kpair_half(const PrefillParams& p, char* smem, c
             const float l = pair_sum(l_run);
             if (wave_active && q < p.Sq) {
                 const int64_t row = split * p.n_rows + ((int64_t)b * p.Hkv * p.ratio + h) * p.Sq + q;
-                store_partial(oacc, m_run, l, HALF == 0 && g == 0, p.part_o, p.part_ml, row, D, C0, g);
+                store_partial(oacc, m_run, l, HALF == 0 && g == 0, p.part_o, p.part_ml, row, D, C0, g,
+                              [](int) { return 1.0f; });
             }
             if constexpr (C::PERSIST) {
                 __syncthreads(); // the next row tile's prologue writes the K/V area

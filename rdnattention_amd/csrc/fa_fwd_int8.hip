@@ -701,8 +701,8 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
     }
     // few query rows per kv head (one MFMA column block): split-K, at every key
     // count; the prefill kernels put 256 rows in a workgroup (B8 Hq32 Hkv8
-    // Sq1 Sk8192 D128: 32 us a call against 206)
-    if ((a.D == 64 || a.D == 128) && (int64_t)p.ratio * a.Sq <= 32) {
+    // Sq1 Sk8192 D128: 43 us a call against 205)
+    if ((a.D == 64 || a.D == 128) && int8_splitk_supported(a)) {
         return fwd_int8_splitk(a, p, stream, err);
     }
     if (a.D == 64 && p.vtok == nullptr) {

@@ -70,6 +70,7 @@ int launch_int8_f16pv(const Int8Params& p, int head_dim, bool scores, int64_t n_
 
 // Split-K decode (fa_fwd_int8_decode.hip): (Hq / Hkv) * Sq <= 32, head_dim 64
 // or 128.
+bool int8_splitk_supported(const AttnArgs& a);
 int fwd_int8_splitk(const AttnArgs& a, const Int8Params& p, hipStream_t stream, std::string& err);
 
 } // namespace rdna_amd

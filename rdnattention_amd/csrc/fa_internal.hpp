@@ -27,7 +27,7 @@ constexpr size_t region_bytes(size_t bytes) {
 
 // What a scratch buffer holds; calls keep one cached buffer per (device,
 // stream, purpose), so buffers of one call never alias.
-enum class ScratchUse : int { RotatedK = 0, SplitKPartials = 1, QuantPartials = 2 };
+enum class ScratchUse : int { RotatedK = 0, SplitKPartials = 1, QuantPartials = 2, Int8Scores = 3 };
 
 // Scratch memory for one call (scratch.cpp).  Without a region: the buffer
 // cached for (device, stream, use); a call that finds it large enough makes
@@ -119,9 +119,9 @@ int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::s
 
 // The same for any split-K kernel: `tile` keys per wave tile, `round` per
 // workgroup round of them, key_bytes of K and V per key, `resident` workgroups
-// on the device.
+// on the device, at most max_keys keys per split.
 SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
-                           size_t max_partials);
+                           size_t max_partials, int64_t max_keys = INT32_MAX);
 
 // Key splits of a prefill launch whose workgroups hold wg_rows rows (of G
 // heads) and take tile_us per 64-key tile, with at most max_partials bytes of

@@ -42,40 +42,6 @@ struct PrefillParams {
     int64_t n_rows; // B * Hq * Sq
 };
 
-// Splits row tile index rt of a split grid into row tile and split, and the
-// tile's n key tiles from t_begin on into the split's share of them.
-__device__ __forceinline__ void split_row_tile(const PrefillParams& p, int& rt, int& split) {
-    split = rt / p.n_row_tiles;
-    rt -= split * p.n_row_tiles;
-}
-__device__ __forceinline__ void split_key_tiles(int splits, int split, int& t_begin, int& n) {
-    const int per = (n + splits - 1) / splits;
-    const int first = min(split * per, n);
-    t_begin += first;
-    n = min(per, n - first);
-}
-
-// Partial of one wave's 32 rows q0 .. q0 + 31 (those < sq) of head h: O^T
-// accumulators for columns c0 .. c0 + 32 NDT - 1, unnormalised, relative to m
-// with row sum l.  A lane's 16 bytes of a row meet the rest of their cache
-// line in the L2 within the next three stores.
-template <int NDT>
-__device__ __forceinline__ void store_partial(const f16x (&oacc)[NDT], float m, float l, bool write_ml, float* part_o,
-                                              float* part_ml, int64_t row, int D, int c0, int g) {
-    float* const o = part_o + row * D + c0 + 4 * g;
-#pragma unroll
-    for (int dt = 0; dt < NDT; dt++) {
-#pragma unroll
-        for (int qq = 0; qq < 4; qq++) {
-            *reinterpret_cast<f4*>(o + 32 * dt + 8 * qq) = f4{oacc[dt][4 * qq], oacc[dt][4 * qq + 1],
-                                                             oacc[dt][4 * qq + 2], oacc[dt][4 * qq + 3]};
-        }
-    }
-    if (write_ml) {
-        *reinterpret_cast<float2*>(part_ml + row * 2) = float2{m, l};
-    }
-}
-
 // Head groups an XCD should work through at a time so that their K/V
 // (kv_bytes each) fit its L2; 0 when the grid cannot be dealt evenly.
 int xcd_head_group_chunk(int n_head_groups, int64_t kv_bytes);

@@ -1,5 +1,5 @@
-// Merges shared by the split-K kernels (device code): of a workgroup's waves,
-// and of the key splits.
+// Shared by the kernels that split the keys (device code): the split of a row
+// tile, its partials, and the merges of a workgroup's waves and of the splits.
 //
 // A split leaves, per query row, O unnormalised in fp32 and (m, l): its
 // reference maximum in log2 units and its row sum relative to it.  The merged
@@ -27,6 +27,42 @@ struct SplitRows {
         return o + b * o_sb + h * o_sh + (int64_t)q * o_ss;
     }
 };
+
+// Splits row tile index rt of a split grid into row tile and split, and the
+// tile's n key tiles from t_begin on into the split's share of them.
+__device__ __forceinline__ void split_row_tile(int n_row_tiles, int& rt, int& split) {
+    split = rt / n_row_tiles;
+    rt -= split * n_row_tiles;
+}
+__device__ __forceinline__ void split_key_tiles(int splits, int split, int& t_begin, int& n) {
+    const int per = (n + splits - 1) / splits;
+    const int first = min(split * per, n);
+    t_begin += first;
+    n = min(per, n - first);
+}
+
+// Partial of one query row per lane pair: O^T accumulators (lane: columns d0 ..
+// d0 + 3, d0 = 32 dt + 8 qq + 4 g, of columns c0 .. c0 + 32 NDT - 1),
+// unnormalised, relative to m with row sum l, times factors(d0).  A lane's 16
+// bytes of a row meet the rest of their cache line in the L2 within the next
+// three stores.
+template <int NDT, class Factors>
+__device__ __forceinline__ void store_partial(const f16x (&oacc)[NDT], float m, float l, bool write_ml, float* part_o,
+                                              float* part_ml, int64_t row, int D, int c0, int g, Factors&& factors) {
+    float* const o = part_o + row * D + c0;
+#pragma unroll
+    for (int dt = 0; dt < NDT; dt++) {
+#pragma unroll
+        for (int qq = 0; qq < 4; qq++) {
+            const int d0 = 32 * dt + 8 * qq + 4 * g;
+            *reinterpret_cast<f4*>(o + d0) =
+                factors(d0) * f4{oacc[dt][4 * qq], oacc[dt][4 * qq + 1], oacc[dt][4 * qq + 2], oacc[dt][4 * qq + 3]};
+        }
+    }
+    if (write_ml) {
+        *reinterpret_cast<float2*>(part_ml + row * 2) = float2{m, l};
+    }
+}
 
 // LDS of finish_rows: half of the waves' O (rows of D + 4 floats, conflict-free
 // 16-byte accesses) and every wave's (m, l).

@@ -438,11 +438,13 @@ DECODE_CASES = [(1, 8, 2, 1, sk, d, False, -1, sc) for d in (64, 128)
 
 @pytest.mark.parametrize("case", DECODE_CASES, ids=["b{}h{}kv{}q{}k{}d{}c{:d}w{}{}".format(*c) for c in DECODE_CASES])
 def test_int8_decode_vs_emulation(gpu, oracle_lib, case):
-    """INT8 bar against the kernel-exact emulation, whose running maximum goes
-    through the keys in order: a wave of the split-K kernel takes every eighth
-    block, so its P may be rounded to a finer step (never a coarser one), which
-    the bar for a rounding of 1/127 covers.  K and V are views into one cache
-    with a row stride of 2 Hkv D; a second call gives the same bits."""
+    """The kernel-exact emulation, with the running maximum over all keys in
+    order, whatever the splits: the INT8 bar on N(0, 1) rows, whose P a split's
+    own maximum would round otherwise, and, as the same P is summed in another
+    order only, 2e-3 of the largest output besides (fp16 output 4.9e-4; a P at
+    a tie rounds the other way in 1 of 10^5, by 1/127 of at most one V).  K and
+    V are views into one cache with a row stride of 2 Hkv D; a second call gives
+    the same bits."""
     import rdnattention as ra
 
     b, hq, hkv, sq, sk, d, causal, window, scales = case
@@ -481,4 +483,4 @@ def test_int8_decode_vs_emulation(gpu, oracle_lib, case):
         emu = emu * np.repeat(vch, hq // hkv, axis=1)[:, :, None, :]
     assert np.isfinite(got).all()
     mx, _, _ = errors(got, emu)
-    assert mx <= I8_MAX_ABS, f"max_abs {mx:.3e}"
+    assert mx <= min(I8_MAX_ABS, 2e-3 * np.abs(emu).max()), f"max_abs {mx:.3e} of {np.abs(emu).max():.3e}"
