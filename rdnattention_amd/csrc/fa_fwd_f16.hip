@@ -760,7 +760,8 @@ static int prefill_group(const AttnArgs& a) {
     return ratio % 4 == 0 ? 4 : (ratio % 2 == 0 ? 2 : 1);
 }
 
-int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, size_t max_partials) {
+int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double split_tile_us, int launches,
+                   size_t max_partials) {
     // Too few workgroups for the CUs and many key tiles for each: split the
     // keys, by the least modelled time.  A workgroup takes about 5 us beside
     // its key tiles; the partials are written and read at about 2.5 MB/us, and
@@ -792,8 +793,9 @@ int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, size_t max_pa
             break;
         }
         const double rounds = (double)((n_wg * s + 255) / 256);
-        const double t = rounds * (5.0 + (double)((tiles + s - 1) / s) * tile_us) +
-                         (s > 1 ? 5.0 + 2.0 * (double)partials / 2.5e6 : 0.0);
+        const double t = s == 1 ? 5.0 + (double)tiles * tile_us
+                                : rounds * (5.0 * launches + (double)((tiles + s - 1) / s) * split_tile_us) +
+                                      5.0 * launches + 2.0 * (double)partials / 2.5e6;
         if (s == 1 || t < best) {
             best = t;
             best_s = (int)s;
@@ -808,8 +810,8 @@ static int f16_prefill_splits(const AttnArgs& a, size_t max_partials) {
     if (a.D > 256) {
         return 1;
     }
-    return a.D > 128 ? prefill_splits(a, kKPairRows, 0.4 + 1.0 * a.D / 256, max_partials)
-                     : prefill_splits(a, 32 * kPPWaves, 0.4 + 1.0 * a.D / 128, max_partials);
+    const double tile_us = 0.4 + (a.D > 128 ? a.D / 256.0 : a.D / 128.0);
+    return prefill_splits(a, a.D > 128 ? kKPairRows : 32 * kPPWaves, tile_us, tile_us, 1, max_partials);
 }
 
 int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err, ScratchRegion* region) {

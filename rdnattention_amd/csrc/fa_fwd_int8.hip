@@ -55,6 +55,7 @@
 #include "fa_int8.hpp"
 #include "fa_internal.hpp"
 #include "fa_prefill.hpp"
+#include "fa_splitk.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -126,8 +127,12 @@ __device__ __forceinline__ i32x4_t uniform_rsrc(i32x4_t r) {
 
 // KSV: per-token K scales (p.ksv) staged per tile; otherwise p.k_scale is
 // folded into the per-row factor.
-template <int D, bool KSV, bool SCORES>
-__global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
+//
+// MODE: see Int8Mode.
+template <int D, bool KSV, bool SCORES, Int8Mode MODE>
+__device__ __forceinline__ void int8_body(Int8Params p) {
+    constexpr bool SPLIT = MODE != Int8Mode::kWhole;
+    constexpr bool ROWMAX = MODE == Int8Mode::kRowMax;
     using C = I8Cfg<D>;
     // [slot][K, V][TILE]; DMA destinations, so the base is 1 KB aligned
     __shared__ __attribute__((aligned(1024))) int8_t sKV[kI8Slots * 2 * C::TILE];
@@ -180,8 +185,11 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
     constexpr int DPT = 2 * C::BPW; // K/V DMAs per group-A wave per tile (wave 0 adds one for the K scales)
 
     auto run_tile = [&](const int wg) {
-        int hg, rt;
-        wg_tile(wg, p.n_head_groups, p.n_row_tiles, p.hg_chunk, hg, rt);
+        int hg, rt, split = 0;
+        wg_tile(wg, p.n_head_groups, SPLIT ? p.n_row_tiles * p.splits : p.n_row_tiles, p.hg_chunk, hg, rt);
+        if constexpr (SPLIT) {
+            split_row_tile(p.n_row_tiles, rt, split);
+        }
         const int per_b = p.Hkv * p.groups_per_kv;
         const int b = hg / per_b;
         const int rem = hg - b * per_b;
@@ -221,6 +229,9 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
             t_begin = klo / kI8BN;
             n = khi / kI8BN + 1 - t_begin;
         }
+        if constexpr (SPLIT) {
+            split_key_tiles(p.splits, split, t_begin, n);
+        }
         int row_lo, row_hi;
         row_key_bounds(p.mask, q, row_lo, row_hi);
 
@@ -251,6 +262,11 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
             of[dt] = f16x{};
         }
         float m_c = -INFINITY, m_a = -INFINITY, l_c = 0.0f, beta = 0.0f;
+        if constexpr (SPLIT && !ROWMAX) {
+            if (q < p.Sq) {
+                m_c = earlier_max(p, split, ((int64_t)b * p.Hq + h) * p.Sq + q);
+            }
+        }
         bool live = false, fold = false; // wave-uniform
         int run_tiles = 0;               // P V tiles summed in oint since its chain last restarted
         // S^T accumulators of the current tile (keys 0..31 and 32..63), turned
@@ -271,7 +287,7 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
             const i32x4_t rk = uniform_rsrc(make_rsrc_v(kbase + (int64_t)key0 * p.k_ss,
                                                         tile_bytes<kI8BN>(Sk - key0, (uint32_t)p.k_ss, D)));
             const i32x4_t rv = uniform_rsrc(make_rsrc_v(vbase + (int64_t)key0 * p.v_ss,
-                                                        tile_bytes<kI8BN>(Sk - key0, (uint32_t)p.v_ss, D)));
+                                                        ROWMAX ? 0u : tile_bytes<kI8BN>(Sk - key0, (uint32_t)p.v_ss, D)));
             const uint32_t mk = (uint32_t)__builtin_amdgcn_readfirstlane(
                 (int)(kv_lds + slot * (2 * C::TILE) + (uint32_t)((wave & 3) * C::BPW * 1024)));
 #pragma unroll
@@ -444,7 +460,7 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
             if (!wave_active) {
                 return;
             }
-            const bool do_pv = !SCORES && i >= 1 && cls_prev != 0;
+            const bool do_pv = !SCORES && !ROWMAX && i >= 1 && cls_prev != 0;
             int cls_now = 0;
             if (i < n) {
                 const int kt0 = (t_begin + i) * kI8BN;
@@ -514,6 +530,10 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
             }
             mx = pair_max(mx) * qeff; // qeff > 0: -inf stays -inf
             const float m_new = fmaxf(m_c, mx);
+            if constexpr (ROWMAX) {
+                m_c = m_new;
+                return;
+            }
             // a moved maximum folds O_int; so does a chain of kI8FoldTiles P V
             // tiles (rows whose maximum settled early, on long key ranges),
             // before the int32 sums could overflow
@@ -592,6 +612,12 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
         if (SCORES || !wave_active) {
             return;
         }
+        if constexpr (ROWMAX) {
+            if (g == 0 && q < p.Sq) {
+                p.row_max[split * p.n_rows + ((int64_t)b * p.Hq + h) * p.Sq + q] = m_c;
+            }
+            return;
+        }
         // O = (of * 2^(m_a - m_c) + oint) * v_scale / l (times the per-channel V
         // scales of this kv head when given), through this wave's sO slot
         const float bf = (m_c == -INFINITY) ? 0.0f : fast_exp2(m_a - m_c);
@@ -603,6 +629,17 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
             }
         }
         const float l = pair_sum(l_c);
+        if constexpr (SPLIT) {
+            const float* vch = p.vch != nullptr ? p.vch + ((int64_t)b * p.Hkv + kvh) * D : nullptr;
+            if (q < p.Sq) {
+                const int64_t row = split * p.n_rows + ((int64_t)b * p.Hq + h) * p.Sq + q;
+                store_partial(of, m_c, l, g == 0, p.part_o, p.part_ml, row, D, 0, g, [&](int d0) {
+                    return vch != nullptr ? p.v_scale * *reinterpret_cast<const f4*>(vch + d0)
+                                          : f4{p.v_scale, p.v_scale, p.v_scale, p.v_scale};
+                });
+            }
+            return;
+        }
         const float f = l > 0.0f ? p.v_scale / l : 0.0f;
         const float* vch = p.vch != nullptr ? p.vch + ((int64_t)b * p.Hkv + kvh) * D : nullptr;
         store_o_tile<D, C::LDO>(
@@ -622,17 +659,34 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
 }
 
 template <int D, bool KSV, bool SCORES>
-int launch_int8(const Int8Params& p, int64_t n_wg, hipStream_t stream, std::string& err) {
+__global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8(Int8Params p) {
+    int8_body<D, KSV, SCORES, Int8Mode::kWhole>(p);
+}
+
+template <int D, bool KSV, Int8Mode MODE>
+__global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_split(Int8Params p) {
+    int8_body<D, KSV, false, MODE>(p);
+}
+
+template <int D, bool KSV, bool SCORES>
+int launch_int8(const Int8Params& p, Int8Mode mode, int64_t n_wg, hipStream_t stream, std::string& err) {
     // persistent: as many workgroups as the device holds at once, each
     // walking its share of the n_wg row tiles
-    const int64_t resident =
-        resident_workgroups(reinterpret_cast<const void*>(&fa_fwd_int8<D, KSV, SCORES>), kI8Threads, err);
+    void (*kernel)(Int8Params) = &fa_fwd_int8<D, KSV, SCORES>;
+    if constexpr (!SCORES) {
+        if (mode == Int8Mode::kRowMax) {
+            kernel = &fa_fwd_int8_split<D, KSV, Int8Mode::kRowMax>;
+        } else if (mode == Int8Mode::kSplit) {
+            kernel = &fa_fwd_int8_split<D, KSV, Int8Mode::kSplit>;
+        }
+    }
+    const int64_t resident = resident_workgroups(reinterpret_cast<const void*>(kernel), kI8Threads, err);
     if (resident <= 0) {
         return -1;
     }
     const int64_t grid = std::min(n_wg, resident);
     KernelTimerGuard timer(stream);
-    hipLaunchKernelGGL((fa_fwd_int8<D, KSV, SCORES>), dim3((uint32_t)grid), dim3(kI8Threads), 0, stream, p);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(kI8Threads), 0, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         err = hipGetErrorString(e);
@@ -695,7 +749,7 @@ int64_t int8_params(const AttnArgs& a, Int8Params& p, std::string& err) {
 
 int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
     Int8Params p;
-    const int64_t n_wg = int8_params(a, p, err);
+    int64_t n_wg = int8_params(a, p, err);
     if (n_wg < 0) {
         return -1;
     }
@@ -705,15 +759,45 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
     if ((a.D == 64 || a.D == 128) && int8_splitk_supported(a)) {
         return fwd_int8_splitk(a, p, stream, err);
     }
-    if (a.D == 64 && p.vtok == nullptr) {
-        return p.ksv != nullptr ? launch_int8<64, true, false>(p, n_wg, stream, err)
-                                : launch_int8<64, false, false>(p, n_wg, stream, err);
+    if (a.D != 64 && a.D != 128) {
+        err = "unsupported head_dim (only 64 and 128 are compiled in for the int8 kernel)";
+        return -1;
     }
-    if (a.D == 64 || a.D == 128) {
-        return launch_int8_f16pv(p, a.D, false, n_wg, stream, err);
+    // too few workgroups for the CUs: split the keys (a 64-key tile takes
+    // about 1.5 us at D = 64, 1.9 us at D = 128, and half as much again in the
+    // launch that finds the row maxima).  Measured, us a call: B1 Hq32 Hkv8
+    // Sq256 Sk8192 D128 242 unsplit, 86 split; B2 Hq16 Hkv8 Sq100 Sk16000 D64
+    // 382 and 69
+    p.splits = prefill_splits(a, 32 * kI8Waves, a.D == 64 ? 1.5 : 1.9, a.D == 64 ? 2.2 : 2.8, 2, SIZE_MAX);
+    n_wg *= p.splits;
+    p.n_items = (int32_t)n_wg;
+    SplitRows out{};
+    StreamScratch ws(ScratchUse::SplitKPartials);
+    if (splitk_begin(a, p.splits, ws, stream, out, err) != 0) {
+        return -1;
     }
-    err = "unsupported head_dim (only 64 and 128 are compiled in for the int8 kernel)";
-    return -1;
+    p.part_o = out.part_o;
+    p.part_ml = out.part_ml;
+    p.n_rows = out.n_rows;
+    auto launch = [&](Int8Mode mode) {
+        if (a.D == 64 && p.vtok == nullptr) {
+            return p.ksv != nullptr ? launch_int8<64, true, false>(p, mode, n_wg, stream, err)
+                                    : launch_int8<64, false, false>(p, mode, n_wg, stream, err);
+        }
+        return launch_int8_f16pv(p, a.D, false, mode, n_wg, stream, err);
+    };
+    if (p.splits == 1) {
+        return launch(Int8Mode::kWhole);
+    }
+    StreamScratch maxima(ScratchUse::Int8Scores);
+    if (maxima.alloc((size_t)p.splits * p.n_rows * sizeof(float), stream, err) != 0) {
+        return -1;
+    }
+    p.row_max = static_cast<float*>(maxima.ptr);
+    if (launch(Int8Mode::kRowMax) != 0 || launch(Int8Mode::kSplit) != 0) {
+        return -1;
+    }
+    return splitk_finish(a, out, stream, err);
 }
 
 int int8_scores(const AttnArgs& in, int32_t* scores, hipStream_t stream, std::string& err) {
@@ -735,8 +819,8 @@ int int8_scores(const AttnArgs& in, int32_t* scores, hipStream_t stream, std::st
     }
     p.scores = scores;
     switch (a.D) {
-    case 64: return launch_int8<64, false, true>(p, n_wg, stream, err);
-    case 128: return launch_int8_f16pv(p, 128, true, n_wg, stream, err);
+    case 64: return launch_int8<64, false, true>(p, Int8Mode::kWhole, n_wg, stream, err);
+    case 128: return launch_int8_f16pv(p, 128, true, Int8Mode::kWhole, n_wg, stream, err);
     default: break;
     }
     err = "unsupported head_dim (only 64 and 128 are compiled in for the int8 kernel)";

@@ -67,6 +67,7 @@
 #include "fa_internal.hpp"
 #include "fa_int8.hpp"
 #include "fa_prefill.hpp"
+#include "fa_splitk.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -167,8 +168,12 @@ __device__ __forceinline__ void i8x16_to_h8x2_scaled(i4 w, float vs, h8& lo, h8&
 //
 // SCORES: the S^T accumulators of every computed key tile are written to
 // p.scores and nothing else is computed (test instantiation).
-template <int D, bool VTOK, bool SCORES>
-__global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p) {
+//
+// MODE: see Int8Mode.
+template <int D, bool VTOK, bool SCORES, Int8Mode MODE>
+__device__ __forceinline__ void int8_f16pv_body(Int8Params p) {
+    constexpr bool SPLIT = MODE != Int8Mode::kWhole;
+    constexpr bool ROWMAX = MODE == Int8Mode::kRowMax;
     using C = I8Cfg<D>;
     __shared__ __attribute__((aligned(16))) int8_t sKs[2 * C::TILE_K];
     __shared__ __attribute__((aligned(16))) _Float16 sVs[2 * C::TILE_V];
@@ -190,8 +195,11 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p)
     // last LDS read of K/V, so the next tile's prologue may overwrite them;
     // each wave's sO slot is its own.
     auto run_tile = [&](const int wg) {
-        int hg, rt;
-        wg_tile(wg, p.n_head_groups, p.n_row_tiles, p.hg_chunk, hg, rt);
+        int hg, rt, split = 0;
+        wg_tile(wg, p.n_head_groups, SPLIT ? p.n_row_tiles * p.splits : p.n_row_tiles, p.hg_chunk, hg, rt);
+        if constexpr (SPLIT) {
+            split_row_tile(p.n_row_tiles, rt, split);
+        }
         const int per_b = p.Hkv * p.groups_per_kv;
         const int b = hg / per_b;
         const int rem = hg - b * per_b;
@@ -241,6 +249,9 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p)
             t_begin = klo / kI8BN;
             n = khi / kI8BN + 1 - t_begin;
         }
+        if constexpr (SPLIT) {
+            split_key_tiles(p.splits, split, t_begin, n);
+        }
         int row_lo, row_hi;
         row_key_bounds(p.mask, q, row_lo, row_hi);
         // class of key tile t_begin + i for this wave's rows (0 skip, 1 no mask, 2 masked)
@@ -254,6 +265,11 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p)
         // m_run: the scheme's exact running max; m_ref: the lagging reference
         // O and l are kept relative to (m_ref <= m_run)
         float m_run = -INFINITY, m_ref = -INFINITY, l_run = 0.0f;
+        if constexpr (SPLIT && !ROWMAX) {
+            if (q < p.Sq) {
+                m_run = earlier_max(p, split, ((int64_t)b * p.Hq + h) * p.Sq + q);
+            }
+        }
         const i16x bias16 = SCORES ? i16x{} : (i16x{} + __float_as_int(kI8Bias));
         f16x tsc[2]; // scores of the current tile, dequantised by ks (t = S * ks)
         tsc[0] = f16x{};
@@ -287,7 +303,7 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p)
             const auto rk = make_rsrc(kbase + (int64_t)tk * kI8BN * p.k_ss,
                                       x < n ? tile_bytes<kI8BN>(Sk - tk * kI8BN, (uint32_t)p.k_ss, D) : 0u);
             const auto rv = make_rsrc(vbase + (int64_t)tv * kI8BN * p.v_ss,
-                                      (x >= 1 && x <= n) ? tile_bytes<kI8BN>(Sk - tv * kI8BN, (uint32_t)p.v_ss, D) : 0u);
+                                      (!ROWMAX && x >= 1 && x <= n) ? tile_bytes<kI8BN>(Sk - tv * kI8BN, (uint32_t)p.v_ss, D) : 0u);
 #pragma unroll
             for (int it = 0; it < C::CT; it++) {
                 kreg[it] = buffer_load_i4(rk, coff_k[it]);
@@ -311,7 +327,7 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p)
                     if (x < n) {
                         *reinterpret_cast<i4*>(&sK[clk[it]]) = kreg[it];
                     }
-                    if (x >= 1 && x <= n) {
+                    if (!ROWMAX && x >= 1 && x <= n) {
                         h8 lo, hi;
                         if constexpr (VTOK) {
                             i8x16_to_h8x2_scaled(vreg[it], vsreg[it], lo, hi);
@@ -452,7 +468,7 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p)
             if (!wave_active) {
                 return;
             }
-            const bool do_pv = !SCORES && i >= 1 && cls_prev != 0;
+            const bool do_pv = !SCORES && !ROWMAX && i >= 1 && cls_prev != 0;
             const int cls_now = i < n ? tile_class(tcls, t_begin + i) : 0;
             using T_ = std::true_type;
             using F_ = std::false_type;
@@ -507,6 +523,9 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p)
             }
             mx = pair_max(mx) * qeff; // qeff > 0: -inf stays -inf
             m_run = fmaxf(m_run, mx);
+            if constexpr (ROWMAX) {
+                return;
+            }
             const bool move = m_run > m_ref + kI8RefThreshold; // false while m_run = -inf
             if (wave_any(move)) {
                 const float alpha = move ? fast_exp2(m_ref - m_run) : 1.0f; // m_ref = -inf -> 0
@@ -583,9 +602,26 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p)
         if (SCORES || !wave_active) {
             return;
         }
+        if constexpr (ROWMAX) {
+            if (g == 0 && q < p.Sq) {
+                p.row_max[split * p.n_rows + ((int64_t)b * p.Hq + h) * p.Sq + q] = m_run;
+            }
+            return;
+        }
         // O = O^T * v_scale / l (times the per-channel V scales of this kv head
         // when given), through this wave's sO slot
         const float l = pair_sum(l_run);
+        if constexpr (SPLIT) {
+            const float* vch = p.vch != nullptr ? p.vch + ((int64_t)b * p.Hkv + kvh) * D : nullptr;
+            if (q < p.Sq) {
+                const int64_t row = split * p.n_rows + ((int64_t)b * p.Hq + h) * p.Sq + q;
+                const float f = p.v_scale / kI8PScale;
+                store_partial(oacc, m_ref, l, g == 0, p.part_o, p.part_ml, row, D, 0, g, [&](int d0) {
+                    return vch != nullptr ? f * *reinterpret_cast<const f4*>(vch + d0) : f4{f, f, f, f};
+                });
+            }
+            return;
+        }
         const float f = l > 0.0f ? p.v_scale / (l * kI8PScale) : 0.0f;
         const float* vch = p.vch != nullptr ? p.vch + ((int64_t)b * p.Hkv + kvh) * D : nullptr;
         store_o_tile<D, C::LDO>(
@@ -605,17 +641,34 @@ __global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p)
 }
 
 template <int D, bool VTOK, bool SCORES>
-int launch_f16pv(const Int8Params& p, int64_t n_wg, hipStream_t stream, std::string& err) {
+__global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv(Int8Params p) {
+    int8_f16pv_body<D, VTOK, SCORES, Int8Mode::kWhole>(p);
+}
+
+template <int D, bool VTOK, Int8Mode MODE>
+__global__ __launch_bounds__(kI8Threads, 1) void fa_fwd_int8_f16pv_split(Int8Params p) {
+    int8_f16pv_body<D, VTOK, false, MODE>(p);
+}
+
+template <int D, bool VTOK, bool SCORES>
+int launch_f16pv(const Int8Params& p, Int8Mode mode, int64_t n_wg, hipStream_t stream, std::string& err) {
     // persistent: as many workgroups as the device holds at once, each
     // walking its share of the n_wg row tiles
-    const int64_t resident =
-        resident_workgroups(reinterpret_cast<const void*>(&fa_fwd_int8_f16pv<D, VTOK, SCORES>), kI8Threads, err);
+    void (*kernel)(Int8Params) = &fa_fwd_int8_f16pv<D, VTOK, SCORES>;
+    if constexpr (!SCORES) {
+        if (mode == Int8Mode::kRowMax) {
+            kernel = &fa_fwd_int8_f16pv_split<D, VTOK, Int8Mode::kRowMax>;
+        } else if (mode == Int8Mode::kSplit) {
+            kernel = &fa_fwd_int8_f16pv_split<D, VTOK, Int8Mode::kSplit>;
+        }
+    }
+    const int64_t resident = resident_workgroups(reinterpret_cast<const void*>(kernel), kI8Threads, err);
     if (resident <= 0) {
         return -1;
     }
     const int64_t grid = std::min(n_wg, resident);
     KernelTimerGuard timer(stream);
-    hipLaunchKernelGGL((fa_fwd_int8_f16pv<D, VTOK, SCORES>), dim3((uint32_t)grid), dim3(kI8Threads), 0, stream, p);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(kI8Threads), 0, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         err = hipGetErrorString(e);
@@ -626,21 +679,21 @@ int launch_f16pv(const Int8Params& p, int64_t n_wg, hipStream_t stream, std::str
 
 } // namespace
 
-int launch_int8_f16pv(const Int8Params& p, int head_dim, bool scores, int64_t n_wg, hipStream_t stream,
-                      std::string& err) {
+int launch_int8_f16pv(const Int8Params& p, int head_dim, bool scores, Int8Mode mode, int64_t n_wg,
+                      hipStream_t stream, std::string& err) {
     const bool vtok = p.vtok != nullptr;
     switch (head_dim) {
     case 64:
         if (vtok && !scores) {
-            return launch_f16pv<64, true, false>(p, n_wg, stream, err);
+            return launch_f16pv<64, true, false>(p, mode, n_wg, stream, err);
         }
         break;
     case 128:
         if (scores) {
-            return launch_f16pv<128, false, true>(p, n_wg, stream, err);
+            return launch_f16pv<128, false, true>(p, mode, n_wg, stream, err);
         }
-        return vtok ? launch_f16pv<128, true, false>(p, n_wg, stream, err)
-                    : launch_f16pv<128, false, false>(p, n_wg, stream, err);
+        return vtok ? launch_f16pv<128, true, false>(p, mode, n_wg, stream, err)
+                    : launch_f16pv<128, false, false>(p, mode, n_wg, stream, err);
     default: break;
     }
     err = "unsupported head_dim for the fp16 P V int8 kernel";

@@ -54,9 +54,32 @@ struct Int8Params {
     int64_t o_sb, o_sh, o_ss;
     int32_t Hq, Sq, Hkv, ratio, G, rows_per_wg, n_row_tiles, n_head_groups, groups_per_kv;
     int32_t hg_chunk; // head groups per XCD at a time (0 = head groups fastest)
-    int32_t n_items;  // n_row_tiles * n_head_groups
+    int32_t n_items;  // n_row_tiles * n_head_groups (* splits)
     MaskSpec mask;
+    // key splits of every row tile (see PrefillParams and Int8Mode)
+    int32_t splits;
+    float* part_o;
+    float* part_ml;
+    float* row_max; // [splits][n_rows] largest score of each row in each split, log2 units
+    int64_t n_rows;
 };
+
+// What a prefill kernel instantiation computes.  kWhole: the output of whole
+// rows.  The scheme quantises P against the running maximum over all earlier
+// keys, so the keys of a row tile are split in two launches: kRowMax finds
+// every row's largest score in each split (no softmax, no P V), and kSplit
+// starts each split's running maximum at the largest of the earlier ones and
+// writes partials for the combine kernel.
+enum class Int8Mode { kWhole, kRowMax, kSplit };
+
+// The running maximum that split `split` of a row starts from.
+__device__ __forceinline__ float earlier_max(const Int8Params& p, int split, int64_t row) {
+    float m = -INFINITY;
+    for (int s = 0; s < split; s++) {
+        m = fmaxf(m, p.row_max[s * p.n_rows + row]);
+    }
+    return m;
+}
 
 // Kernel parameters and grid size of an INT8 launch.  Returns the number of
 // row tiles (workgroups of a one-tile-per-workgroup grid), or -1 with `err`.
@@ -65,8 +88,8 @@ int64_t int8_params(const AttnArgs& a, Int8Params& p, std::string& err);
 // The kernel with P V on fp16 MFMA (fa_fwd_int8_f16pv.hip): head_dim 128
 // (forward and, with `scores`, the score export) and the per-token V scale at
 // head_dim 64 or 128.
-int launch_int8_f16pv(const Int8Params& p, int head_dim, bool scores, int64_t n_wg, hipStream_t stream,
-                      std::string& err);
+int launch_int8_f16pv(const Int8Params& p, int head_dim, bool scores, Int8Mode mode, int64_t n_wg,
+                      hipStream_t stream, std::string& err);
 
 // Split-K decode (fa_fwd_int8_decode.hip): (Hq / Hkv) * Sq <= 32, head_dim 64
 // or 128.

@@ -123,10 +123,12 @@ int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::s
 SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
                            size_t max_partials, int64_t max_keys = INT32_MAX);
 
-// Key splits of a prefill launch whose workgroups hold wg_rows rows (of G
-// heads) and take tile_us per 64-key tile, with at most max_partials bytes of
-// partials; 1 where splitting does not pay.
-int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, size_t max_partials);
+// Key splits of a prefill call whose workgroups hold wg_rows rows (of G heads)
+// and take tile_us per 64-key tile (split_tile_us over `launches` launches where
+// the keys are split), with at most max_partials bytes of partials; 1 where
+// splitting does not pay.
+int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double split_tile_us, int launches,
+                   size_t max_partials);
 
 // Before and after a launch of `splits` key splits: `r` from the arguments, with
 // the partials taken from `ws`; and the combine launch.  0, or -1 with `err`.

@@ -436,8 +436,19 @@ DECODE_CASES = [(1, 8, 2, 1, sk, d, False, -1, sc) for d in (64, 128)
 ]
 
 
-@pytest.mark.parametrize("case", DECODE_CASES, ids=["b{}h{}kv{}q{}k{}d{}c{:d}w{}{}".format(*c) for c in DECODE_CASES])
-def test_int8_decode_vs_emulation(gpu, oracle_lib, case):
+# more rows than one column block, too few workgroups for the CUs: the keys of
+# the prefill kernels are split
+SPLIT_CASES = [(1, 8, 2, 70, 3000, d, True, -1, sc) for d in (64, 128)
+               for sc in ("tensor", "token", "channel", "vtoken")] + [
+    (1, 4, 4, 257, 2049, 128, False, -1, "token"),
+    (1, 4, 2, 300, 2500, 64, True, 900, "token"),
+    (1, 4, 1, 1500, 1100, 128, True, -1, "channel"),  # rows without keys
+]
+
+
+@pytest.mark.parametrize("case", DECODE_CASES + SPLIT_CASES,
+                         ids=["b{}h{}kv{}q{}k{}d{}c{:d}w{}{}".format(*c) for c in DECODE_CASES + SPLIT_CASES])
+def test_int8_split_keys_vs_emulation(gpu, oracle_lib, case):
     """The kernel-exact emulation, with the running maximum over all keys in
     order, whatever the splits: the INT8 bar on N(0, 1) rows, whose P a split's
     own maximum would round otherwise, and, as the same P is summed in another
