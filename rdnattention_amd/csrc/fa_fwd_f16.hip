@@ -114,11 +114,26 @@ struct PPCfg {
 // multiply-add.  The accumulators are shifted only when the running max
 // moves.  Without PRE, Q carries only the sign and p = 2^(acc c - m).
 //
-// SPLIT: every row tile's key tiles are dealt to p.splits workgroups, which
-// write partials for the combine kernel.
-template <int D, bool PRE, bool SPLIT>
+// MODE: kWhole as described; kSplit, every row tile's key tiles are dealt to
+// p.splits workgroups, which write partials for the combine kernel; kAlternate,
+// for launches whose few row tiles are long serial chains: both groups hold
+// the same 128 rows and take the key tiles in turn, group A tiles 0, 2, 4, ...
+// and group B tiles 1, 3, 5, ..., each staging its own tiles into one K and one
+// V slot (pair (K(i+1), V(i)) of its sequence at the start of its V(i), when
+// its M(i) has read their predecessors), and group B's O is merged into group
+// A's through LDS at the end.  A row tile then takes half as many steps.
+enum class PPMode { kWhole, kSplit, kAlternate };
+
+template <int D, bool PRE, PPMode MODE>
 __device__ __forceinline__ void pp_body(PrefillParams p) {
     using C = PPCfg<D>;
+    constexpr bool SPLIT = MODE == PPMode::kSplit;
+    constexpr bool ALT = MODE == PPMode::kAlternate;
+    constexpr int ROW_WAVES = ALT ? kPPWaves / 2 : kPPWaves; // waves with rows of their own
+    // K (and V) chunks that one group stages, and per thread of it
+    constexpr int TASK = ALT ? 2 * C::HALF_TASK : C::HALF_TASK;
+    constexpr int CT = (TASK + 255) / 256;
+    constexpr int QCT = ROW_WAVES * 32 * C::KCH / kPPThreads; // Q chunks per thread
     // sK[slot], sV[slot], sQ
     __shared__ __attribute__((aligned(16))) _Float16 smem[2 * C::TILE_K + 2 * C::TILE_V + C::TILE_Q];
     _Float16* const sKs = smem;
@@ -132,15 +147,17 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
     const int g = lane >> 5;
     const int grp = wave >> 2;       // 0 = group A, 1 = group B
     const int gtid = tid & 255;      // thread index inside the group
+    const int rw = ALT ? wave & 3 : wave; // wave by its rows
+    const int ugrp = ALT ? __builtin_amdgcn_readfirstlane(grp) : 0;
 
     // ---- staging: this group's half (rows 32*grp .. +31) of K(x) and V(x-1)
-    uint32_t coff_k[C::CT], coff_v[C::CT];
-    int clk[C::CT], clv[C::CT]; // LDS element offsets inside a tile, -1 = no chunk
+    uint32_t coff_k[CT], coff_v[CT];
+    int clk[CT], clv[CT]; // LDS element offsets inside a tile, -1 = no chunk
 #pragma unroll
-    for (int it = 0; it < C::CT; it++) {
+    for (int it = 0; it < CT; it++) {
         const int e = gtid + it * 256;
-        const bool ok = C::HALF_TASK % 256 == 0 || e < C::HALF_TASK;
-        const int row = 32 * grp + (ok ? e / C::KCH : 0);
+        const bool ok = TASK % 256 == 0 || e < TASK;
+        const int row = (ALT ? 0 : 32 * grp) + (ok ? e / C::KCH : 0);
         const int ch = ok ? e - (e / C::KCH) * C::KCH : 0;
         coff_k[it] = (uint32_t)(((int64_t)row * p.k_ss + 8 * ch) * 2);
         coff_v[it] = (uint32_t)(((int64_t)row * p.v_ss + 8 * ch) * 2);
@@ -174,9 +191,9 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
         const int rem = hg - b * per_b;
         const int kvh = rem / p.groups_per_kv;
         const int sub = rem - kvh * p.groups_per_kv;
-        const int h = kvh * p.ratio + sub * p.G + (wave % p.G);
+        const int h = kvh * p.ratio + sub * p.G + (rw % p.G);
         const int wg_q0 = rt * p.rows_per_wg;
-        const int q0 = wg_q0 + (wave / p.G) * 32;
+        const int q0 = wg_q0 + (rw / p.G) * 32;
         const int q = q0 + l32;
         const bool wave_active = q0 < p.Sq;
         const int q_hi = min(q0 + 31, p.Sq - 1);
@@ -203,7 +220,7 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
             // (a division by rows_per_wg cost ~30 instructions per chunk).
             // Recomputed from an opaque copy of the thread id at each use so
             // that no index stays live across the loads' latency.
-            const uint32_t rsh = 8u - (uint32_t)(p.G >> 1); // log2 rows_per_wg
+            const uint32_t rsh = (ALT ? 7u : 8u) - (uint32_t)(p.G >> 1); // log2 rows_per_wg
             struct Chunk {
                 uint32_t j, r, ch;
             };
@@ -213,8 +230,8 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
                 return Chunk{rj >> rsh, rj & ((1u << rsh) - 1u), idx - rj * C::KCH};
             };
             auto src_row = [&](const Chunk& k) { return wg_q0 + (int)k.r < p.Sq ? (uint32_t)wg_q0 + k.r : 0u; };
-            h8 x[C::QCT];
-            f4 cs[C::QCT], sn[C::QCT];
+            h8 x[QCT];
+            f4 cs[QCT], sn[QCT];
             uint32_t t = tid;
             asm volatile("" : "+v"(t));
             // The table loads are issued first, so that they and the Q loads
@@ -223,7 +240,7 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
             // plain scaling start with were hoisted above the branch).
             if (p.rope_q) {
 #pragma unroll
-                for (int c = 0; c < C::QCT; c++) {
+                for (int c = 0; c < QCT; c++) {
                     const Chunk k = chunk(t, c);
                     const uint64_t off = (uint64_t)src_row(k) * (D / 2) + 4 * k.ch;
                     cs[c] = *reinterpret_cast<const f4*>(p.rot_cos + off);
@@ -231,33 +248,33 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
                 }
             }
 #pragma unroll
-            for (int c = 0; c < C::QCT; c++) {
+            for (int c = 0; c < QCT; c++) {
                 const Chunk k = chunk(t, c);
                 x[c] = *reinterpret_cast<const h8*>(qb + (int64_t)k.j * p.q_sh + (int64_t)src_row(k) * p.q_ss +
                                                     8 * k.ch);
             }
             if (p.rope_q) {
 #pragma unroll
-                for (int c = 0; c < C::QCT; c++) {
+                for (int c = 0; c < QCT; c++) {
                     x[c] = PRE ? rope8_cs_mul(x[c], cs[c], sn[c], p.qmul) : rope8_cs(x[c], cs[c], sn[c]);
                 }
             } else if constexpr (PRE) {
 #pragma unroll
-                for (int c = 0; c < C::QCT; c++) {
+                for (int c = 0; c < QCT; c++) {
                     x[c] = scale8(x[c], p.qmul);
                 }
             }
             const bool neg = !PRE && p.q_sign < 0.0f; // PRE: the sign is in qmul
             asm volatile("" : "+v"(t));
 #pragma unroll
-            for (int c = 0; c < C::QCT; c++) {
+            for (int c = 0; c < QCT; c++) {
                 const Chunk k = chunk(t, c);
                 const uint32_t dst = ((k.j + p.G * (k.r >> 5)) * 32 + (k.r & 31)) * C::LDQ + 8 * k.ch;
                 *reinterpret_cast<h8*>(&sQ[dst]) = wg_q0 + (int)k.r < p.Sq ? (neg ? -x[c] : x[c]) : h8{};
             }
         };
         auto read_q = [&]() {
-            const _Float16* src = sQ + (wave * 32 + l32) * C::LDQ + 8 * g;
+            const _Float16* src = sQ + (rw * 32 + l32) * C::LDQ + 8 * g;
 #pragma unroll
             for (int st = 0; st < C::NS; st++) {
                 qreg[st] = *reinterpret_cast<const h8*>(src + 16 * st);
@@ -275,6 +292,9 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
         if constexpr (SPLIT) {
             split_key_tiles(p.splits, split, t_begin, n);
         }
+        // key tile i of this wave's sequence of ng tiles
+        const int ng = ALT ? (n + 1 - ugrp) / 2 : n;
+        auto tile_at = [&](int i) { return ALT ? t_begin + 2 * i + ugrp : t_begin + i; };
         const int Sk = p.mask.sk;
         const uint32_t k_row_b = (uint32_t)(p.k_ss * 2), v_row_b = (uint32_t)(p.v_ss * 2);
         int row_lo, row_hi;
@@ -301,7 +321,7 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
         }
         int cls_prev = 0; // classification of the tile whose P is held in pb
 
-        h8 kreg[C::CT], vreg[C::CT];
+        h8 kreg[CT], vreg[CT];
         // registers <- HBM for pair x (K tile x if x < n, V tile x-1 if 1 <= x <= n);
         // a missing tile gets num_records 0, so its loads return 0 and touch nothing.
         // A tile spans at most kBN rows at a seq stride <= 2^24 elements, so its
@@ -310,19 +330,20 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
         // Each group calls load_pair with x = 0, 1, 2, ... in order, so the tile
         // addresses advance by one tile stride per call (unsigned arithmetic:
         // V tile -1 of the first call is never read, its num_records is 0).
-        uint64_t k_addr = reinterpret_cast<uint64_t>(kbase) + (uint64_t)((int64_t)t_begin * kBN * p.k_ss * 2);
-        uint64_t v_addr = reinterpret_cast<uint64_t>(vbase) + (uint64_t)((int64_t)(t_begin - 1) * kBN * p.v_ss * 2);
-        const uint64_t k_step = (uint64_t)(kBN * p.k_ss * 2), v_step = (uint64_t)(kBN * p.v_ss * 2);
+        uint64_t k_addr = reinterpret_cast<uint64_t>(kbase) + (uint64_t)((int64_t)tile_at(0) * kBN * p.k_ss * 2);
+        uint64_t v_addr = reinterpret_cast<uint64_t>(vbase) + (uint64_t)((int64_t)tile_at(-1) * kBN * p.v_ss * 2);
+        constexpr int STEP = ALT ? 2 * kBN : kBN;
+        const uint64_t k_step = (uint64_t)(STEP * p.k_ss * 2), v_step = (uint64_t)(STEP * p.v_ss * 2);
         auto load_pair = [&](int x) {
-            const int tk = t_begin + x, tv = t_begin + x - 1;
+            const int tk = tile_at(x), tv = ALT ? tile_at(x - 1) : t_begin + x - 1;
             const auto rk = make_rsrc(reinterpret_cast<const void*>(k_addr),
-                                      x < n ? tile_bytes<kBN>(Sk - tk * kBN, k_row_b, D * 2) : 0u);
+                                      x < ng ? tile_bytes<kBN>(Sk - tk * kBN, k_row_b, D * 2) : 0u);
             const auto rv = make_rsrc(reinterpret_cast<const void*>(v_addr),
-                                      (x >= 1 && x <= n) ? tile_bytes<kBN>(Sk - tv * kBN, v_row_b, D * 2) : 0u);
+                                      (x >= 1 && x <= ng) ? tile_bytes<kBN>(Sk - tv * kBN, v_row_b, D * 2) : 0u);
             k_addr += k_step;
             v_addr += v_step;
 #pragma unroll
-            for (int it = 0; it < C::CT; it++) {
+            for (int it = 0; it < CT; it++) {
                 kreg[it] = buffer_load_h8(rk, coff_k[it], 0);
                 vreg[it] = buffer_load_h8(rv, coff_v[it], 0);
             }
@@ -333,11 +354,11 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
         // written on the same schedule as for an existing tile, after the last
         // read of its previous contents.  No branches in the VALU phase.
         auto store_pair = [&](int x) {
-            _Float16* sK = sKs + (x & 1) * C::TILE_K;
-            _Float16* sV = sVs + ((x - 1) & 1) * C::TILE_V;
+            _Float16* sK = sKs + (ALT ? ugrp : x & 1) * C::TILE_K;
+            _Float16* sV = sVs + (ALT ? ugrp : (x - 1) & 1) * C::TILE_V;
 #pragma unroll
-            for (int it = 0; it < C::CT; it++) {
-                if (C::HALF_TASK % 256 == 0 || clk[it] >= 0) {
+            for (int it = 0; it < CT; it++) {
+                if (TASK % 256 == 0 || clk[it] >= 0) {
                     *reinterpret_cast<h8*>(&sK[clk[it]]) = kreg[it];
                     *reinterpret_cast<h8*>(&sV[clv[it]]) = vreg[it];
                 }
@@ -360,16 +381,16 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
             return r;
         };
         auto dma_pair = [&](int x) {
-            const int tk = t_begin + x, tv = t_begin + x - 1;
+            const int tk = tile_at(x), tv = ALT ? tile_at(x - 1) : t_begin + x - 1;
             DmaPair d;
             d.rk = uniform(make_rsrc_v(reinterpret_cast<const void*>(k_addr),
-                                       x < n ? tile_bytes<kBN>(Sk - tk * kBN, k_row_b, D * 2) : 0u));
+                                       x < ng ? tile_bytes<kBN>(Sk - tk * kBN, k_row_b, D * 2) : 0u));
             d.rv = uniform(make_rsrc_v(reinterpret_cast<const void*>(v_addr),
-                                       (x >= 1 && x <= n) ? tile_bytes<kBN>(Sk - tv * kBN, v_row_b, D * 2) : 0u));
+                                       (x >= 1 && x <= ng) ? tile_bytes<kBN>(Sk - tv * kBN, v_row_b, D * 2) : 0u));
             d.mk = (uint32_t)__builtin_amdgcn_readfirstlane(
-                (int)(lds_k + (uint32_t)(((x & 1) * C::TILE_K + (int)dma_j0 * C::PSK) * 2)));
+                (int)(lds_k + (uint32_t)(((ALT ? ugrp : x & 1) * C::TILE_K + (int)dma_j0 * C::PSK) * 2)));
             d.mv = (uint32_t)__builtin_amdgcn_readfirstlane(
-                (int)(lds_v + (uint32_t)((((x - 1) & 1) * C::TILE_V + (int)dma_j0 * C::PSV) * 2)));
+                (int)(lds_v + (uint32_t)(((ALT ? ugrp : (x - 1) & 1) * C::TILE_V + (int)dma_j0 * C::PSV) * 2)));
             k_addr += k_step;
             v_addr += v_step;
             return d;
@@ -403,9 +424,9 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
             constexpr int T = NPV + NSK;
             constexpr int DEPTH = T < kOpDepth ? T : kOpDepth;
             const int j16 = lane & 15;
-            const _Float16* vrow = sVs + ((i - 1) & 1) * C::TILE_V + (4 * g + (j16 >> 2)) * C::LDV +
+            const _Float16* vrow = sVs + (ALT ? ugrp : (i - 1) & 1) * C::TILE_V + (4 * g + (j16 >> 2)) * C::LDV +
                                    16 * ((lane >> 4) & 1) + 4 * (j16 & 3);
-            const _Float16* krow = sKs + (i & 1) * C::TILE_K + l32 * C::LDK + 8 * g;
+            const _Float16* krow = sKs + (ALT ? ugrp : i & 1) * C::TILE_K + l32 * C::LDK + 8 * g;
             // DMA layout: K row l32 (+32 kt) is row b = l32 % 4 of group l32 / 4
             // (+8 kt), its chunk 2 st + g at position 2 (st ^ 2b) + g, i.e. at
             // 16 (st % 2) + 32 ((st / 2) ^ b) halves: one base per st / 2.  V
@@ -416,8 +437,8 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
             const _Float16* vb[C::DMA ? C::NDT : 1];
             if constexpr (C::DMA) {
                 const int bk = l32 & 3, bv = (j16 >> 2) & 3;
-                const _Float16* k0 = sKs + (i & 1) * C::TILE_K + (l32 >> 2) * C::PSK + 128 * bk + 8 * g;
-                const _Float16* v0 = sVs + ((i - 1) & 1) * C::TILE_V + g * C::PSV + 128 * bv +
+                const _Float16* k0 = sKs + (ALT ? ugrp : i & 1) * C::TILE_K + (l32 >> 2) * C::PSK + 128 * bk + 8 * g;
+                const _Float16* v0 = sVs + (ALT ? ugrp : (i - 1) & 1) * C::TILE_V + g * C::PSV + 128 * bv +
                                      16 * ((lane >> 4) & 1) + 4 * (j16 & 3);
 #pragma unroll
                 for (int s2 = 0; s2 < 4; s2++) {
@@ -484,7 +505,7 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
                 return;
             }
             const bool do_pv = i >= 1 && cls_prev != 0;
-            const int cls_now = i < n ? tile_class(tcls, t_begin + i) : 0;
+            const int cls_now = i < ng ? tile_class(tcls, tile_at(i)) : 0;
             using T_ = std::true_type;
             using F_ = std::false_type;
             if (do_pv && cls_now != 0) {
@@ -503,7 +524,7 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
                 return;
             }
             if (cls_prev == 2) {
-                const int kt0 = (t_begin + i) * kBN;
+                const int kt0 = tile_at(i) * kBN;
                 const int a = row_lo - kt0 - 4 * g;
                 const int bnd = row_hi - kt0 - 4 * g;
 #pragma unroll
@@ -563,7 +584,7 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
         // (DMA: group B's K(0) in flight while Q stages)
         const bool dma_wave = __builtin_amdgcn_readfirstlane(grp) == 1;
         if constexpr (C::DMA) {
-            if (dma_wave && n > 0) {
+            if ((ALT || dma_wave) && n > 0) {
                 const DmaPair d0 = dma_pair(0);
 #pragma unroll
                 for (int k = 0; k < 8; k += 2) {
@@ -575,7 +596,7 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
         }
         stage_q();
         if constexpr (C::DMA) {
-            if (dma_wave) {
+            if (ALT || dma_wave) {
                 __builtin_amdgcn_s_waitcnt(waitcnt_vm(0)); // K(0) landed (not tracked by the compiler)
             }
         } else if (n > 0) {
@@ -585,7 +606,39 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
         __syncthreads();
         read_q();
         // Both groups pass 2n + 2 barriers; group B starts one phase late.
-        if (n > 0) {
+        if constexpr (ALT) {
+            // n2 steps of group A; group B's last may be missing
+            const int n2 = (n + 1) / 2;
+            if (n > 0) {
+                if (dma_wave) {
+                    __syncthreads();
+                }
+                for (int i = 0; i < n2; i++) {
+                    phase_m(i);
+                    __syncthreads();
+                    if constexpr (C::DMA) {
+                        const DmaPair d = dma_pair(i + 1);
+#pragma unroll
+                        for (int k = 0; k < 8; k++) {
+                            dma_issue(d, k);
+                        }
+                    } else {
+                        store_pair(i + 1);
+                        load_pair(i + 2);
+                    }
+                    phase_v(i);
+                    if constexpr (C::DMA) {
+                        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0)); // K(i + 1), V(i) landed
+                    }
+                    __syncthreads();
+                }
+                phase_m(n2);
+                __syncthreads();
+                if (!dma_wave) {
+                    __syncthreads();
+                }
+            }
+        } else if (n > 0) {
             if (grp == 0) {
                 if constexpr (C::DMA) {
                     (void)dma_pair(0); // the address stepping starts at pair 0
@@ -663,6 +716,49 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
                 store_partial(oacc, m_run, l, g == 0, p.part_o, p.part_ml, row, D, 0, g,
                               [](int) { return 1.0f; });
             }
+        } else if constexpr (ALT) {
+            // group B's O into group A's: fp32 rows in the K/V area (free after
+            // the last barrier), (m, l) in the unused half of sQ
+            constexpr int LDM = D + 4;
+            static_assert(ROW_WAVES * 32 * LDM * 4 <= (2 * C::TILE_K + 2 * C::TILE_V) * 2, "O fits the K/V area");
+            float* const so = reinterpret_cast<float*>(smem) + (rw * 32 + l32) * LDM + 4 * g;
+            float2* const sml = reinterpret_cast<float2*>(sQ + ROW_WAVES * 32 * C::LDQ) + rw * 32 + l32;
+            const float l = pair_sum(l_run);
+            if (grp == 1 && wave_active) {
+#pragma unroll
+                for (int dt = 0; dt < C::NDT; dt++) {
+#pragma unroll
+                    for (int qq = 0; qq < 4; qq++) {
+                        *reinterpret_cast<f4*>(so + 32 * dt + 8 * qq) = f4{oacc[dt][4 * qq], oacc[dt][4 * qq + 1],
+                                                                           oacc[dt][4 * qq + 2], oacc[dt][4 * qq + 3]};
+                    }
+                }
+                if (g == 0) {
+                    *sml = float2{m_run, l};
+                }
+            }
+            __syncthreads();
+            if (grp == 0 && wave_active) {
+                const float2 other = *sml;
+                const float m = fmaxf(l > 0.0f ? m_run : -INFINITY, other.y > 0.0f ? other.x : -INFINITY);
+                const float wa = l > 0.0f ? fast_exp2(m_run - m) : 0.0f;
+                const float wb = other.y > 0.0f ? fast_exp2(other.x - m) : 0.0f;
+                const float ls = l * wa + other.y * wb;
+                const float inv = ls > 0.0f ? 1.0f / ls : 0.0f;
+#pragma unroll
+                for (int dt = 0; dt < C::NDT; dt++) {
+#pragma unroll
+                    for (int qq = 0; qq < 4; qq++) {
+                        const f4 x = *reinterpret_cast<const f4*>(so + 32 * dt + 8 * qq);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            oacc[dt][4 * qq + e] = oacc[dt][4 * qq + e] * wa + x[e] * wb;
+                        }
+                    }
+                }
+                store_o_tile<D, C::LDQ>(oacc, [&](int) { return f4{inv, inv, inv, inv}; }, sQ + rw * 32 * C::LDQ,
+                                        obase, q0, p.Sq, p.o_ss, lane);
+            }
         } else if (wave_active) {
             // O = O^T / l, through this wave's sQ slot (free since read_q)
             const float l = pair_sum(l_run);
@@ -689,19 +785,26 @@ __device__ __forceinline__ void pp_body(PrefillParams p) {
 
 template <int D, bool PRE>
 __global__ __launch_bounds__(kPPThreads, 1) void fa_fwd_f16_pp(PrefillParams p) {
-    pp_body<D, PRE, false>(p);
+    pp_body<D, PRE, PPMode::kWhole>(p);
 }
 
 template <int D, bool PRE>
 __global__ __launch_bounds__(kPPThreads, 1) void fa_fwd_f16_pp_split(PrefillParams p) {
-    pp_body<D, PRE, true>(p);
+    pp_body<D, PRE, PPMode::kSplit>(p);
+}
+
+template <int D, bool PRE>
+__global__ __launch_bounds__(kPPThreads, 1) void fa_fwd_f16_pp_alt(PrefillParams p) {
+    pp_body<D, PRE, PPMode::kAlternate>(p);
 }
 
 template <int D, bool PRE>
 int launch_pp_as(const PrefillParams& p, int64_t n_wg, hipStream_t stream, std::string& err) {
     // persistent: as many workgroups as the device holds at once, each
     // walking its share of the n_wg row tiles
-    auto* const kernel = p.splits > 1 ? &fa_fwd_f16_pp_split<D, PRE> : &fa_fwd_f16_pp<D, PRE>;
+    auto* const kernel = p.splits > 1   ? &fa_fwd_f16_pp_split<D, PRE>
+                         : p.alternate ? &fa_fwd_f16_pp_alt<D, PRE>
+                                       : &fa_fwd_f16_pp<D, PRE>;
     int64_t grid = n_wg;
     if (PPCfg<D>::PERSIST) {
         const int64_t resident = resident_workgroups(reinterpret_cast<const void*>(kernel), kPPThreads, err);
@@ -814,6 +917,63 @@ static int f16_prefill_splits(const AttnArgs& a, size_t max_partials) {
     return prefill_splits(a, a.D > 128 ? kKPairRows : 32 * kPPWaves, tile_us, tile_us, 1, max_partials);
 }
 
+// Steps of the longest sequence of row tiles that a workgroup of a persistent
+// prefill launch walks, `fixed` steps added per row tile: `rows` rows of G heads
+// per workgroup, `tiles_per_step` key tiles per step, head groups dealt to the
+// XCDs `chunk` at a time.  Follows persistent_item and wg_tile for XCD 0 of 8
+// with 32 workgroups (the others hold the same), of which every fourth and
+// the last are looked at.
+static double longest_walk(const AttnArgs& a, int rows, int tiles_per_step, double fixed, int chunk) {
+    const MaskSpec mask{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
+    const int row_tiles = (a.Sq + rows - 1) / rows;
+    const int head_groups = a.B * (a.Hq / prefill_group(a));
+    const int items = row_tiles * head_groups;
+    auto steps = [&](int rt) {
+        int lo, hi;
+        visible_key_range(mask, rt * rows, std::min((rt + 1) * rows, a.Sq) - 1, lo, hi);
+        return hi >= lo ? (hi / kBN - lo / kBN + tiles_per_step) / tiles_per_step : 0;
+    };
+    double longest = 0.0;
+    for (int w = 0; w < 32; w = w == 28 ? 31 : w + 4) {
+        double walk = 0.0;
+        for (int k = 0;; k++) {
+            const int slot = 32 * k + ((k & 1) ? 31 - w : w);
+            if (8 * slot >= items) {
+                break;
+            }
+            const int rt = chunk > 0 ? slot % (chunk * row_tiles) / chunk : 8 * slot / head_groups;
+            walk += fixed + steps(row_tiles - 1 - rt);
+        }
+        longest = std::max(longest, walk);
+    }
+    return longest;
+}
+
+bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us) {
+    // Twice as many row tiles of half as many steps, where the longest row
+    // tile of a launch sets its time: up to two row tiles per CU.  A row tile
+    // takes about 5 us beside its steps.
+    const int rows = 32 * kPPWaves / prefill_group(a);
+    const int head_groups = a.B * (a.Hq / prefill_group(a));
+    if (a.Sk <= 2 * kBN || (int64_t)((a.Sq + rows - 1) / rows) * head_groups > 512) {
+        return false;
+    }
+    const int chunk = xcd_head_group_chunk(head_groups, 4 * (int64_t)a.Sk * a.D);
+    return step_us * longest_walk(a, rows / 2, 2, 5.0 / step_us, chunk) <
+           0.97 * tile_us * longest_walk(a, rows, 1, 5.0 / tile_us, chunk);
+}
+
+// Whether the two groups of a workgroup take the key tiles in turn (D <= 128).
+// A step of 128 rows and two tiles takes about 1.4 times a step of 256 rows and
+// one.  Measured, us a call, whole against alternating (Hq 32 Hkv 8, causal): B1
+// S1024 D128 29.0 / 20.6, D64 22.5 / 15.8; B1 S2048 D128 55 / 45; B2 S1024 D128
+// 31.8 / 30.5; and where the rule keeps whole row tiles: B1 S2048 D128 not
+// causal 71 / 79, B2 S1500 49 / 58, B2 S2048 78 / 92.
+static bool f16_prefill_alternate(const AttnArgs& a) {
+    const double tile_us = 0.4 + a.D / 128.0;
+    return a.D <= 128 && prefill_alternate(a, tile_us, 1.4 * tile_us);
+}
+
 int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err, ScratchRegion* region) {
     PrefillParams p{};
     p.q = static_cast<const _Float16*>(a.q);
@@ -844,6 +1004,11 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
     // or 4 pairs of waves of 32 rows (D > 128)
     p.G = prefill_group(a);
     p.rows_per_wg = (kpair ? kKPairRows : dpair ? kDPairRows : 32 * kPPWaves) / p.G;
+    p.splits = f16_prefill_splits(a, region != nullptr ? region->bytes - region->used : SIZE_MAX);
+    p.alternate = p.splits == 1 && f16_prefill_alternate(a);
+    if (p.alternate) {
+        p.rows_per_wg /= 2;
+    }
     p.n_row_tiles = (a.Sq + p.rows_per_wg - 1) / p.rows_per_wg;
     p.groups_per_kv = p.ratio / p.G;
     p.n_head_groups = a.B * a.Hkv * p.groups_per_kv;
@@ -854,7 +1019,6 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
     p.mask = MaskSpec{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
     p.rope_q = rope_q ? 1 : 0;
 
-    p.splits = f16_prefill_splits(a, region != nullptr ? region->bytes - region->used : SIZE_MAX);
     const int64_t n_wg = (int64_t)p.n_row_tiles * p.n_head_groups * p.splits;
     p.n_items = (int32_t)std::min<int64_t>(n_wg, INT32_MAX);
     if (n_wg <= 0) {

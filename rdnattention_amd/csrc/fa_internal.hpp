@@ -130,6 +130,11 @@ SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_b
 int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double split_tile_us, int launches,
                    size_t max_partials);
 
+// Whether a prefill launch of the ping-pong kernels (256 rows of G heads per
+// workgroup, tile_us per 64-key tile) ends sooner with 128 rows and two tiles
+// per step of step_us.
+bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us);
+
 // Before and after a launch of `splits` key splits: `r` from the arguments, with
 // the partials taken from `ws`; and the combine launch.  0, or -1 with `err`.
 struct SplitRows;

@@ -37,6 +37,7 @@ struct PrefillParams {
     // key splits of every row tile (the split instantiations): the grid has
     // splits * n_row_tiles "row tiles", and each writes its rows' partials
     int32_t splits;
+    int32_t alternate; // the instantiations whose two groups take the key tiles in turn (128 rows)
     float* part_o;  // [splits][B * Hq * Sq][D] (SplitRows)
     float* part_ml; // [splits][B * Hq * Sq][2]
     int64_t n_rows; // B * Hq * Sq

@@ -520,3 +520,42 @@ def test_cached_scratch_two_streams_and_growth(gpu, oracle_lib):
                           reference_f16(q.cpu(), k.cpu(), v.cpu(), causal, -1, cd.cpu().numpy(), sd.cpu().numpy()),
                           f"cached scratch {i}")
     rdnattention.trim_scratch()
+
+
+# d, hq, hkv, sq, sk, causal, window, rope, scale: launches of few row tiles,
+# whose two groups of waves take the key tiles in turn: odd and even tile
+# counts, a group without tiles in some row tiles (causal), rows without keys,
+# ragged ends, windows, RoPE, Q not pre-scaled (|scale| log2 e > 1) and negative
+ALTERNATE_CASES = [(d, 8, 2, s, s, c, -1, False, None) for d in (32, 64, 96, 128)
+                   for s, c in ((321, True), (640, False), (705, True))] + [
+    (128, 4, 4, 500, 500, True, -1, True, None),
+    (128, 8, 1, 130, 450, True, 200, False, None),
+    (64, 4, 2, 600, 600, False, 300, True, None),
+    (128, 4, 2, 700, 400, True, -1, False, None),
+    (64, 4, 4, 400, 400, True, -1, False, 1.5),
+    (128, 2, 1, 400, 400, False, -1, False, -0.2),
+    (96, 5, 1, 333, 333, True, -1, False, -1.0),
+]
+
+
+@pytest.mark.parametrize("case", ALTERNATE_CASES,
+                         ids=["d{}h{}kv{}q{}k{}c{:d}w{}r{:d}s{}".format(*c) for c in ALTERNATE_CASES])
+def test_few_row_tiles_vs_oracle(gpu, oracle_lib, case):
+    """FP16 bar against the oracle (V at the bar's N(0, 1))."""
+    d, hq, hkv, sq, sk, causal, window, rope, scale = case
+    log(f"[few row tiles] {case}")
+    q, k, v = seeded_inputs(61, 2, hq, hkv, sq, sk, d)
+    cos = sin = cd = sd = None
+    if rope:
+        cos, sin = oracle.rope_tables(max(sq, sk), d)
+        cd, sd = torch.from_numpy(cos).to(gpu), torch.from_numpy(sin).to(gpu)
+    if scale is not None:  # keep the scores' spread at that of 1 / sqrt(d)
+        k = (k.float() / (abs(scale) * d ** 0.5)).half()
+    ref = reference_f16(q, k, v, causal, window, cos, sin, scale=scale)
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    outs = [torch.full_like(qd, float("nan")) for _ in range(2)]
+    for o in outs:
+        assert forward_raw(qd, kd, vd, o, causal, window, cd, sd, scale=scale) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    assert_f16_parity(outs[0].float().cpu().numpy(), ref, "few row tiles")
