@@ -30,6 +30,7 @@ logger = logging.getLogger(__name__)
 __version__ = "0.1.0"
 
 _lib = None
+_torch_module = None  # torch, once a call has needed it (the package imports without it)
 
 SUPPORTED_HEAD_DIMS = tuple(range(32, 513, 32))
 SUPPORTED_HEAD_DIMS_INT8 = (64, 128)
@@ -151,14 +152,13 @@ def last_error() -> str:
     return _lib_handle().rdna_get_error().decode()
 
 
-def _validate_inputs(query, key, value, expected_dtype) -> None:
-    # rdnattention/__init__.py:138-155
-    import torch
-
-    if not isinstance(query, torch.Tensor):
+def _validate_inputs(query, key, value, expected_dtype):
+    # rdnattention/__init__.py:138-155; returns _check_shapes' shapes
+    tensor = _torch().Tensor
+    if not isinstance(query, tensor):
         raise TypeError("requires torch.Tensor inputs (GPU tensors already on this device)")
     for name, t in (("query", query), ("key", key), ("value", value)):
-        if not isinstance(t, torch.Tensor):
+        if not isinstance(t, tensor):
             raise TypeError("requires torch.Tensor inputs (GPU tensors already on this device)")
         if not t.is_cuda:
             raise ValueError(f"{name} must be on a HIP device")
@@ -168,23 +168,27 @@ def _validate_inputs(query, key, value, expected_dtype) -> None:
             raise ValueError(f"{name} must be 4D [batch, heads, seq, head_dim], got shape {tuple(t.shape)}")
         if not t.is_contiguous():
             raise ValueError(f"{name} must be contiguous - call .contiguous() first")
-    _check_shapes(query, key, value)
+    return _check_shapes(query, key, value)
 
 
-def _check_shapes(query, key, value) -> None:
+def _check_shapes(query, key, value):
     """The shape relations every kernel relies on: one batch size, V shaped
     like K, one head_dim, and a whole number of query heads per kv head.  The
     first and last are the reference's checks (rdnattention/__init__.py:151-
     155); the kernels would read past the end of a smaller K/V otherwise, so
-    the middle two are added here."""
-    if query.shape[0] != key.shape[0] or query.shape[0] != value.shape[0]:
+    the middle two are added here.  Returns the shapes of query and key as
+    tuples (each .shape builds a torch.Size: the ten of this function took
+    half as long as a kernel launch)."""
+    qs, ks, vs = tuple(query.shape), tuple(key.shape), tuple(value.shape)
+    if qs[0] != ks[0] or qs[0] != vs[0]:
         raise ValueError(f"Batch size must match: Q={query.shape}, K={key.shape}, V={value.shape}")
-    if tuple(key.shape) != tuple(value.shape):
-        raise ValueError(f"key and value must have the same shape: K={tuple(key.shape)}, V={tuple(value.shape)}")
-    if key.shape[3] != query.shape[3]:
-        raise ValueError(f"key head_dim ({key.shape[3]}) must equal query head_dim ({query.shape[3]})")
-    if key.shape[1] == 0 or query.shape[1] % key.shape[1] != 0:
-        raise ValueError(f"Q heads ({query.shape[1]}) must be a multiple of K heads ({key.shape[1]})")
+    if ks != vs:
+        raise ValueError(f"key and value must have the same shape: K={ks}, V={vs}")
+    if ks[3] != qs[3]:
+        raise ValueError(f"key head_dim ({ks[3]}) must equal query head_dim ({qs[3]})")
+    if ks[1] == 0 or qs[1] % ks[1] != 0:
+        raise ValueError(f"Q heads ({qs[1]}) must be a multiple of K heads ({ks[1]})")
+    return qs, ks
 
 
 def _check_head_dim(head_dim: int, who: str, allowed=SUPPORTED_HEAD_DIMS):
@@ -198,10 +202,9 @@ def _check_head_dim(head_dim: int, who: str, allowed=SUPPORTED_HEAD_DIMS):
 def _rope_ptrs(rot_cos, rot_sin, query, seq_len, key_seq_len, head_dim):
     """Validates the angle tables (rdnattention/__init__.py:165-192).
     Returns (cos_ptr, sin_ptr, has_rope)."""
-    import torch
-
     if rot_cos is None and rot_sin is None:
         return None, None, 0
+    torch = _torch()
     if rot_cos is None or rot_sin is None:
         raise ValueError("pass both rot_cos and rot_sin, or neither")
     rows = max(seq_len, key_seq_len)
@@ -223,10 +226,23 @@ def _rope_ptrs(rot_cos, rot_sin, query, seq_len, key_seq_len, head_dim):
     return rot_cos.data_ptr(), rot_sin.data_ptr(), 1
 
 
-def _stream():
-    import torch
+def _torch():
+    global _torch_module
+    if _torch_module is None:
+        import torch
 
-    return torch.cuda.current_stream().cuda_stream
+        _torch_module = torch
+    return _torch_module
+
+
+def _stream():
+    """The current device's current stream, as torch.cuda.current_stream()
+    .cuda_stream names it (without the Stream object around it, 2.8 us)."""
+    torch = _torch()
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch.cuda.current_device())
 
 
 def flash_attn(query, key, value, is_causal: bool = False, window_size: int = -1, rot_cos=None, rot_sin=None):
@@ -240,14 +256,12 @@ def flash_attn(query, key, value, is_causal: bool = False, window_size: int = -1
     Q and K inside the kernel (channels 2i, 2i+1 rotate by column i).
     The softmax scale is 1/sqrt(head_dim).  Returns a new tensor like query.
     """
-    import torch
-
-    _validate_inputs(query, key, value, torch.float16)
-    _check_head_dim(query.shape[-1], "flash_attn")
+    torch = _torch()
+    (batch, heads, seq_len, head_dim), (_, kv_heads, key_seq_len, _) = _validate_inputs(query, key, value,
+                                                                                       torch.float16)
+    _check_head_dim(head_dim, "flash_attn")
     if not has_device():
         raise RDNAttentionError("no usable HIP device found")
-    batch, heads, seq_len, head_dim = query.shape
-    _, kv_heads, key_seq_len, _ = key.shape
     cos_ptr, sin_ptr, has_rope = _rope_ptrs(rot_cos, rot_sin, query, seq_len, key_seq_len, head_dim)
     output = torch.empty_like(query)
     if output.numel() == 0:
@@ -274,8 +288,7 @@ def attention_forward_into(query, key, value, output, *, is_causal: bool = False
     of 8 elements, e.g. K/V sliced from a [B, S, 2, Hkv, D] cache).
     `scale` defaults to 1/sqrt(head_dim); `path` is PATH_AUTO, PATH_PREFILL or
     PATH_SPLITK.  Asynchronous on torch's current stream."""
-    import torch
-
+    torch = _torch()
     for name, t in (("query", query), ("key", key), ("value", value), ("output", output)):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{name} must be a torch.Tensor")
@@ -285,9 +298,7 @@ def attention_forward_into(query, key, value, output, *, is_causal: bool = False
             raise ValueError(f"{name} must have a contiguous head_dim axis")
     if output.shape != query.shape:
         raise ValueError("output must have the shape of query")
-    _check_shapes(query, key, value)
-    batch, heads, seq_len, head_dim = query.shape
-    _, kv_heads, key_seq_len, _ = key.shape
+    (batch, heads, seq_len, head_dim), (_, kv_heads, key_seq_len, _) = _check_shapes(query, key, value)
     cos_ptr, sin_ptr, has_rope = _rope_ptrs(rot_cos, rot_sin, query, seq_len, key_seq_len, head_dim)
     qs, ks, vs, os_ = query.stride(), key.stride(), value.stride(), output.stride()
     result = _lib_handle().rdna_attention_forward_path(
@@ -309,18 +320,14 @@ def flash_attn_int8qk(query, key, value, q_scale, k_scale, v_scale: float, is_ca
     of per-token scales shaped (batch, heads, seq_len) / (batch, kv_heads,
     key_seq_len); v_scale: float.  Output float16.  No RoPE.
     """
-    import torch
-
-    _validate_inputs(query, key, value, torch.int8)
-    heads, kv_heads_ = query.shape[1], key.shape[1]
-    if kv_heads_ == 0 or heads % kv_heads_ != 0:
+    torch = _torch()
+    (batch, heads, seq_len, head_dim), (_, kv_heads, key_seq_len, _) = _validate_inputs(query, key, value, torch.int8)
+    if kv_heads == 0 or heads % kv_heads != 0:
         raise RDNAttentionError(
-            f"flash_attn_int8qk: query heads ({heads}) must be a positive multiple of key/value heads ({kv_heads_})")
-    _check_head_dim(query.shape[-1], "flash_attn_int8qk", allowed=SUPPORTED_HEAD_DIMS_INT8)
+            f"flash_attn_int8qk: query heads ({heads}) must be a positive multiple of key/value heads ({kv_heads})")
+    _check_head_dim(head_dim, "flash_attn_int8qk", allowed=SUPPORTED_HEAD_DIMS_INT8)
     if not has_device():
         raise RDNAttentionError("no usable HIP device found")
-    batch, heads, seq_len, head_dim = query.shape
-    _, kv_heads, key_seq_len, _ = key.shape
 
     def _scale_arg(x, name, want):
         if not isinstance(x, torch.Tensor):
@@ -365,16 +372,13 @@ def attention_int8_forward_into(query, key, value, output, q_scale, k_scale, v_s
     of per-token V scales, each V row dequantised by its own scale in the
     kernel (rdna_attention_forward_int8qk_vtoken; exclusive with v_channel).
     Asynchronous on torch's current stream."""
-    import torch
-
+    torch = _torch()
     for name, t in (("query", query), ("key", key), ("value", value)):
         if not isinstance(t, torch.Tensor) or t.dtype != torch.int8 or t.dim() != 4 or not t.is_cuda:
             raise ValueError(f"{name} must be a 4D int8 HIP tensor")
     if output.dtype != torch.float16 or output.shape != query.shape or not output.is_cuda:
         raise ValueError("output must be a float16 HIP tensor with the shape of query")
-    _check_shapes(query, key, value)
-    batch, heads, seq_len, head_dim = query.shape
-    _, kv_heads, key_seq_len, _ = key.shape
+    (batch, heads, seq_len, head_dim), (_, kv_heads, key_seq_len, _) = _check_shapes(query, key, value)
 
     def _scale_arg(x, name, want):
         if not isinstance(x, torch.Tensor):
