@@ -158,6 +158,20 @@ RDNA_API int32_t rdna_quantize_int8(
     int32_t per_channel, const void* rot_cos, const void* rot_sin,
     void* q_out, void* scale_out, void* hip_stream);
 
+/* rdna_quantize_int8 of the Q, K and V of one attention call in one launch (two
+ * with a per-channel V), the same values: q [batch, num_heads, seq_len,
+ * head_dim] and k, v [batch, num_kv_heads, key_seq_len, head_dim], all of one
+ * dtype; Q and K per token, rotated first when rot_cos / rot_sin are given, V
+ * per channel (v_per_channel != 0) or per token.  Outputs and checks as for
+ * rdna_quantize_int8.  No reference counterpart. */
+RDNA_API int32_t rdna_quantize_int8_qkv(
+    const void* q, const void* k, const void* v, int32_t dtype, int64_t q_stride_b, int64_t q_stride_h,
+    int64_t q_stride_s, int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_s, int64_t v_stride_b,
+    int64_t v_stride_h, int64_t v_stride_s, uint32_t batch_size, uint32_t num_heads, uint32_t num_kv_heads,
+    uint32_t seq_len, uint32_t key_seq_len, uint32_t head_dim, int32_t v_per_channel, const void* rot_cos,
+    const void* rot_sin, void* q_out, void* k_out, void* v_out, void* q_scale_out, void* k_scale_out,
+    void* v_scale_out, void* hip_stream);
+
 /* Kernel timer.  While enabled, each launch of a main attention kernel
  * (prefill, split-K, int8; not the RoPE pre-rotation or split-K combine
  * kernels) is bracketed by a HIP event pair recorded on its stream.

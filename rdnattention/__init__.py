@@ -119,6 +119,11 @@ def _lib_handle():
         lib.rdna_attention_forward_int8qk_vtoken.restype = _I32
         lib.rdna_quantize_int8.argtypes = [_VP, _I32] + [_I64] * 3 + [_U32] * 4 + [_I32, _VP, _VP, _VP, _VP, _VP]
         lib.rdna_quantize_int8.restype = _I32
+        try:  # absent from libraries built before it existed
+            lib.rdna_quantize_int8_qkv.argtypes = [_VP] * 3 + [_I32] + [_I64] * 9 + [_U32] * 6 + [_I32] + [_VP] * 9
+            lib.rdna_quantize_int8_qkv.restype = _I32
+        except AttributeError:
+            pass
         lib.rdna_int8_qk_scores.argtypes = [_VP] * 3 + [_I64] * 6 + [_U32] * 6 + [_VP]
         lib.rdna_int8_qk_scores.restype = _I32
         try:  # absent from libraries built before it existed
@@ -492,9 +497,10 @@ def _quantize_gpu(x, per_channel: bool, rot_cos=None, rot_sin=None):
     if has_rope and per_channel:
         raise ValueError("RoPE applies to the per-token (query/key) quantiser only")
     q = torch.empty((b, h, s, d), dtype=torch.int8, device=x.device)
-    sc = torch.ones((b, h, d) if per_channel else (b, h, s), dtype=torch.float32, device=x.device)
+    sc_shape = (b, h, d) if per_channel else (b, h, s)
     if q.numel() == 0:
-        return q, sc
+        return q, torch.ones(sc_shape, dtype=torch.float32, device=x.device)
+    sc = torch.empty(sc_shape, dtype=torch.float32, device=x.device)
     st = x.stride()
     rc = _lib_handle().rdna_quantize_int8(x.data_ptr(), dt, st[0], st[1], st[2], b, h, s, d, 1 if per_channel else 0,
                                           cos_ptr, sin_ptr, q.data_ptr(), sc.data_ptr(), _stream())
@@ -605,8 +611,8 @@ def flash_attn_int8qk_quantized(query, key, value, is_causal: bool = False, wind
     inside the per-token quantiser (the FP16 path's arithmetic), so RoPE costs
     no extra pass.
 
-    Three quantiser kernels and one attention kernel: the per-channel V
-    rescale is applied in the attention kernel's epilogue
+    Two quantiser launches (rdna_quantize_int8_qkv; one with v_per_token) and
+    the attention kernel: the per-channel V rescale is applied in the attention kernel's epilogue
     (rdna_attention_forward_int8qk_vchannel) instead of a separate pass over
     the output, and the per-tensor Q/K quantisation the reference computes and
     discards is skipped.  The output is rounded to fp16 once (the reference
@@ -619,8 +625,7 @@ def flash_attn_int8qk_quantized(query, key, value, is_causal: bool = False, wind
     v_per_token (an extension): V is quantised per token instead of per
     channel, and the kernel dequantises each V row by its scale
     (rdna_attention_forward_int8qk_vtoken)."""
-    import torch
-
+    torch = _torch()
     for name, t in (("query", query), ("key", key), ("value", value)):
         if not isinstance(t, torch.Tensor):
             raise TypeError("requires torch.Tensor inputs (GPU tensors already on this device)")
@@ -632,14 +637,38 @@ def flash_attn_int8qk_quantized(query, key, value, is_causal: bool = False, wind
     if kv_heads == 0 or heads % kv_heads != 0:
         raise RDNAttentionError(
             f"flash_attn_int8qk: query heads ({heads}) must be a positive multiple of key/value heads ({kv_heads})")
-    _check_shapes(query, key, value)
-    _check_head_dim(query.shape[-1], "flash_attn_int8qk", allowed=SUPPORTED_HEAD_DIMS_INT8)
+    (batch, heads, seq_len, head_dim), (_, kv_heads, key_seq_len, _) = _check_shapes(query, key, value)
+    _check_head_dim(head_dim, "flash_attn_int8qk", allowed=SUPPORTED_HEAD_DIMS_INT8)
     if not has_device():
         raise RDNAttentionError("no usable HIP device found")
-    _rope_ptrs(rot_cos, rot_sin, query, query.shape[2], key.shape[2], query.shape[3])
-    qi, q_scale = _quantize_gpu(query, per_channel=False, rot_cos=rot_cos, rot_sin=rot_sin)
-    ki, k_scale = _quantize_gpu(key, per_channel=False, rot_cos=rot_cos, rot_sin=rot_sin)
-    vi, v_sc = _quantize_gpu(value, per_channel=not v_per_token)
+    cos_ptr, sin_ptr, _ = _rope_ptrs(rot_cos, rot_sin, query, seq_len, key_seq_len, head_dim)
+    strides = query.stride() + key.stride() + value.stride()
+    mult = 8 if query.dtype == torch.float16 else 4
+    fused = (query.dtype in (torch.float16, torch.float32) and query.dtype == key.dtype == value.dtype
+             and query.device == key.device == value.device and query.numel() > 0 and key.numel() > 0
+             and strides[3] == strides[7] == strides[11] == 1
+             and not any(strides[i] % mult for i in (0, 1, 2, 4, 5, 6, 8, 9, 10))
+             and not (query.data_ptr() | key.data_ptr() | value.data_ptr()) % 16
+             and hasattr(_lib_handle(), "rdna_quantize_int8_qkv"))
+    if not fused:  # other layouts and dtypes: tensor by tensor
+        qi, q_scale = _quantize_gpu(query, per_channel=False, rot_cos=rot_cos, rot_sin=rot_sin)
+        ki, k_scale = _quantize_gpu(key, per_channel=False, rot_cos=rot_cos, rot_sin=rot_sin)
+        vi, v_sc = _quantize_gpu(value, per_channel=not v_per_token)
+    else:
+        dev = query.device
+        qi = torch.empty((batch, heads, seq_len, head_dim), dtype=torch.int8, device=dev)
+        ki, vi = torch.empty((2, batch, kv_heads, key_seq_len, head_dim), dtype=torch.int8, device=dev).unbind(0)
+        q_scale = torch.empty((batch, heads, seq_len), dtype=torch.float32, device=dev)
+        k_scale = torch.empty((batch, kv_heads, key_seq_len), dtype=torch.float32, device=dev)
+        v_sc = torch.empty((batch, kv_heads, key_seq_len if v_per_token else head_dim), dtype=torch.float32,
+                           device=dev)
+        rc = _lib_handle().rdna_quantize_int8_qkv(
+            query.data_ptr(), key.data_ptr(), value.data_ptr(), 0 if query.dtype == torch.float16 else 1,
+            *strides[0:3], *strides[4:7], *strides[8:11], batch, heads, kv_heads, seq_len, key_seq_len, head_dim,
+            0 if v_per_token else 1, cos_ptr, sin_ptr, qi.data_ptr(), ki.data_ptr(), vi.data_ptr(),
+            q_scale.data_ptr(), k_scale.data_ptr(), v_sc.data_ptr(), _stream())
+        if rc != 0:
+            raise RDNAttentionError(f"quantisation failed: {last_error()}")
     output = torch.empty(query.shape, dtype=torch.float16, device=query.device)
     if output.numel() == 0:
         return output

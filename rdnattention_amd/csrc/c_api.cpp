@@ -402,49 +402,85 @@ RDNA_API int32_t rdna_attention_forward_int8qk_vtoken(
 #endif
 }
 
+// Quantiser arguments, checked: "" or what is wrong.
+static std::string quant_args(const void* x, int32_t x_dtype, int64_t x_stride_b, int64_t x_stride_h,
+                              int64_t x_stride_s, uint32_t batch_size, uint32_t num_heads, uint32_t seq_len,
+                              uint32_t head_dim, int32_t per_channel, const void* rot_cos, const void* rot_sin,
+                              void* q_out, void* scale_out, rdna_amd::QuantArgs& a) {
+    const int64_t mult = x_dtype == 1 ? 4 : 8; // elements per 16 bytes
+    if (x_dtype != 0 && x_dtype != 1) {
+        return "x_dtype must be 0 (fp16) or 1 (fp32)";
+    } else if (head_dim < 8 || head_dim > 512 || head_dim % 8 != 0) {
+        return "head_dim must be a multiple of 8 from 8 to 512";
+    } else if (batch_size == 0 || num_heads == 0 || seq_len == 0) {
+        return "empty tensor (batch_size, num_heads and seq_len must be non-zero)";
+    } else if (seq_len > kMaxSeq || (uint64_t)batch_size * num_heads > (uint64_t)INT32_MAX / 2) {
+        return "tensor dimensions exceed the supported range";
+    } else if (x == nullptr || q_out == nullptr || scale_out == nullptr) {
+        return "null tensor pointer";
+    } else if (!aligned(x, 16) || !aligned(q_out, 16) || !aligned(scale_out, 4)) {
+        return "x and q_out must be 16-byte aligned, scale_out 4-byte aligned";
+    } else if (x_stride_b % mult != 0 || x_stride_h % mult != 0 || x_stride_s % mult != 0) {
+        return "batch/head/seq strides of x must be multiples of 16 bytes";
+    } else if ((rot_cos == nullptr) != (rot_sin == nullptr)) {
+        return "pass both rot_cos and rot_sin, or neither";
+    } else if (rot_cos != nullptr && per_channel != 0) {
+        return "RoPE applies to the per-token scheme only";
+    } else if (!aligned(rot_cos, 16) || !aligned(rot_sin, 16)) {
+        return "rot_cos and rot_sin must be 16-byte aligned";
+    }
+    a.x = x;
+    a.x_fp32 = x_dtype == 1 ? 1 : 0;
+    a.xs[0] = x_stride_b, a.xs[1] = x_stride_h, a.xs[2] = x_stride_s;
+    a.B = (int32_t)batch_size;
+    a.H = (int32_t)num_heads;
+    a.S = (int32_t)seq_len;
+    a.D = (int32_t)head_dim;
+    a.per_channel = per_channel != 0 ? 1 : 0;
+    a.rot_cos = static_cast<const float*>(rot_cos);
+    a.rot_sin = static_cast<const float*>(rot_sin);
+    a.q = q_out;
+    a.scale = static_cast<float*>(scale_out);
+    return "";
+}
+
 RDNA_API int32_t rdna_quantize_int8(const void* x, int32_t x_dtype, int64_t x_stride_b, int64_t x_stride_h,
                                     int64_t x_stride_s, uint32_t batch_size, uint32_t num_heads, uint32_t seq_len,
                                     uint32_t head_dim, int32_t per_channel, const void* rot_cos,
                                     const void* rot_sin, void* q_out, void* scale_out, void* hip_stream) {
-    std::string err;
-    const int64_t mult = x_dtype == 1 ? 4 : 8; // elements per 16 bytes
-    if (x_dtype != 0 && x_dtype != 1) {
-        err = "x_dtype must be 0 (fp16) or 1 (fp32)";
-    } else if (head_dim < 8 || head_dim > 512 || head_dim % 8 != 0) {
-        err = "head_dim must be a multiple of 8 from 8 to 512";
-    } else if (batch_size == 0 || num_heads == 0 || seq_len == 0) {
-        err = "empty tensor (batch_size, num_heads and seq_len must be non-zero)";
-    } else if (seq_len > kMaxSeq || (uint64_t)batch_size * num_heads > (uint64_t)INT32_MAX / 2) {
-        err = "tensor dimensions exceed the supported range";
-    } else if (x == nullptr || q_out == nullptr || scale_out == nullptr) {
-        err = "null tensor pointer";
-    } else if (!aligned(x, 16) || !aligned(q_out, 16) || !aligned(scale_out, 4)) {
-        err = "x and q_out must be 16-byte aligned, scale_out 4-byte aligned";
-    } else if (x_stride_b % mult != 0 || x_stride_h % mult != 0 || x_stride_s % mult != 0) {
-        err = "batch/head/seq strides of x must be multiples of 16 bytes";
-    } else if ((rot_cos == nullptr) != (rot_sin == nullptr)) {
-        err = "pass both rot_cos and rot_sin, or neither";
-    } else if (rot_cos != nullptr && per_channel != 0) {
-        err = "RoPE applies to the per-token scheme only";
-    } else if (!aligned(rot_cos, 16) || !aligned(rot_sin, 16)) {
-        err = "rot_cos and rot_sin must be 16-byte aligned";
-    } else {
-        rdna_amd::QuantArgs a;
-        a.x = x;
-        a.x_fp32 = x_dtype == 1 ? 1 : 0;
-        a.xs[0] = x_stride_b, a.xs[1] = x_stride_h, a.xs[2] = x_stride_s;
-        a.B = (int32_t)batch_size;
-        a.H = (int32_t)num_heads;
-        a.S = (int32_t)seq_len;
-        a.D = (int32_t)head_dim;
-        a.per_channel = per_channel != 0 ? 1 : 0;
-        a.rot_cos = static_cast<const float*>(rot_cos);
-        a.rot_sin = static_cast<const float*>(rot_sin);
-        a.q = q_out;
-        a.scale = static_cast<float*>(scale_out);
-        if (rdna_amd::quantize_int8(a, static_cast<hipStream_t>(hip_stream), err) == 0) {
-            return 0;
-        }
+    rdna_amd::QuantArgs a;
+    std::string err = quant_args(x, x_dtype, x_stride_b, x_stride_h, x_stride_s, batch_size, num_heads, seq_len,
+                                 head_dim, per_channel, rot_cos, rot_sin, q_out, scale_out, a);
+    if (err.empty() && rdna_amd::quantize_int8(a, static_cast<hipStream_t>(hip_stream), err) == 0) {
+        return 0;
+    }
+    set_error("Quantize (int8) failed: %s", err);
+    return -3;
+}
+
+RDNA_API int32_t rdna_quantize_int8_qkv(const void* q, const void* k, const void* v, int32_t dtype,
+                                        int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_s,
+                                        int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_s,
+                                        int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_s,
+                                        uint32_t batch_size, uint32_t num_heads, uint32_t num_kv_heads,
+                                        uint32_t seq_len, uint32_t key_seq_len, uint32_t head_dim,
+                                        int32_t v_per_channel, const void* rot_cos, const void* rot_sin, void* q_out,
+                                        void* k_out, void* v_out, void* q_scale_out, void* k_scale_out,
+                                        void* v_scale_out, void* hip_stream) {
+    rdna_amd::QuantArgs aq, ak, av;
+    std::string err = quant_args(q, dtype, q_stride_b, q_stride_h, q_stride_s, batch_size, num_heads, seq_len,
+                                 head_dim, 0, rot_cos, rot_sin, q_out, q_scale_out, aq);
+    if (err.empty()) {
+        err = quant_args(k, dtype, k_stride_b, k_stride_h, k_stride_s, batch_size, num_kv_heads, key_seq_len,
+                         head_dim, 0, rot_cos, rot_sin, k_out, k_scale_out, ak);
+    }
+    if (err.empty()) {
+        err = quant_args(v, dtype, v_stride_b, v_stride_h, v_stride_s, batch_size, num_kv_heads, key_seq_len,
+                         head_dim, v_per_channel, nullptr, nullptr, v_out, v_scale_out, av);
+    }
+    if (err.empty() &&
+        rdna_amd::quantize_int8_qkv(aq, ak, av, static_cast<hipStream_t>(hip_stream), err) == 0) {
+        return 0;
     }
     set_error("Quantize (int8) failed: %s", err);
     return -3;

@@ -75,6 +75,11 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err);
 // INT8 quantisation on the GPU (fa_quant.hip).  Returns 0 or sets `err`.
 int quantize_int8(const QuantArgs& a, hipStream_t stream, std::string& err);
 
+// Q and K per token and V (per token or per channel) of one attention call: the
+// same B, D, x_fp32 and, for Q and K, tables.  Returns 0 or sets `err`.
+int quantize_int8_qkv(const QuantArgs& q, const QuantArgs& k, const QuantArgs& v, hipStream_t stream,
+                      std::string& err);
+
 // Test export: exact int32 S = Q_i8 K_i8^T into `scores` [B,Hq,Sq,Sk] (contiguous).
 int int8_scores(const AttnArgs& a, int32_t* scores, hipStream_t stream, std::string& err);
 

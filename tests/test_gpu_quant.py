@@ -246,3 +246,44 @@ def test_quantized_rope_end_to_end(gpu, oracle_lib, causal, hkv):
     mx, mean, _ = errors(got, emu * vscale)
     log(f"[quant]   vs emulation max={mx:.2e} mean={mean:.2e}")
     assert mx <= I8_MAX_ABS
+
+
+# b, hq, hkv, sq, sk, d: one row, one chunk of 64 rows and its edges, many chunks
+QKV_CASES = [(1, 4, 2, 1, 1, 64), (1, 2, 2, 63, 64, 128), (2, 8, 2, 65, 129, 64), (1, 16, 4, 2050, 2050, 64),
+             (2, 8, 8, 700, 3000, 128), (40, 32, 32, 3, 70, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["f16", "f32"])
+@pytest.mark.parametrize("rope,v_per_token", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("case", QKV_CASES, ids=["b{}h{}kv{}q{}k{}d{}".format(*c) for c in QKV_CASES])
+def test_qkv_quantiser_matches_tensor_by_tensor(gpu, case, rope, v_per_token, dtype):
+    """rdna_quantize_int8_qkv writes the bits that three rdna_quantize_int8
+    calls write (strided K and V: views into one cache), also into the
+    partials of an earlier, larger call."""
+    import rdnattention as ra
+
+    b, hq, hkv, sq, sk, d = case
+    log(f"[quant qkv] {case} rope={rope} v_per_token={v_per_token} {dtype}")
+    g = torch.Generator(device=gpu).manual_seed(71)
+    q = torch.randn(b, hq, sq, d, device=gpu, generator=g).to(dtype)
+    cache = torch.randn(b, sk, 2, hkv, d, device=gpu, generator=g).to(dtype)
+    k, v = cache[:, :, 0].transpose(1, 2), cache[:, :, 1].transpose(1, 2)
+    v[..., 3] = 0  # a channel of zeros: scale 1
+    cos = sin = None
+    if rope:
+        ct, st = oracle.rope_tables(max(sq, sk), d)
+        cos, sin = torch.from_numpy(ct).to(gpu), torch.from_numpy(st).to(gpu)
+    want = [ra._quantize_gpu(q, False, cos, sin), ra._quantize_gpu(k, False, cos, sin),
+            ra._quantize_gpu(v, not v_per_token)]
+    got = [(torch.full_like(x, 77), torch.full_like(s, float("nan"))) for x, s in want]
+    for _ in range(2):
+        rc = ra._lib_handle().rdna_quantize_int8_qkv(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), 0 if dtype == torch.float16 else 1, *q.stride()[:3],
+            *k.stride()[:3], *v.stride()[:3], b, hq, hkv, sq, sk, d, int(not v_per_token),
+            cos.data_ptr() if rope else None, sin.data_ptr() if rope else None, got[0][0].data_ptr(),
+            got[1][0].data_ptr(), got[2][0].data_ptr(), got[0][1].data_ptr(), got[1][1].data_ptr(),
+            got[2][1].data_ptr(), torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, ra.last_error()
+    torch.cuda.synchronize()
+    for (qi, s), (wi, ws) in zip(got, want):
+        assert torch.equal(qi, wi) and torch.equal(s, ws)
