@@ -46,10 +46,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_rotate_rows(const _Float16*
         for (int s = (int)blockIdx.x * kRopeRows + r0; s < row_end; s += rpp) {
             h8 x = *reinterpret_cast<const h8*>(sp + (int64_t)s * ss);
             x = rope8(x, cos_t + (int64_t)s * half, sin_t + (int64_t)s * half, 4 * ch);
-            // cached: the attention kernel reads the copy next (stored
-            // non-temporally, a causal S = 1237 GQA call took 30.8 us, not 29.3;
-            // copies larger than the caches, 64 and 128 MB, made no difference)
-            *reinterpret_cast<h8*>(dp + (int64_t)s * D) = x;
+            __builtin_nontemporal_store(x, reinterpret_cast<h8*>(dp + (int64_t)s * D));
         }
     }
 }
