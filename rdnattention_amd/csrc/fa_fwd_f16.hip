@@ -863,8 +863,8 @@ static int prefill_group(const AttnArgs& a) {
     return ratio % 4 == 0 ? 4 : (ratio % 2 == 0 ? 2 : 1);
 }
 
-int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double split_tile_us, int launches,
-                   size_t max_partials) {
+int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double alternate_us, double split_tile_us,
+                   int launches, size_t max_partials) {
     // Too few workgroups for the CUs and many key tiles for each: split the
     // keys, by the least modelled time.  A workgroup takes about 5 us beside
     // its key tiles; the partials are written and read at about 2.5 MB/us, and
@@ -896,7 +896,8 @@ int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double split_
             break;
         }
         const double rounds = (double)((n_wg * s + 255) / 256);
-        const double t = s == 1 ? 5.0 + (double)tiles * tile_us
+        const double t = s == 1 ? 5.0 + (alternate_us > 0.0 && n_wg <= 128 ? (double)((tiles + 1) / 2) * alternate_us
+                                                                           : (double)tiles * tile_us)
                                 : rounds * (5.0 * launches + (double)((tiles + s - 1) / s) * split_tile_us) +
                                       5.0 * launches + 2.0 * (double)partials / 2.5e6;
         if (s == 1 || t < best) {
@@ -914,7 +915,8 @@ static int f16_prefill_splits(const AttnArgs& a, size_t max_partials) {
         return 1;
     }
     const double tile_us = 0.4 + (a.D > 128 ? a.D / 256.0 : a.D / 128.0);
-    return prefill_splits(a, a.D > 128 ? kKPairRows : 32 * kPPWaves, tile_us, tile_us, 1, max_partials);
+    return prefill_splits(a, a.D > 128 ? kKPairRows : 32 * kPPWaves, tile_us, a.D > 128 ? 0.0 : 1.4 * tile_us, tile_us,
+                          1, max_partials);
 }
 
 // Steps of the longest sequence of row tiles that a workgroup of a persistent
@@ -949,7 +951,7 @@ static double longest_walk(const AttnArgs& a, int rows, int tiles_per_step, doub
     return longest;
 }
 
-bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us) {
+bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us, int chunk) {
     // Twice as many row tiles of half as many steps, where the longest row
     // tile of a launch sets its time: up to two row tiles per CU.  A row tile
     // takes about 5 us beside its steps.
@@ -958,7 +960,6 @@ bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us) {
     if (a.Sk <= 2 * kBN || (int64_t)((a.Sq + rows - 1) / rows) * head_groups > 512) {
         return false;
     }
-    const int chunk = xcd_head_group_chunk(head_groups, 4 * (int64_t)a.Sk * a.D);
     return step_us * longest_walk(a, rows / 2, 2, 5.0 / step_us, chunk) <
            0.97 * tile_us * longest_walk(a, rows, 1, 5.0 / tile_us, chunk);
 }
@@ -969,9 +970,9 @@ bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us) {
 // S1024 D128 29.0 / 20.6, D64 22.5 / 15.8; B1 S2048 D128 55 / 45; B2 S1024 D128
 // 31.8 / 30.5; and where the rule keeps whole row tiles: B1 S2048 D128 not
 // causal 71 / 79, B2 S1500 49 / 58, B2 S2048 78 / 92.
-static bool f16_prefill_alternate(const AttnArgs& a) {
+static bool f16_prefill_alternate(const AttnArgs& a, int chunk) {
     const double tile_us = 0.4 + a.D / 128.0;
-    return a.D <= 128 && prefill_alternate(a, tile_us, 1.4 * tile_us);
+    return a.D <= 128 && prefill_alternate(a, tile_us, 1.4 * tile_us, chunk);
 }
 
 int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err, ScratchRegion* region) {
@@ -1004,15 +1005,15 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
     // or 4 pairs of waves of 32 rows (D > 128)
     p.G = prefill_group(a);
     p.rows_per_wg = (kpair ? kKPairRows : dpair ? kDPairRows : 32 * kPPWaves) / p.G;
+    p.groups_per_kv = p.ratio / p.G;
+    p.n_head_groups = a.B * a.Hkv * p.groups_per_kv;
+    p.hg_chunk = xcd_head_group_chunk(p.n_head_groups, 2 * (int64_t)a.Sk * a.D * (int64_t)sizeof(_Float16));
     p.splits = f16_prefill_splits(a, region != nullptr ? region->bytes - region->used : SIZE_MAX);
-    p.alternate = p.splits == 1 && f16_prefill_alternate(a);
+    p.alternate = p.splits == 1 && f16_prefill_alternate(a, p.hg_chunk);
     if (p.alternate) {
         p.rows_per_wg /= 2;
     }
     p.n_row_tiles = (a.Sq + p.rows_per_wg - 1) / p.rows_per_wg;
-    p.groups_per_kv = p.ratio / p.G;
-    p.n_head_groups = a.B * a.Hkv * p.groups_per_kv;
-    p.hg_chunk = xcd_head_group_chunk(p.n_head_groups, 2 * (int64_t)a.Sk * a.D * (int64_t)sizeof(_Float16));
     p.c = softmax_log2_scale(a.scale);
     p.q_sign = a.scale < 0.0f ? -1.0f : 1.0f;
     p.qmul = p.q_sign * p.c;

@@ -131,7 +131,8 @@ __device__ __forceinline__ i32x4_t uniform_rsrc(i32x4_t r) {
 // MODE: see Int8Mode.
 template <int D, bool KSV, bool SCORES, Int8Mode MODE>
 __device__ __forceinline__ void int8_body(Int8Params p) {
-    constexpr bool SPLIT = MODE != Int8Mode::kWhole;
+    constexpr bool SPLIT = MODE == Int8Mode::kSplit || MODE == Int8Mode::kRowMax;
+    constexpr bool ALT = MODE == Int8Mode::kAlternate;
     constexpr bool ROWMAX = MODE == Int8Mode::kRowMax;
     using C = I8Cfg<D>;
     // [slot][K, V][TILE]; DMA destinations, so the base is 1 KB aligned
@@ -146,6 +147,10 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
     const int l32 = lane & 31;
     const int g = lane >> 5;
     const int grp = wave >> 2;
+    const int rw = ALT ? wave & 3 : wave; // wave by its rows
+    const int ugrp = ALT ? __builtin_amdgcn_readfirstlane(grp) : 0;
+    // kAlternate: every row's running maximum, and group B's (m, l)
+    __shared__ float sm_max[ALT ? 128 : 1];
     const uint32_t kv_lds = (uint32_t)reinterpret_cast<uintptr_t>(sKV);
     const uint32_t ks_lds = (uint32_t)reinterpret_cast<uintptr_t>(sks);
 
@@ -195,9 +200,9 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
         const int rem = hg - b * per_b;
         const int kvh = rem / p.groups_per_kv;
         const int sub = rem - kvh * p.groups_per_kv;
-        const int h = kvh * p.ratio + sub * p.G + (wave % p.G);
+        const int h = kvh * p.ratio + sub * p.G + (rw % p.G);
         const int wg_q0 = rt * p.rows_per_wg;
-        const int q0 = wg_q0 + (wave / p.G) * 32;
+        const int q0 = wg_q0 + (rw / p.G) * 32;
         const int q = q0 + l32;
         const bool wave_active = q0 < p.Sq;
         const int q_hi = min(q0 + 31, p.Sq - 1);
@@ -232,6 +237,9 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
         if constexpr (SPLIT) {
             split_key_tiles(p.splits, split, t_begin, n);
         }
+        // key tile i of this wave's sequence of ng tiles
+        const int ng = ALT ? (n + 1 - ugrp) / 2 : n;
+        auto tile_at = [&](int i) { return ALT ? t_begin + 2 * i + ugrp : t_begin + i; };
         int row_lo, row_hi;
         row_key_bounds(p.mask, q, row_lo, row_hi);
 
@@ -282,8 +290,8 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
         // ---- DMA of tile x (K, V and the per-token K scales) into slot x % 4,
         // issued by group A's waves
         auto issue = [&](int x) {
-            const int key0 = (t_begin + x) * kI8BN;
-            const uint32_t slot = (uint32_t)(x & (kI8Slots - 1));
+            const int key0 = ALT ? tile_at(x) * kI8BN : (t_begin + x) * kI8BN;
+            const uint32_t slot = (uint32_t)((ALT ? 2 * x + ugrp : x) & (kI8Slots - 1));
             const i32x4_t rk = uniform_rsrc(make_rsrc_v(kbase + (int64_t)key0 * p.k_ss,
                                                         tile_bytes<kI8BN>(Sk - key0, (uint32_t)p.k_ss, D)));
             const i32x4_t rv = uniform_rsrc(make_rsrc_v(vbase + (int64_t)key0 * p.v_ss,
@@ -298,7 +306,7 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
             for (int jj = 0; jj < C::BPW; jj++) {
                 dma_load16(rv, dv[jj], mk + C::TILE + 1024 * jj);
             }
-            if (KSV && wave == 0) {
+            if (KSV && (ALT ? rw : wave) == 0) {
                 // the tile's 64 K scales, one dword per lane (keys past Sk read 0)
                 const int left = Sk - key0;
                 const i32x4_t rs =
@@ -365,9 +373,11 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
             constexpr int T = NSK + NPV;
             constexpr int DEPTH = T < kI8OpDepth ? T : kI8OpDepth;
             constexpr int GPS = NPV > 0 ? 8 / NPV : 0; // dequant groups per P V MFMA
-            const int8_t* sk = sKV + (i & (kI8Slots - 1)) * (2 * C::TILE);
-            const int8_t* sv = sKV + ((i - 1) & (kI8Slots - 1)) * (2 * C::TILE) + C::TILE;
-            const float* ksl = sks + (i & (kI8Slots - 1)) * kI8BN;
+            const int kslot = (ALT ? 2 * i + ugrp : i) & (kI8Slots - 1);
+            const int vslot = (ALT ? 2 * i - 2 + ugrp : i - 1) & (kI8Slots - 1);
+            const int8_t* sk = sKV + kslot * (2 * C::TILE);
+            const int8_t* sv = sKV + vslot * (2 * C::TILE) + C::TILE;
+            const float* ksl = sks + kslot * kI8BN;
             auto q_op = [&](int st) -> i4 { return *reinterpret_cast<const i4*>(sQu + kofs[st]); };
             auto op = [&](int j) -> i4 {
                 if (j < NSK) {
@@ -462,8 +472,8 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
             }
             const bool do_pv = !SCORES && !ROWMAX && i >= 1 && cls_prev != 0;
             int cls_now = 0;
-            if (i < n) {
-                const int kt0 = (t_begin + i) * kI8BN;
+            if (i < ng) {
+                const int kt0 = ALT ? tile_at(i) * kI8BN : (t_begin + i) * kI8BN;
                 cls_now = classify_tile(p.mask, q0, q_hi, kt0, kt0 + kI8BN - 1);
             }
             using T_ = std::true_type;
@@ -508,7 +518,7 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
                 }
             }
             if (cls_prev == 2) {
-                const int kt0 = (t_begin + i) * kI8BN + 4 * g;
+                const int kt0 = (ALT ? tile_at(i) : t_begin + i) * kI8BN + 4 * g;
                 const int a = row_lo - kt0;
                 const int bnd = row_hi - kt0;
 #pragma unroll
@@ -529,7 +539,13 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
                 }
             }
             mx = pair_max(mx) * qeff; // qeff > 0: -inf stays -inf
-            const float m_new = fmaxf(m_c, mx);
+            float m_new = fmaxf(m_c, mx);
+            if constexpr (ALT) { // the other group's tile just before this one
+                m_new = fmaxf(m_new, sm_max[rw * 32 + l32]);
+                if (g == 0) {
+                    sm_max[rw * 32 + l32] = m_new;
+                }
+            }
             if constexpr (ROWMAX) {
                 m_c = m_new;
                 return;
@@ -566,7 +582,17 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
             l_c += psum;
         };
 
-        if (grp == 0 && n > 0) {
+        if constexpr (ALT) {
+            if (n > 0) {
+                if (ng > 0) {
+                    issue(0);
+                }
+                __builtin_amdgcn_s_waitcnt(waitcnt_vm(0)); // Q and the group's first tile landed
+            }
+            if (grp == 0 && g == 0) {
+                sm_max[rw * 32 + l32] = -INFINITY;
+            }
+        } else if (grp == 0 && n > 0) {
             issue(0);
             if (n > 1) {
                 issue(1);
@@ -581,7 +607,33 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
         // by A then B).  Its DMAs are issued at the start of phase 2x - 4 into
         // the slot tile x - 4 left at the end of phase 2x - 5, and group A waits
         // for them at the end of phase 2x - 1.  Both groups pass 2n + 3 barriers.
-        if (n > 0) {
+        //
+        // kAlternate: each group issues its own next tile at the start of its
+        // V(i) and waits for it at the end; the slot's last tile, the group's
+        // i - 1, was read in its M(i) the last time.
+        if constexpr (ALT) {
+            const int n2 = (n + 1) / 2; // steps of group A
+            if (n > 0) {
+                if (ugrp == 1) {
+                    __syncthreads();
+                }
+                for (int i = 0; i < n2; i++) {
+                    phase_m(i);
+                    __syncthreads();
+                    if (i + 1 < ng) {
+                        issue(i + 1);
+                    }
+                    phase_v(i);
+                    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+                    __syncthreads();
+                }
+                phase_m(n2);
+                __syncthreads();
+                if (ugrp == 0) {
+                    __syncthreads();
+                }
+            }
+        } else if (n > 0) {
             if (grp == 0) {
                 for (int i = 0; i < n; i++) {
                     if (i + 2 < n) {
@@ -609,7 +661,7 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
             }
         }
 
-        if (SCORES || !wave_active) {
+        if (SCORES || (!ALT && !wave_active)) {
             return;
         }
         if constexpr (ROWMAX) {
@@ -628,7 +680,52 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
                 of[dt][e] = fmaf(of[dt][e], bf, (float)oint[dt][e]);
             }
         }
-        const float l = pair_sum(l_c);
+        float l = pair_sum(l_c);
+        if constexpr (ALT) {
+            // group B's O (relative to its own maximum) into group A's, through
+            // LDS that nothing else reads after the last barrier
+            static_assert(4 * 32 * D * 4 <= sizeof(sKV) && 4 * 32 * 8 <= sizeof(sks), "O and (m, l) fit");
+            float* const so = reinterpret_cast<float*>(sKV) + (rw * 32 + l32) * D;
+            float2* const sml = reinterpret_cast<float2*>(sks) + rw * 32 + l32;
+            // column d0 at 16-byte chunk (d0 / 4) ^ (row % 16): conflict-free
+            auto at = [&](int dt, int qq) { return so + 4 * ((8 * dt + 2 * qq + g) ^ (l32 & 15)); };
+            if (ugrp == 1 && wave_active) {
+#pragma unroll
+                for (int dt = 0; dt < C::NDT; dt++) {
+#pragma unroll
+                    for (int qq = 0; qq < 4; qq++) {
+                        *reinterpret_cast<f4*>(at(dt, qq)) =
+                            f4{of[dt][4 * qq], of[dt][4 * qq + 1], of[dt][4 * qq + 2], of[dt][4 * qq + 3]};
+                    }
+                }
+                if (g == 0) {
+                    *sml = float2{m_c, l};
+                }
+            }
+            __syncthreads();
+            if (ugrp == 0 && wave_active) {
+                const float2 other = *sml;
+                const float m = fmaxf(l > 0.0f ? m_c : -INFINITY, other.y > 0.0f ? other.x : -INFINITY);
+                const float wa = l > 0.0f ? fast_exp2(m_c - m) : 0.0f;
+                const float wb = other.y > 0.0f ? fast_exp2(other.x - m) : 0.0f;
+                l = l * wa + other.y * wb;
+#pragma unroll
+                for (int dt = 0; dt < C::NDT; dt++) {
+#pragma unroll
+                    for (int qq = 0; qq < 4; qq++) {
+                        const f4 x = *reinterpret_cast<const f4*>(at(dt, qq));
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            of[dt][4 * qq + e] = of[dt][4 * qq + e] * wa + x[e] * wb;
+                        }
+                    }
+                }
+            }
+            __syncthreads(); // before the next row tile's DMAs
+            if (ugrp == 1 || !wave_active) {
+                return;
+            }
+        }
         if constexpr (SPLIT) {
             const float* vch = p.vch != nullptr ? p.vch + ((int64_t)b * p.Hkv + kvh) * D : nullptr;
             if (q < p.Sq) {
@@ -647,7 +744,7 @@ __device__ __forceinline__ void int8_body(Int8Params p) {
             [&](int d0) {
                 return vch != nullptr ? f * *reinterpret_cast<const f4*>(vch + d0) : f4{f, f, f, f};
             },
-            sO + wave * 32 * C::LDO, obase, q0, p.Sq, p.o_ss, lane);
+            sO + rw * 32 * C::LDO, obase, q0, p.Sq, p.o_ss, lane);
     };
     for (int item = 0;; item++) {
         const int wg = persistent_item(blockIdx.x, gridDim.x, item, p.n_items);
@@ -678,6 +775,8 @@ int launch_int8(const Int8Params& p, Int8Mode mode, int64_t n_wg, hipStream_t st
             kernel = &fa_fwd_int8_split<D, KSV, Int8Mode::kRowMax>;
         } else if (mode == Int8Mode::kSplit) {
             kernel = &fa_fwd_int8_split<D, KSV, Int8Mode::kSplit>;
+        } else if (mode == Int8Mode::kAlternate) {
+            kernel = &fa_fwd_int8_split<D, KSV, Int8Mode::kAlternate>;
         }
     }
     const int64_t resident = resident_workgroups(reinterpret_cast<const void*>(kernel), kI8Threads, err);
@@ -768,7 +867,8 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
     // launch that finds the row maxima).  Measured, us a call: B1 Hq32 Hkv8
     // Sq256 Sk8192 D128 242 unsplit, 86 split; B2 Hq16 Hkv8 Sq100 Sk16000 D64
     // 382 and 69
-    p.splits = prefill_splits(a, 32 * kI8Waves, a.D == 64 ? 1.5 : 1.9, a.D == 64 ? 2.2 : 2.8, 2, SIZE_MAX);
+    const double tile_us = a.D == 64 ? 1.5 : 1.9;
+    p.splits = prefill_splits(a, 32 * kI8Waves, tile_us, 1.3 * tile_us, 1.5 * tile_us, 2, SIZE_MAX);
     n_wg *= p.splits;
     p.n_items = (int32_t)n_wg;
     SplitRows out{};
@@ -787,7 +887,20 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
         return launch_int8_f16pv(p, a.D, false, mode, n_wg, stream, err);
     };
     if (p.splits == 1) {
-        return launch(Int8Mode::kWhole);
+        // few row tiles: alternating key tiles, a step of two tiles for 128 rows
+        // taking about 1.3 times one of a tile for 256.  Measured, us a call,
+        // whole against alternating (Hq 32 Hkv 8): B1 S1024 causal D64 31.5 /
+        // 21.5, D128 37.0 / 25.8; B1 S2048 causal D64 56 / 40, D128 67 / 51; B2
+        // S512 D128 22.3 / 17.4; and where the rule keeps whole row tiles: B1
+        // S2048 D128 not causal 69 / 83, B2 S2048 causal 79 / 98
+        if (!prefill_alternate(a, tile_us, 1.3 * tile_us, p.hg_chunk)) {
+            return launch(Int8Mode::kWhole);
+        }
+        p.rows_per_wg /= 2;
+        p.n_row_tiles = (a.Sq + p.rows_per_wg - 1) / p.rows_per_wg;
+        n_wg = (int64_t)p.n_row_tiles * p.n_head_groups;
+        p.n_items = (int32_t)n_wg;
+        return launch(Int8Mode::kAlternate);
     }
     StreamScratch maxima(ScratchUse::Int8Scores);
     if (maxima.alloc((size_t)p.splits * p.n_rows * sizeof(float), stream, err) != 0) {

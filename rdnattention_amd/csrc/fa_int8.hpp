@@ -69,8 +69,12 @@ struct Int8Params {
 // keys, so the keys of a row tile are split in two launches: kRowMax finds
 // every row's largest score in each split (no softmax, no P V), and kSplit
 // starts each split's running maximum at the largest of the earlier ones and
-// writes partials for the combine kernel.
-enum class Int8Mode { kWhole, kRowMax, kSplit };
+// writes partials for the combine kernel.  kAlternate, for launches of few row
+// tiles: both wave groups hold the same 128 rows and take the key tiles in turn
+// (PPMode::kAlternate of the FP16 kernel), handing the running maximum to each
+// other through LDS from softmax phase to softmax phase, which follow the key
+// order; so P is quantised as without it.
+enum class Int8Mode { kWhole, kRowMax, kSplit, kAlternate };
 
 // The running maximum that split `split` of a row starts from.
 __device__ __forceinline__ float earlier_max(const Int8Params& p, int split, int64_t row) {

@@ -125,15 +125,16 @@ SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_b
 
 // Key splits of a prefill call whose workgroups hold wg_rows rows (of G heads)
 // and take tile_us per 64-key tile (split_tile_us over `launches` launches where
-// the keys are split), with at most max_partials bytes of partials; 1 where
-// splitting does not pay.
-int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double split_tile_us, int launches,
-                   size_t max_partials);
+// the keys are split; alternate_us per two tiles of half the rows where the
+// kernel can alternate them, else 0), with at most max_partials bytes of
+// partials; 1 where splitting does not pay.
+int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double alternate_us, double split_tile_us,
+                   int launches, size_t max_partials);
 
 // Whether a prefill launch of the ping-pong kernels (256 rows of G heads per
-// workgroup, tile_us per 64-key tile) ends sooner with 128 rows and two tiles
-// per step of step_us.
-bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us);
+// workgroup, tile_us per 64-key tile, hg_chunk = chunk) ends sooner with 128
+// rows and two tiles per step of step_us.
+bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us, int chunk);
 
 // Before and after a launch of `splits` key splits: `r` from the arguments, with
 // the partials taken from `ws`; and the combine launch.  0, or -1 with `err`.

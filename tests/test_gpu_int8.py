@@ -446,8 +446,21 @@ SPLIT_CASES = [(1, 8, 2, 70, 3000, d, True, -1, sc) for d in (64, 128)
 ]
 
 
-@pytest.mark.parametrize("case", DECODE_CASES + SPLIT_CASES,
-                         ids=["b{}h{}kv{}q{}k{}d{}c{:d}w{}{}".format(*c) for c in DECODE_CASES + SPLIT_CASES])
+# few row tiles, whose two wave groups take the key tiles in turn and hand each
+# other the running maximum: odd and even tile counts, ragged ends, a group
+# without tiles in some row tiles, a window, rows without keys
+ALTERNATE_CASES = [(1, 8, 2, s, s, d, c, -1, sc) for d in (64, 128)
+                   for s, c, sc in ((321, True, "token"), (640, False, "channel"), (705, True, "vtoken"),
+                                    (300, True, "tensor"))] + [
+    (2, 4, 4, 500, 500, 128, True, 200, "token"),
+    (1, 4, 2, 600, 600, 64, False, 300, "token"),
+    (1, 4, 2, 700, 400, 64, True, -1, "channel"),
+]
+
+
+@pytest.mark.parametrize("case", DECODE_CASES + SPLIT_CASES + ALTERNATE_CASES,
+                         ids=["b{}h{}kv{}q{}k{}d{}c{:d}w{}{}".format(*c)
+                              for c in DECODE_CASES + SPLIT_CASES + ALTERNATE_CASES])
 def test_int8_split_keys_vs_emulation(gpu, oracle_lib, case):
     """The kernel-exact emulation, with the running maximum over all keys in
     order, whatever the splits: the INT8 bar on N(0, 1) rows, whose P a split's
