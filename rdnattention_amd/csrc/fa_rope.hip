@@ -21,9 +21,21 @@ namespace {
 // chunks of one column (D / 8 threads per row), row after row, with no
 // division per chunk.  A flat index with three 64-bit divisions per chunk ran
 // at 5.8 TB/s.
+//
+// Copies of up to 12 MiB run with heads fastest (HEADS_FAST: blocks x and y
+// swapped, the row blocks of neighbouring heads staggered): head h is then
+// rotated on XCD h % 8, where the attention kernel works on it when each head is
+// a head group.  Us a call, rows fastest / heads fastest: 2.5 MB (causal GQA
+// Hkv 8 S 1237 D 128) 31.0 / 28.8, 1.2 MB 22.6 / 21.6, 8.2 MB (Hkv 8 B 4 S 1000)
+// 30.7 / 30.0, 12.3 MB 38.6 / 38.2; but 16.8 MB 156.4 / 156.9, 33.5 MB 539.7 /
+// 542.9 and 134 MB 1100 / 1116 (heads a power of two of bytes apart).  Cached
+// instead of non-temporal stores gained as much on the first and lost 2-4 % on
+// others.
 constexpr int kRopeThreads = 256;
 constexpr int kRopeRows = 64;
+constexpr int64_t kRopeHeadsFastBytes = int64_t(12) << 20;
 
+template <bool HEADS_FAST>
 __global__ __launch_bounds__(kRopeThreads) void rope_rotate_rows(const _Float16* __restrict__ src,
                                                                  _Float16* __restrict__ dst,
                                                                  const float* __restrict__ cos_t,
@@ -38,12 +50,13 @@ __global__ __launch_bounds__(kRopeThreads) void rope_rotate_rows(const _Float16*
         return; // D / 8 does not divide the block (D = 96, 160, ...)
     }
     const int half = D / 2;
-    const int row_end = min(S, (int)(blockIdx.x + 1) * kRopeRows);
-    for (int64_t bh = blockIdx.y; bh < heads; bh += gridDim.y) {
+    const int rb = (int)(HEADS_FAST ? (blockIdx.y + blockIdx.x) % gridDim.y : blockIdx.x);
+    const int row_end = min(S, (rb + 1) * kRopeRows);
+    for (int64_t bh = HEADS_FAST ? blockIdx.x : blockIdx.y; bh < heads; bh += HEADS_FAST ? gridDim.x : gridDim.y) {
         const int64_t b = bh / H, h = bh - (bh / H) * H;
         const _Float16* sp = src + b * sb + h * sh + 8 * ch;
         _Float16* dp = dst + bh * S * D + 8 * ch;
-        for (int s = (int)blockIdx.x * kRopeRows + r0; s < row_end; s += rpp) {
+        for (int s = rb * kRopeRows + r0; s < row_end; s += rpp) {
             h8 x = *reinterpret_cast<const h8*>(sp + (int64_t)s * ss);
             x = rope8(x, cos_t + (int64_t)s * half, sin_t + (int64_t)s * half, 4 * ch);
             __builtin_nontemporal_store(x, reinterpret_cast<h8*>(dp + (int64_t)s * D));
@@ -60,9 +73,11 @@ int rope_rotate_k(const AttnArgs& a, void* dst, hipStream_t stream, std::string&
     }
     const uint32_t row_blocks = (uint32_t)((a.Sk + kRopeRows - 1) / kRopeRows);
     const uint32_t head_blocks = (uint32_t)(heads < 65535 ? heads : 65535);
-    hipLaunchKernelGGL(rope_rotate_rows, dim3(row_blocks, head_blocks), dim3(kRopeThreads), 0, stream,
-                       static_cast<const _Float16*>(a.k), static_cast<_Float16*>(dst), a.rot_cos, a.rot_sin,
-                       a.ks[0], a.ks[1], a.ks[2], a.Hkv, a.Sk, a.D, heads);
+    const bool heads_fast = heads * a.Sk * a.D * (int64_t)sizeof(_Float16) <= kRopeHeadsFastBytes && row_blocks < 65536;
+    auto* const kernel = heads_fast ? &rope_rotate_rows<true> : &rope_rotate_rows<false>;
+    hipLaunchKernelGGL(kernel, heads_fast ? dim3(head_blocks, row_blocks) : dim3(row_blocks, head_blocks),
+                       dim3(kRopeThreads), 0, stream, static_cast<const _Float16*>(a.k), static_cast<_Float16*>(dst),
+                       a.rot_cos, a.rot_sin, a.ks[0], a.ks[1], a.ks[2], a.Hkv, a.Sk, a.D, heads);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         err = hipGetErrorString(e);
