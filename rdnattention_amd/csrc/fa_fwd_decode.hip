@@ -378,10 +378,11 @@ SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_b
     // of `resident` workgroups (one per CU at D = 128); a workgroup takes
     // about 2 us beside its keys and streams at most 40 KB/us (measured: 40
     // with 128 workgroups, 48 to 50 with 8 to 64, D = 128 to 256), all
-    // together 6.8 TB/s; merging takes about 2 us.  So a count just above a
-    // whole round (264 workgroups for 24 kv heads) is never taken, which
-    // rounding resident / n_bkv up did.  Measured, us a call, against the
-    // count chosen: n_bkv 128, Sk 32768: 420 (1), 317 (2, chosen), 349 (3);
+    // together 6.8 TB/s; the merge, a second launch, adds about 5 us.  So a
+    // count just above a whole round (264 workgroups for 24 kv heads) is never
+    // taken, which rounding resident / n_bkv up did.  Measured, us a call,
+    // against the count chosen: n_bkv 8, Sk 512: 10.8 (1, chosen), 13.9 (2);
+    // D = 64, 8, 768: 8.4 (1, chosen), 12.4 (3); n_bkv 128, Sk 32768: 420 (1), 317 (2, chosen), 349 (3);
     // 32, 4096: 23 (4), 19.2 (8, chosen), 25.7 (16); 8, 32768: 37 (16),
     // 29.7 (32, chosen), 33.7 (64); D = 64, 256, 2048: 27.6 (1, chosen), 33 (2).
     const int64_t rounds_of_keys = (keys + round - 1) / round;
@@ -395,7 +396,7 @@ SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_b
         const int64_t waves_of_wgs = (wgs + resident - 1) / resident;
         const double rate = std::min(40e3, 6.8e6 / (double)std::min(wgs, resident)); // bytes per us
         const double t = (double)waves_of_wgs * (2.0 + (double)(std::min(kps, keys) * key_bytes) / rate) +
-                         (s > 1 ? 2.0 : 0.0);
+                         (s > 1 ? 5.0 : 0.0);
         if (t < best) {
             best = t;
             plan.splits = (int)s;

@@ -873,7 +873,10 @@ int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double altern
     // the 33.5 MB launch); Sq64 Sk4096 92 / 27; B2 Sq256 Sk8192 183 / 85; B1
     // Hq16 Hkv4 Sq128 Sk2000 D64 37 / 19.  Whole prompts this small stay
     // unsplit (1 x 8 heads, S 512, D64: 13.9 / 18.3; S 1024 causal 22.8 /
-    // 23.2).  With more workgroups than CUs the persistent grid balances them.
+    // 23.2).  Above D = 128 the larger rows make it 7 us (D = 256, 128 kv heads
+    // with one row, Sk 512: 17.5 / 19.5).  With more workgroups than CUs the
+    // persistent grid balances them.
+    const double merge_us = a.D > 128 ? 7.0 : 5.0;
     const int G = prefill_group(a);
     const int rows = wg_rows / G;
     const int64_t row_tiles = (a.Sq + rows - 1) / rows;
@@ -899,7 +902,7 @@ int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double altern
         const double t = s == 1 ? 5.0 + (alternate_us > 0.0 && n_wg <= 128 ? (double)((tiles + 1) / 2) * alternate_us
                                                                            : (double)tiles * tile_us)
                                 : rounds * (5.0 * launches + (double)((tiles + s - 1) / s) * split_tile_us) +
-                                      5.0 * launches + 2.0 * (double)partials / 2.5e6;
+                                      merge_us * launches + 2.0 * (double)partials / 2.5e6;
         if (s == 1 || t < best) {
             best = t;
             best_s = (int)s;
@@ -1060,10 +1063,32 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
 bool splitk_supported(const AttnArgs& a);
 bool splitk_built(const AttnArgs& a);
 
-// Auto: few query rows per kv head against a long key sequence -> split-K
-// (HBM-bound, parallel over the key axis); everything else -> prefill tiles.
+// Auto: the decode kernel for few query rows per kv head, the prefill tiles
+// otherwise.  us a call, prefill / decode, each from an HBM-sized set of caches
+// unless marked [r], where one cache is read again and again:
+//   * up to Sk = 128 both are the launch (8.9 / 8.9); from there one decode
+//     workgroup per kv head, no merge, is quicker as long as they run at once
+//     (D = 128, 8 kv heads: 10.7 / 9.1 at 256, 13.4 / 9.7 at 400; D = 192, 256
+//     kv heads: 22.6 / 18.4 at 511), but not from 1024 of them on (D = 128, Sk
+//     256: 36 / 40)
+//   * above D = 192 the decode kernel has one wave per SIMD.  It streams HBM
+//     better (D = 256, 64 kv heads of Sk 8192: 102 / 91), and rows of eight
+//     query heads together are read once and not per head (128 kv heads of
+//     2048: 87 / 57).  A cache up to 64 MB is quicker through the prefill
+//     kernel (8 kv heads of 4096: 17.3 / 18.9), and up to the 256 MiB that the
+//     last-level cache holds it is when the cache is read again, since only
+//     its loads are kept there (128 kv heads of 2048: 47.7 / 51.9 [r], 54.8 /
+//     52.6 else)
 bool prefer_splitk(const AttnArgs& a) {
-    return splitk_built(a) && a.Sk >= 512;
+    if (!splitk_built(a)) {
+        return false;
+    }
+    const int64_t n_bkv = (int64_t)a.B * a.Hkv;
+    if (a.D > 192) {
+        const int64_t kv_bytes = n_bkv * a.Sk * a.D * (int64_t)(2 * sizeof(_Float16));
+        return a.Sk >= 512 && (a.Hq > 4 * a.Hkv || kv_bytes > (int64_t)256 << 20);
+    }
+    return a.Sk >= 512 || (a.Sk > 128 && n_bkv <= 256);
 }
 
 int64_t fwd_f16_scratch_bytes(const AttnArgs& a, F16Path path, std::string& err) {

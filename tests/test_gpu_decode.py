@@ -101,8 +101,8 @@ def test_splitk_unsupported_shape_is_rejected(gpu):
 
 # d, b, hq, hkv, sq, sk, causal, window: every head dim the automatic choice
 # sends to split-K, at the edges of its tiles (32 keys), rounds (32 keys per
-# wave) and columns (1 .. 32 rows per kv head); merged by the last workgroup
-# (few splits or rows), by the combine kernel (MQA with many), or not at all
+# wave) and columns (1 .. 32 rows per kv head), with one split and several, and
+# both sides of the lines where the choice goes to the prefill kernel
 AUTO_CASES = [(d, 1, 8, 2, 1, 513, False, -1) for d in range(32, 257, 32)] + [
     (256, 2, 4, 4, 1, 2049, False, -1),
     (256, 1, 32, 1, 1, 4100, False, -1),
@@ -113,14 +113,21 @@ AUTO_CASES = [(d, 1, 8, 2, 1, 513, False, -1) for d in range(32, 257, 32)] + [
     (96, 1, 8, 2, 2, 4000, False, 900),
     (128, 1, 32, 1, 1, 30000, False, -1),
     (128, 33, 8, 8, 1, 520, False, -1),
+    (128, 1, 8, 2, 1, 128, False, -1),  # below the decode kernel's shortest cache, and just above it
+    (128, 1, 8, 2, 1, 129, False, -1),
+    (64, 3, 4, 2, 4, 300, True, -1),
+    (192, 1, 16, 2, 4, 511, True, 200),
+    (32, 33, 8, 8, 1, 200, False, -1),  # 264 kv heads: prefill
+    (256, 1, 16, 2, 2, 700, True, -1),  # D > 192: eight query heads per kv head
+    (256, 1, 4, 2, 1, 700, False, -1),  # and two
+    (224, 64, 8, 8, 1, 512, False, -1),
 ]
 
 
 @pytest.mark.parametrize("case", AUTO_CASES, ids=["d{}b{}h{}kv{}q{}k{}c{:d}w{}".format(*c) for c in AUTO_CASES])
 def test_auto_decode_vs_oracle(gpu, oracle_lib, case):
-    """FP16 bar against the oracle; a second call (the arrival counters of the
-    first must have returned to zero), the no-allocation entry point's two
-    launches and a captured graph's give the same bits."""
+    """FP16 bar against the oracle; a second call, the no-allocation entry point
+    and a captured graph's replays give the same bits."""
     from tests.gpu_util import lib
 
     d, b, hq, hkv, sq, sk, causal, window = case
