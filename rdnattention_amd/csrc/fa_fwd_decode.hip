@@ -362,7 +362,7 @@ size_t splitk_partial_bytes(const AttnArgs& a, int splits) {
 SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
                            size_t max_partials, int64_t max_keys) {
     // The keys that some row sees, from a tile boundary on, are dealt to the
-    // splits in whole rounds of tiles (one tile per wave).
+    // splits in multiples of `round` keys.
     const MaskSpec mask{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
     int lo, hi;
     visible_key_range(mask, 0, a.Sq - 1, lo, hi);
@@ -414,7 +414,11 @@ int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::s
         if (resident <= 0) {
             return -1;
         }
-        plan = splitk_plan_for(a, kDecTile, C::WAVES * kDecTile, 2 * C::RB, resident, max_partials);
+        // Half rounds of the waves: whole ones leave the last split short (64
+        // kv heads, Sk 6244, D = 128: 3 x 1792 keys and 868, 39.9 us against
+        // 38.9 of 3 x 1664 and 1252; 128 of 2303: 30.4 / 29.7); single tiles
+        // measure the same as these.
+        plan = splitk_plan_for(a, kDecTile, C::WAVES / 2 * kDecTile, 2 * C::RB, resident, max_partials);
         return 0;
     });
 }
