@@ -265,7 +265,7 @@ def make_step(wl: Workload, dev, host=None):
 def int8_quantized_e2e(dev, steps: int = 10, warmup: int = 20):
     """flash_attn_int8qk_quantized on fp16 inputs of the INT8 workload's shape
     (B=2, Hq=32, Hkv=8, S=8192, D=128, causal), timed whole: this library's
-    path (three quantiser kernels + the INT8 kernel with the per-channel V
+    path (quantiser kernels + the INT8 kernel with the per-channel V
     rescale in its epilogue) against the reference wrapper's composition
     (rdnattention/__init__.py:303-357: torch quantisers, including the
     per-tensor Q/K pass it discards, the INT8 kernel, then a torch multiply of

@@ -30,10 +30,11 @@ RDNA_API int32_t rdna_attention_forward_path(
     int32_t path, void* hip_stream);
 
 /* Releases the device memory the library keeps for reuse: the scratch
- * buffers (RoPE-rotated K copies, split-K partials, quantiser partials) it
- * caches per (device, stream, use), grown to the largest call so far (at most
- * 256 MiB each, at most 1 GiB per device over all streams and uses), and the
- * free blocks of the devices' default memory pools.  A call never frees or
+ * buffers (RoPE-rotated K copies, split-K partials, quantiser partials, INT8
+ * decode scores) it caches per (device, stream, use), grown to the largest
+ * call so far (at most 256 MiB each, at most 1 GiB per device over all
+ * streams and uses), and the free blocks of the devices' default memory
+ * pools.  A call never frees or
  * allocates scratch on the host's time: a cached buffer large enough is
  * reused with no allocator call; growth and eviction are stream-ordered
  * (hipFreeAsync / hipMallocAsync).  This trim is the one synchronising path:
@@ -54,7 +55,7 @@ RDNA_API int32_t rdna_scratch_stats(int32_t device, uint64_t* cached_bytes, int6
  * hipMalloc).  No reference counterpart: the reference needs no scratch.
  * Same arguments, results and return codes as rdna_attention_forward(); the
  * scratch that path takes -- the RoPE-rotated K copy (B*Hkv*Sk*D fp16) and
- * the split-K decode partials -- comes from a static 64 MiB device array the
+ * the partials of split keys -- comes from a static 64 MiB device array the
  * library holds on each GPU it runs on, so the call makes no hipMalloc,
  * hipFree or pool allocation.  A call needing more than 64 MiB of scratch
  * returns -3 ("... bytes of scratch ...") before launching anything.  Every

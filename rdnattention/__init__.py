@@ -424,7 +424,7 @@ def attention_int8_forward_into(query, key, value, output, q_scale, k_scale, v_s
 def trim_scratch() -> None:
     """Returns the scratch memory the library keeps for reuse to the devices:
     the buffers cached per (device, stream, use) for RoPE-rotated K copies,
-    split-K partials and quantiser partials (each grown to the largest call so
+    split-K partials, quantiser partials and INT8 decode scores (each grown to the largest call so
     far; at most 1 GiB per device), and the free blocks of the devices'
     default memory pools; e.g. before handing memory to another allocator.
     Synchronises the devices.  An extension; the reference allocates nothing."""

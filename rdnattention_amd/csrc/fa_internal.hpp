@@ -117,8 +117,8 @@ struct SplitKPlan {
 };
 int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::string& err);
 
-// The same for any split-K kernel: `tile` keys per wave tile, `round` per
-// workgroup round of them, key_bytes of K and V per key, `resident` workgroups
+// The same for any split-K kernel: `tile` keys per wave tile, the splits
+// multiples of `round` keys, key_bytes of K and V per key, `resident` workgroups
 // on the device, at most max_keys keys per split.
 SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
                            size_t max_partials, int64_t max_keys = INT32_MAX);

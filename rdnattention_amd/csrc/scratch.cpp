@@ -1,5 +1,5 @@
 // Stream-ordered scratch memory for the attention calls (the RoPE-rotated K
-// copy, split-K partials, quantiser partials).
+// copy, split-K partials, quantiser partials, INT8 decode scores).
 //
 // The reference allocates nothing (src/c_api.hpp:3-6); its kernels need no
 // scratch.  Here a call that needs scratch takes the buffer cached for its
