@@ -24,6 +24,9 @@
 //     result is the same softmax; P stays <= 256, exact in fp16's range), so
 //     the O accumulator is rarely rescaled
 //   * RoPE: Q is rotated once when loaded, K once up front (fa_rope.hip)
+//   * calls too small for the chip split their keys over workgroups
+//     (prefill_splits) or let the two groups take the key tiles in turn
+//     (prefill_alternate)
 #include "fa_common.hpp"
 #include "fa_host.hpp"
 #include "fa_internal.hpp"
