@@ -3,8 +3,10 @@
 //
 // A split leaves, per query row, O unnormalised in fp32 and (m, l): its
 // reference maximum in log2 units and its row sum relative to it.  The merged
-// row is sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s with M the largest m_s
-// of the splits that saw a key (l_s > 0).
+// row is sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s with M the largest m_s.
+// A split without a visible key has l_s = 0 and an m_s that is -inf or another
+// split's.  A score that is NaN or +inf makes l_s and O_s NaN; as in the kernels
+// that see all keys of a row, so does it the row.
 #pragma once
 
 #include "fa_common.hpp"
@@ -12,6 +14,12 @@
 namespace rdna_amd {
 
 constexpr int kMaxSplits = 256; // weights of one row in the merge's LDS
+
+// 2^(m - mref) for m <= mref; 1 for equal infinities (the NaN of their
+// difference is dropped by the minimum).
+__device__ __forceinline__ float part_weight(float m, float mref) {
+    return fast_exp2(fminf(m - mref, 0.0f));
+}
 
 // The output rows of a launch and the partials of their splits.  Row
 // (b * Hq + h) * Sq + q of split s is partial s * n_rows + row.
@@ -101,19 +109,14 @@ __device__ __forceinline__ void finish_rows(f16x (&oacc)[D / 32], float m_run, f
     float mref = -INFINITY, lsum = 0.0f; // of column l32 over the waves
 #pragma unroll
     for (int w = 0; w < WAVES; w++) {
-        if (sm_ml[(w * 32 + l32) * 2 + 1] > 0.0f) {
-            mref = fmaxf(mref, sm_ml[(w * 32 + l32) * 2 + 0]);
-        }
+        mref = fmaxf(mref, sm_ml[(w * 32 + l32) * 2 + 0]);
     }
 #pragma unroll
     for (int w = 0; w < WAVES; w++) {
-        const float lw = sm_ml[(w * 32 + l32) * 2 + 1];
-        if (lw > 0.0f) {
-            lsum += lw * fast_exp2(sm_ml[(w * 32 + l32) * 2 + 0] - mref);
-        }
+        lsum += sm_ml[(w * 32 + l32) * 2 + 1] * part_weight(sm_ml[(w * 32 + l32) * 2 + 0], mref);
     }
     const bool whole = r.splits == 1;
-    float scale_w = (l_tot > 0.0f) ? fast_exp2(m_run - mref) : 0.0f;
+    float scale_w = part_weight(m_run, mref);
     if (whole) {
         scale_w *= lsum > 0.0f ? 1.0f / lsum : 0.0f;
     }
@@ -220,7 +223,7 @@ __device__ __forceinline__ void merge_splits(const SplitParts& p, float* lds, St
             m[i] = v.x;
             l[i] = v.y;
         }
-        mx = l[i] > 0.0f ? fmaxf(mx, m[i]) : mx;
+        mx = fmaxf(mx, m[i]);
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -229,18 +232,20 @@ __device__ __forceinline__ void merge_splits(const SplitParts& p, float* lds, St
     float sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < PER; i++) {
-        m[i] = l[i] > 0.0f ? fast_exp2(m[i] - mx) : 0.0f;
+        m[i] = part_weight(m[i], mx);
         sum += l[i] * m[i];
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         sum += __shfl_xor(sum, off);
     }
+    // NaN: 0, as a row sum that is not positive gives in the prefill kernels; O
+    // is NaN where the row is
     const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
 #pragma unroll
     for (int i = 0; i < PER; i++) {
         if (tid < 64 && lane + 64 * i < p.splits) {
-            wgt[lane + 64 * i] = m[i] * inv;
+            wgt[lane + 64 * i] = l[i] != 0.0f ? m[i] * inv : -1.0f;
         }
     }
     __syncthreads();
@@ -249,8 +254,8 @@ __device__ __forceinline__ void merge_splits(const SplitParts& p, float* lds, St
     const int sg = tid / E;
     const int e = tid - sg * E;
     f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    // a split without a visible key (weight 0) adds nothing
-    auto add = [&](f4 x, float w) { acc += w > 0.0f ? x * w : f4{0.0f, 0.0f, 0.0f, 0.0f}; };
+    // a split without a visible key (weight -1) adds nothing
+    auto add = [&](f4 x, float w) { acc += w < 0.0f ? f4{0.0f, 0.0f, 0.0f, 0.0f} : x * w; };
     if (sg < SG) {
         const float* o = p.part_o + 4 * e;
         int s = sg;

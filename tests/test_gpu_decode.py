@@ -188,3 +188,54 @@ def test_split_prefill_vs_oracle(gpu, oracle_lib, case):
     torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1])
     assert_f16_parity(outs[0].float().cpu().numpy(), ref, "split prefill")
+
+
+# d, b, hq, hkv, sq, sk: split prefill (both kernels), decode with several splits
+# and with one, alternating groups
+NONFINITE_CASES = [(64, 1, 8, 2, 70, 3000), (128, 1, 8, 2, 70, 3000), (256, 1, 8, 2, 70, 3000),
+                   (128, 1, 8, 2, 4, 8192), (96, 1, 8, 2, 1, 4000), (256, 1, 32, 2, 1, 5000),
+                   (128, 32, 8, 8, 1, 512), (64, 1, 8, 8, 512, 512), (128, 1, 8, 8, 512, 512)]
+NONFINITE = ["q_nan", "k_nan", "k_inf", "k_neg_inf", "k_lowest", "v_inf"]
+
+
+@pytest.mark.parametrize("what", NONFINITE)
+@pytest.mark.parametrize("case", NONFINITE_CASES, ids=["d{}b{}h{}kv{}q{}k{}".format(*c) for c in NONFINITE_CASES])
+def test_nonfinite_through_the_merges(gpu, case, what):
+    """NaN, infinities and lowest scores as torch's float32 softmax treats them: a
+    query row of NaN is NaN and leaves the other rows alone; a key whose score is
+    NaN or +inf makes every row NaN that sees it, also where its split's partial
+    is one of many; keys at -inf (here all of the first splits') or at the lowest
+    scores (all of the last splits') weigh nothing; an infinite V reaches the
+    output.  (The lowest scores come last: a running maximum that starts at
+    -1e5 leaves the scores of the tile that ends it 2^-7 apart.)"""
+    d, b, hq, hkv, sq, sk = case
+    log(f"[non-finite] {case} {what}")
+    g = torch.Generator(device=gpu).manual_seed(61)
+    q = torch.randn(b, hq, sq, d, generator=g, device=gpu).abs().half() * 0.3  # positive: the sign of a score is K's
+    k = torch.randn(b, hkv, sk, d, generator=g, device=gpu).half() * 0.3
+    v = torch.randn(b, hkv, sk, d, generator=g, device=gpu).half()
+    if what == "q_nan":
+        q[:, :, sq // 2] = float("nan")
+    elif what == "k_nan":
+        k[:, :, 100] = float("nan")
+    elif what == "k_inf":
+        k[:, :, 100] = float("inf")
+    elif what == "k_neg_inf":
+        k[:, :, : sk // 2] = float("-inf")
+    elif what == "k_lowest":
+        k[:, :, sk // 2:] = -65504.0
+    else:
+        v[:, :, 100] = float("inf")
+    out = torch.full_like(q, 7.0)
+    assert forward_raw(q, k, v, out) == 0
+    torch.cuda.synchronize()
+    kr = k.float().repeat_interleave(hq // hkv, dim=1).transpose(2, 3).contiguous()
+    vr = v.float().repeat_interleave(hq // hkv, dim=1)
+    ref = torch.softmax(torch.matmul(q.float(), kr) * d ** -0.5, dim=-1)
+    ref = torch.matmul(ref, vr)
+    got = out.float()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(torch.isposinf(got), torch.isposinf(ref))
+    finite = torch.isfinite(ref)
+    if finite.any():
+        assert_f16_parity(got[finite].cpu().numpy(), ref[finite].cpu().numpy(), what)
