@@ -173,6 +173,21 @@ RDNA_API int32_t rdna_quantize_int8_qkv(
     const void* rot_sin, void* q_out, void* k_out, void* v_out, void* q_scale_out, void* k_scale_out,
     void* v_scale_out, void* hip_stream);
 
+/* The kernels that a call of these sizes takes, for tests and measurements:
+ * rdna_attention_forward (int8 == 0) or rdna_attention_forward_int8qk and its
+ * variants (int8 != 0).  *form: 0 whole row tiles, 1 row tiles with their keys
+ * split over workgroups, 2 the wave groups of a workgroup taking the key tiles
+ * in turn, 3 split-K decode; *splits the key splits (0 where decode's cannot be
+ * planned without a device), *scratch_bytes the bytes of their partials and,
+ * for INT8, of the scores or row maxima.  max_partials limits the partials of
+ * an FP16 call, as the rest of the no-allocation array does (UINT64_MAX: no
+ * limit).  Launches nothing.  Returns 0, -3 (arguments) or -4 (built without
+ * INT8).  No reference counterpart. */
+RDNA_API int32_t rdna_attention_call_plan(
+    int32_t int8, uint32_t batch_size, uint32_t num_heads, uint32_t num_kv_heads,
+    uint32_t seq_len, uint32_t key_seq_len, uint32_t head_dim, int32_t causal, int32_t window_size,
+    uint64_t max_partials, int32_t* form, int32_t* splits, uint64_t* scratch_bytes);
+
 /* Kernel timer.  While enabled, each launch of a main attention kernel
  * (prefill, split-K, int8; not the RoPE pre-rotation or split-K combine
  * kernels) is bracketed by a HIP event pair recorded on its stream.

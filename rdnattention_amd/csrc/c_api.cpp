@@ -18,6 +18,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -484,6 +486,61 @@ RDNA_API int32_t rdna_quantize_int8_qkv(const void* q, const void* k, const void
     }
     set_error("Quantize (int8) failed: %s", err);
     return -3;
+}
+
+RDNA_API int32_t rdna_attention_call_plan(int32_t int8, uint32_t batch_size, uint32_t num_heads,
+                                          uint32_t num_kv_heads, uint32_t seq_len, uint32_t key_seq_len,
+                                          uint32_t head_dim, int32_t causal, int32_t window_size,
+                                          uint64_t max_partials, int32_t* form, int32_t* splits,
+                                          uint64_t* scratch_bytes) {
+    std::string err;
+    AttnArgs a;
+    alignas(16) char nothing[16]; // stands for the tensors, whose pointers are not looked at
+    a.q = a.k = a.v = nothing;
+    a.o = nothing;
+    if (form == nullptr || splits == nullptr || scratch_bytes == nullptr) {
+        err = "null output pointer";
+    } else if (int8 != 0 ? head_dim != 64 && head_dim != 128 : !head_dim_f16_ok(head_dim)) {
+        err = "unsupported head_dim";
+    } else {
+        err = check_common(a, batch_size, num_heads, num_kv_heads, seq_len, key_seq_len, 16);
+    }
+#if defined(RDNATTENTION_NO_INT8)
+    if (err.empty() && int8 != 0) {
+        set_error("Attention (int8qk) unavailable: %s", kNoInt8);
+        return -4;
+    }
+#endif
+    if (!err.empty()) {
+        set_error("Attention call plan failed: %s", err);
+        return -3;
+    }
+    a.B = (int32_t)batch_size;
+    a.Hq = (int32_t)num_heads;
+    a.Hkv = (int32_t)num_kv_heads;
+    a.Sq = (int32_t)seq_len;
+    a.Sk = (int32_t)key_seq_len;
+    a.D = (int32_t)head_dim;
+    a.causal = causal != 0 ? 1 : 0;
+    a.window = window_size > 0 ? window_size : 0;
+    rdna_amd::CallPlan plan;
+    int rc = -1;
+#if !defined(RDNATTENTION_NO_INT8)
+    if (int8 != 0) {
+        rc = rdna_amd::int8_call_plan(a, plan, err);
+    } else
+#endif
+    {
+        rc = rdna_amd::f16_call_plan(a, (size_t)std::min<uint64_t>(max_partials, SIZE_MAX), plan, err);
+    }
+    if (rc != 0 && plan.splits != 0) { // 0: decode, whose splits a device decides
+        set_error("Attention call plan failed: %s", err);
+        return -3;
+    }
+    *form = (int32_t)plan.form;
+    *splits = plan.splits;
+    *scratch_bytes = plan.scratch;
+    return 0;
 }
 
 RDNA_API int32_t rdna_int8_qk_scores(const void* q, const void* k, int32_t* scores, int64_t q_stride_b,

@@ -352,7 +352,7 @@ bool splitk_supported(const AttnArgs& a) {
 }
 
 bool splitk_built(const AttnArgs& a) {
-    return a.D <= 256 && (int64_t)(a.Hq / a.Hkv) * a.Sq <= 32;
+    return a.D <= 256 && (int64_t)(a.Hq / a.Hkv) * a.Sq <= 32 && (int64_t)a.B * a.Hkv <= kMaxGridY;
 }
 
 size_t splitk_partial_bytes(const AttnArgs& a, int splits) {

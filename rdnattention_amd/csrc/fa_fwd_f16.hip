@@ -981,6 +981,23 @@ static bool f16_prefill_alternate(const AttnArgs& a, int chunk) {
     return a.D <= 128 && prefill_alternate(a, tile_us, 1.4 * tile_us, chunk);
 }
 
+static int f16_hg_chunk(const AttnArgs& a) {
+    return xcd_head_group_chunk(a.B * (a.Hq / prefill_group(a)),
+                                2 * (int64_t)a.Sk * a.D * (int64_t)sizeof(_Float16));
+}
+
+static CallPlan f16_prefill_plan(const AttnArgs& a, size_t max_partials) {
+    CallPlan plan;
+    plan.splits = f16_prefill_splits(a, max_partials);
+    if (plan.splits > 1) {
+        plan.form = CallForm::kSplit;
+        plan.scratch = splitk_partial_bytes(a, plan.splits);
+    } else if (f16_prefill_alternate(a, f16_hg_chunk(a))) {
+        plan.form = CallForm::kAlternate;
+    }
+    return plan;
+}
+
 int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err, ScratchRegion* region) {
     PrefillParams p{};
     p.q = static_cast<const _Float16*>(a.q);
@@ -1013,9 +1030,10 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
     p.rows_per_wg = (kpair ? kKPairRows : dpair ? kDPairRows : 32 * kPPWaves) / p.G;
     p.groups_per_kv = p.ratio / p.G;
     p.n_head_groups = a.B * a.Hkv * p.groups_per_kv;
-    p.hg_chunk = xcd_head_group_chunk(p.n_head_groups, 2 * (int64_t)a.Sk * a.D * (int64_t)sizeof(_Float16));
-    p.splits = f16_prefill_splits(a, region != nullptr ? region->bytes - region->used : SIZE_MAX);
-    p.alternate = p.splits == 1 && f16_prefill_alternate(a, p.hg_chunk);
+    p.hg_chunk = f16_hg_chunk(a);
+    const CallPlan plan = f16_prefill_plan(a, region != nullptr ? region->bytes - region->used : SIZE_MAX);
+    p.splits = plan.splits;
+    p.alternate = plan.form == CallForm::kAlternate;
     if (p.alternate) {
         p.rows_per_wg /= 2;
     }
@@ -1092,6 +1110,21 @@ bool prefer_splitk(const AttnArgs& a) {
         return a.Sk >= 512 && (a.Hq > 4 * a.Hkv || kv_bytes > (int64_t)256 << 20);
     }
     return a.Sk >= 512 || (a.Sk > 128 && n_bkv <= 256);
+}
+
+int f16_call_plan(const AttnArgs& a, size_t max_partials, CallPlan& plan, std::string& err) {
+    if (!prefer_splitk(a)) {
+        plan = f16_prefill_plan(a, max_partials);
+        return 0;
+    }
+    plan = CallPlan{CallForm::kDecode, 0, 0};
+    SplitKPlan splits;
+    if (splitk_plan(a, max_partials, splits, err) != 0) {
+        return -1;
+    }
+    plan.splits = splits.splits;
+    plan.scratch = splitk_partial_bytes(a, splits.splits);
+    return 0;
 }
 
 int64_t fwd_f16_scratch_bytes(const AttnArgs& a, F16Path path, std::string& err) {

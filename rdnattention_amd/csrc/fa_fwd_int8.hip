@@ -796,6 +796,12 @@ int launch_int8(const Int8Params& p, Int8Mode mode, int64_t n_wg, hipStream_t st
 
 } // namespace
 
+// Query heads per workgroup of the prefill kernels.
+static int int8_group(const AttnArgs& a) {
+    const int ratio = a.Hq / a.Hkv;
+    return (ratio % 4 == 0) ? 4 : ((ratio % 2 == 0) ? 2 : 1);
+}
+
 int64_t int8_params(const AttnArgs& a, Int8Params& p, std::string& err) {
     if (a.ks[2] < 0 || a.vs[2] < 0 || a.ks[2] > (1 << 24) || a.vs[2] > (1 << 24)) {
         err = "key/value seq strides must be in [0, 2^24] elements";
@@ -830,7 +836,7 @@ int64_t int8_params(const AttnArgs& a, Int8Params& p, std::string& err) {
     p.Sq = a.Sq;
     p.Hkv = a.Hkv;
     p.ratio = a.Hq / a.Hkv;
-    p.G = (p.ratio % 4 == 0) ? 4 : ((p.ratio % 2 == 0) ? 2 : 1);
+    p.G = int8_group(a);
     p.rows_per_wg = 32 * kI8Waves / p.G;
     p.n_row_tiles = (a.Sq + p.rows_per_wg - 1) / p.rows_per_wg;
     p.groups_per_kv = p.ratio / p.G;
@@ -846,29 +852,63 @@ int64_t int8_params(const AttnArgs& a, Int8Params& p, std::string& err) {
     return n_wg;
 }
 
-int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
-    Int8Params p;
-    int64_t n_wg = int8_params(a, p, err);
-    if (n_wg < 0) {
-        return -1;
-    }
-    // few query rows per kv head (one MFMA column block): split-K, at every key
-    // count; the prefill kernels put 256 rows in a workgroup (B8 Hq32 Hkv8
-    // Sq1 Sk8192 D128: 43 us a call against 205)
-    if ((a.D == 64 || a.D == 128) && int8_splitk_supported(a)) {
-        return fwd_int8_splitk(a, p, stream, err);
-    }
-    if (a.D != 64 && a.D != 128) {
-        err = "unsupported head_dim (only 64 and 128 are compiled in for the int8 kernel)";
-        return -1;
-    }
+static int64_t int8_row_max_bytes(const AttnArgs& a, int splits) {
+    return (int64_t)splits * a.B * a.Hq * a.Sq * (int64_t)sizeof(float);
+}
+
+static CallPlan int8_prefill_plan(const AttnArgs& a, int hg_chunk) {
     // too few workgroups for the CUs: split the keys (a 64-key tile takes
     // about 1.5 us at D = 64, 1.9 us at D = 128, and half as much again in the
     // launch that finds the row maxima).  Measured, us a call: B1 Hq32 Hkv8
     // Sq256 Sk8192 D128 242 unsplit, 86 split; B2 Hq16 Hkv8 Sq100 Sk16000 D64
     // 382 and 69
     const double tile_us = a.D == 64 ? 1.5 : 1.9;
-    p.splits = prefill_splits(a, 32 * kI8Waves, tile_us, 1.3 * tile_us, 1.5 * tile_us, 2, SIZE_MAX);
+    CallPlan plan;
+    plan.splits = prefill_splits(a, 32 * kI8Waves, tile_us, 1.3 * tile_us, 1.5 * tile_us, 2, SIZE_MAX);
+    if (plan.splits > 1) {
+        plan.form = CallForm::kSplit;
+        plan.scratch = splitk_partial_bytes(a, plan.splits) + int8_row_max_bytes(a, plan.splits);
+        return plan;
+    }
+    // few row tiles: alternating key tiles, a step of two tiles for 128 rows
+    // taking about 1.3 times one of a tile for 256.  Measured, us a call, whole
+    // against alternating (Hq 32 Hkv 8): B1 S1024 causal D64 31.5 / 21.5, D128
+    // 37.0 / 25.8; B1 S2048 causal D64 56 / 40, D128 67 / 51; B2 S512 D128 22.3
+    // / 17.4; and where the rule keeps whole row tiles: B1 S2048 D128 not causal
+    // 69 / 83, B2 S2048 causal 79 / 98
+    if (prefill_alternate(a, tile_us, 1.3 * tile_us, hg_chunk)) {
+        plan.form = CallForm::kAlternate;
+    }
+    return plan;
+}
+
+int int8_call_plan(const AttnArgs& a, CallPlan& plan, std::string& err) {
+    if (int8_splitk_supported(a)) {
+        return int8_decode_plan(a, plan, err);
+    }
+    const int64_t head_groups = (int64_t)a.B * (a.Hq / int8_group(a));
+    plan = int8_prefill_plan(a, xcd_head_group_chunk((int)head_groups, 2 * (int64_t)a.Sk * a.D));
+    return 0;
+}
+
+int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
+    Int8Params p;
+    int64_t n_wg = int8_params(a, p, err);
+    if (n_wg < 0) {
+        return -1;
+    }
+    if (a.D != 64 && a.D != 128) {
+        err = "unsupported head_dim (only 64 and 128 are compiled in for the int8 kernel)";
+        return -1;
+    }
+    // few query rows per kv head (one MFMA column block): split-K, at every key
+    // count; the prefill kernels put 256 rows in a workgroup (B8 Hq32 Hkv8
+    // Sq1 Sk8192 D128: 43 us a call against 205)
+    if (int8_splitk_supported(a)) {
+        return fwd_int8_splitk(a, p, stream, err);
+    }
+    const CallPlan plan = int8_prefill_plan(a, p.hg_chunk);
+    p.splits = plan.splits;
     n_wg *= p.splits;
     p.n_items = (int32_t)n_wg;
     SplitRows out{};
@@ -887,13 +927,7 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
         return launch_int8_f16pv(p, a.D, false, mode, n_wg, stream, err);
     };
     if (p.splits == 1) {
-        // few row tiles: alternating key tiles, a step of two tiles for 128 rows
-        // taking about 1.3 times one of a tile for 256.  Measured, us a call,
-        // whole against alternating (Hq 32 Hkv 8): B1 S1024 causal D64 31.5 /
-        // 21.5, D128 37.0 / 25.8; B1 S2048 causal D64 56 / 40, D128 67 / 51; B2
-        // S512 D128 22.3 / 17.4; and where the rule keeps whole row tiles: B1
-        // S2048 D128 not causal 69 / 83, B2 S2048 causal 79 / 98
-        if (!prefill_alternate(a, tile_us, 1.3 * tile_us, p.hg_chunk)) {
+        if (plan.form != CallForm::kAlternate) {
             return launch(Int8Mode::kWhole);
         }
         p.rows_per_wg /= 2;
@@ -903,7 +937,7 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
         return launch(Int8Mode::kAlternate);
     }
     StreamScratch maxima(ScratchUse::Int8Scores);
-    if (maxima.alloc((size_t)p.splits * p.n_rows * sizeof(float), stream, err) != 0) {
+    if (maxima.alloc((size_t)int8_row_max_bytes(a, p.splits), stream, err) != 0) {
         return -1;
     }
     p.row_max = static_cast<float*>(maxima.ptr);

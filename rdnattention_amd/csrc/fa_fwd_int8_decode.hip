@@ -457,24 +457,47 @@ __global__ __launch_bounds__(kI8DecThreads, TC == 4 && !(VTOK && D == 128) ? 4 :
     });
 }
 
+// Columns in the scratch (TC) of a call with up to 32 rows per kv head.
+int scratch_columns(const AttnArgs& a) {
+    return (int64_t)(a.Hq / a.Hkv) * a.Sq <= 4 ? 4 : 32;
+}
+
+// 64-key blocks from key0 on that the splits of a plan cover.
+int64_t plan_blocks(const SplitKPlan& plan) {
+    return ((int64_t)plan.splits * plan.keys_per_split + kI8BN - 1) / kI8BN;
+}
+
+// Scores and block maxima of a call.
+int64_t score_bytes(const AttnArgs& a, const SplitKPlan& plan) {
+    return (int64_t)a.B * a.Hkv * plan_blocks(plan) * (kI8BN + 1) * scratch_columns(a) * (int64_t)sizeof(float);
+}
+
 template <int D, bool VTOK, int TC>
-int launch_int8_decode(const AttnArgs& a, const Int8Params& ip, hipStream_t stream, std::string& err) {
+int int8_decode_splits(const AttnArgs& a, SplitKPlan& plan, std::string& err) {
     const int64_t resident =
         resident_workgroups(reinterpret_cast<const void*>(&fa_int8_decode_pv<D, VTOK, TC>), kI8DecThreads, err);
     if (resident <= 0) {
         return -1;
     }
-    const SplitKPlan plan = splitk_plan_for(a, kI8BN, kI8DecWaves * kI8BN, 2 * D, resident, SIZE_MAX,
-                                            TCfg<TC>::MAX_TILES * kI8BN);
+    plan = splitk_plan_for(a, kI8BN, kI8DecWaves * kI8BN, 2 * D, resident, SIZE_MAX, TCfg<TC>::MAX_TILES * kI8BN);
+    return 0;
+}
+
+template <int D, bool VTOK, int TC>
+int launch_int8_decode(const AttnArgs& a, const Int8Params& ip, hipStream_t stream, std::string& err) {
+    SplitKPlan plan;
+    if (int8_decode_splits<D, VTOK, TC>(a, plan, err) != 0) {
+        return -1;
+    }
     Int8DecodeParams p{};
     p.a = ip;
     p.keys_per_split = plan.keys_per_split;
     p.key0 = plan.key0;
-    p.blocks = (int32_t)(((int64_t)plan.splits * plan.keys_per_split + kI8BN - 1) / kI8BN);
+    p.blocks = (int32_t)plan_blocks(plan);
     const size_t blocks = (size_t)a.B * a.Hkv * p.blocks;
     StreamScratch ws(ScratchUse::SplitKPartials), scores(ScratchUse::Int8Scores);
     if (splitk_begin(a, plan.splits, ws, stream, p.out, err) != 0 ||
-        scores.alloc(blocks * (kI8BN + 1) * TC * sizeof(float), stream, err) != 0) {
+        scores.alloc((size_t)score_bytes(a, plan), stream, err) != 0) {
         return -1;
     }
     p.t = static_cast<float*>(scores.ptr);
@@ -495,19 +518,37 @@ int launch_int8_decode(const AttnArgs& a, const Int8Params& ip, hipStream_t stre
 
 template <int D, bool VTOK>
 int launch_int8_decode_as(const AttnArgs& a, const Int8Params& p, hipStream_t stream, std::string& err) {
-    return p.ratio * a.Sq <= 4 ? launch_int8_decode<D, VTOK, 4>(a, p, stream, err)
-                               : launch_int8_decode<D, VTOK, 32>(a, p, stream, err);
+    return scratch_columns(a) == 4 ? launch_int8_decode<D, VTOK, 4>(a, p, stream, err)
+                                   : launch_int8_decode<D, VTOK, 32>(a, p, stream, err);
+}
+
+template <int D>
+int decode_splits_as(const AttnArgs& a, SplitKPlan& plan, std::string& err) {
+    return scratch_columns(a) == 4 ? int8_decode_splits<D, false, 4>(a, plan, err)
+                                   : int8_decode_splits<D, false, 32>(a, plan, err);
 }
 
 } // namespace
 
 bool int8_splitk_supported(const AttnArgs& a) {
-    // one block of MFMA columns, few enough keys for kMaxSplits splits, and at
-    // most 1 GiB of scores
+    // one block of MFMA columns, few enough keys for kMaxSplits splits, at most 1
+    // GiB of scores, a grid (y = kv heads) within HIP's limit
     const int64_t M = (int64_t)(a.Hq / a.Hkv) * a.Sq;
-    const int64_t tc = M <= 4 ? 4 : 32;
-    const int64_t max_keys = (int64_t)kMaxSplits * kI8BN * (M <= 4 ? TCfg<4>::MAX_TILES : TCfg<32>::MAX_TILES);
-    return M <= 32 && a.Sk <= max_keys && (int64_t)a.B * a.Hkv * a.Sk * tc * (int64_t)sizeof(float) <= (1 << 30);
+    const int64_t tc = scratch_columns(a);
+    const int64_t max_keys = (int64_t)kMaxSplits * kI8BN * (tc == 4 ? TCfg<4>::MAX_TILES : TCfg<32>::MAX_TILES);
+    return M <= 32 && (int64_t)a.B * a.Hkv <= kMaxGridY && a.Sk <= max_keys &&
+           (int64_t)a.B * a.Hkv * a.Sk * tc * (int64_t)sizeof(float) <= (1 << 30);
+}
+
+int int8_decode_plan(const AttnArgs& a, CallPlan& plan, std::string& err) {
+    plan = CallPlan{CallForm::kDecode, 0, 0};
+    SplitKPlan splits;
+    if ((a.D == 64 ? decode_splits_as<64>(a, splits, err) : decode_splits_as<128>(a, splits, err)) != 0) {
+        return -1;
+    }
+    plan.splits = splits.splits;
+    plan.scratch = splitk_partial_bytes(a, splits.splits) + (size_t)score_bytes(a, splits);
+    return 0;
 }
 
 int fwd_int8_splitk(const AttnArgs& a, const Int8Params& p, hipStream_t stream, std::string& err) {

@@ -99,5 +99,7 @@ int launch_int8_f16pv(const Int8Params& p, int head_dim, bool scores, Int8Mode m
 // or 128.
 bool int8_splitk_supported(const AttnArgs& a);
 int fwd_int8_splitk(const AttnArgs& a, const Int8Params& p, hipStream_t stream, std::string& err);
+struct CallPlan;
+int int8_decode_plan(const AttnArgs& a, CallPlan& plan, std::string& err);
 
 } // namespace rdna_amd

@@ -20,6 +20,9 @@ struct ScratchRegion {
     size_t used = 0;
 };
 
+// Largest y extent of a launch grid that HIP documents.
+constexpr int64_t kMaxGridY = 65535;
+
 // Bytes a buffer of `bytes` takes from a ScratchRegion (256-byte aligned).
 constexpr size_t region_bytes(size_t bytes) {
     return (bytes + 255) / 256 * 256;
@@ -135,6 +138,22 @@ int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double altern
 // workgroup, tile_us per 64-key tile, hg_chunk = chunk) ends sooner with 128
 // rows and two tiles per step of step_us.
 bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us, int chunk);
+
+// The kernels a call takes: prefill by whole row tiles, with split keys, with the
+// wave groups taking the key tiles in turn, or split-K decode; the key splits,
+// and the bytes of their scratch (partials, and of INT8 the scores or row maxima).
+enum class CallForm : int32_t { kWhole = 0, kSplit = 1, kAlternate = 2, kDecode = 3 };
+struct CallPlan {
+    CallForm form = CallForm::kWhole;
+    int splits = 1;
+    size_t scratch = 0;
+};
+
+// The plan of an FP16 call (with at most max_partials bytes of partials) or an
+// INT8 call.  0, or -1 with `err` (a decode form whose occupancy query failed;
+// plan.form is set).
+int f16_call_plan(const AttnArgs& a, size_t max_partials, CallPlan& plan, std::string& err);
+int int8_call_plan(const AttnArgs& a, CallPlan& plan, std::string& err);
 
 // Before and after a launch of `splits` key splits: `r` from the arguments, with
 // the partials taken from `ws`; and the combine launch.  0, or -1 with `err`.

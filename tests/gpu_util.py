@@ -52,6 +52,21 @@ def forward_raw(q, k, v, out, causal=False, window=-1, cos=None, sin=None, scale
     return rc
 
 
+WHOLE, SPLIT, ALTERNATE, DECODE = range(4)
+
+
+def call_plan(int8, b, hq, hkv, sq, sk, d, causal=False, window=-1, max_partials=2 ** 64 - 1):
+    """rdna_attention_call_plan: (form, splits, scratch bytes) of a call."""
+    form, splits, scratch = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_uint64()
+    fn = lib().rdna_attention_call_plan
+    fn.argtypes = ([ctypes.c_int32] + [ctypes.c_uint32] * 6 + [ctypes.c_int32] * 2 + [ctypes.c_uint64] +
+                   [ctypes.c_void_p] * 3)
+    rc = fn(int(int8), b, hq, hkv, sq, sk, d, int(causal), window, max_partials, ctypes.addressof(form),
+            ctypes.addressof(splits), ctypes.addressof(scratch))
+    assert rc == 0, lib().rdna_get_error()
+    return form.value, splits.value, scratch.value
+
+
 def seeded_inputs(seed, b, hq, hkv, sq, sk, d, std=1.0):
     """CPU torch.Generator(seed) -> fp32 -> fp16 (the inputs of the measured workloads)."""
     import torch

@@ -239,3 +239,31 @@ def test_nonfinite_through_the_merges(gpu, case, what):
     finite = torch.isfinite(ref)
     if finite.any():
         assert_f16_parity(got[finite].cpu().numpy(), ref[finite].cpu().numpy(), what)
+
+
+@pytest.mark.parametrize("int8,d,sk", [(False, 96, 512), (False, 64, 600), (True, 64, 24), (True, 128, 70)])
+def test_more_kv_heads_than_a_grid_dimension(gpu, int8, d, sk):
+    """65536 (batch, kv head) pairs, one above what HIP allows in y, on one K and V
+    (batch stride 0): every batch entry gives the bits of the first, which agrees
+    with a call for it alone (decode kernels)."""
+    import rdnattention as ra
+
+    b, h = 8192, 8
+    log(f"[kv heads] int8={int8} d{d} sk{sk}")
+    g = torch.Generator(device=gpu).manual_seed(71)
+    draw = (lambda *s: torch.randint(-127, 128, s, generator=g, device=gpu, dtype=torch.int8)) if int8 else (
+        lambda *s: torch.randn(*s, generator=g, device=gpu).half())
+    q, k, v = (draw(1, h, s, d) for s in (1, sk, sk))
+    outs = []
+    for n in (1, b):
+        qn, kn, vn = (t.expand(n, -1, -1, -1) for t in (q, k, v))
+        out = torch.full((n, h, 1, d), float("nan"), dtype=torch.float16, device=gpu)
+        if int8:
+            ra.attention_int8_forward_into(qn, kn, vn, out, 0.01, 0.01, 1 / 127)
+        else:
+            ra.attention_forward_into(qn, kn, vn, out)
+        outs.append(out)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[1], outs[1][:1].expand_as(outs[1]))
+    diff = (outs[1][0].float() - outs[0][0].float()).abs().max().item()
+    assert diff <= 2e-3, diff  # another order of the sums; the same INT8 P
