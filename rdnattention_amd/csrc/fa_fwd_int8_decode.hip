@@ -462,14 +462,17 @@ int scratch_columns(const AttnArgs& a) {
     return (int64_t)(a.Hq / a.Hkv) * a.Sq <= 4 ? 4 : 32;
 }
 
-// 64-key blocks from key0 on that the splits of a plan cover.
-int64_t plan_blocks(const SplitKPlan& plan) {
-    return ((int64_t)plan.splits * plan.keys_per_split + kI8BN - 1) / kI8BN;
+// 64-key blocks from the first to the last key that some row sees.
+int64_t visible_blocks(const AttnArgs& a) {
+    const MaskSpec mask{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
+    int lo, hi;
+    visible_key_range(mask, 0, a.Sq - 1, lo, hi);
+    return hi < lo ? 0 : hi / kI8BN + 1 - lo / kI8BN;
 }
 
 // Scores and block maxima of a call.
-int64_t score_bytes(const AttnArgs& a, const SplitKPlan& plan) {
-    return (int64_t)a.B * a.Hkv * plan_blocks(plan) * (kI8BN + 1) * scratch_columns(a) * (int64_t)sizeof(float);
+int64_t score_bytes(const AttnArgs& a) {
+    return (int64_t)a.B * a.Hkv * visible_blocks(a) * (kI8BN + 1) * scratch_columns(a) * (int64_t)sizeof(float);
 }
 
 template <int D, bool VTOK, int TC>
@@ -493,11 +496,11 @@ int launch_int8_decode(const AttnArgs& a, const Int8Params& ip, hipStream_t stre
     p.a = ip;
     p.keys_per_split = plan.keys_per_split;
     p.key0 = plan.key0;
-    p.blocks = (int32_t)plan_blocks(plan);
+    p.blocks = (int32_t)visible_blocks(a); // key0 begins the first of them
     const size_t blocks = (size_t)a.B * a.Hkv * p.blocks;
     StreamScratch ws(ScratchUse::SplitKPartials), scores(ScratchUse::Int8Scores);
     if (splitk_begin(a, plan.splits, ws, stream, p.out, err) != 0 ||
-        scores.alloc((size_t)score_bytes(a, plan), stream, err) != 0) {
+        scores.alloc((size_t)score_bytes(a), stream, err) != 0) {
         return -1;
     }
     p.t = static_cast<float*>(scores.ptr);
@@ -532,22 +535,22 @@ int decode_splits_as(const AttnArgs& a, SplitKPlan& plan, std::string& err) {
 
 bool int8_splitk_supported(const AttnArgs& a) {
     // one block of MFMA columns, few enough keys for kMaxSplits splits, at most 1
-    // GiB of scores, a grid (y = kv heads) within HIP's limit
+    // GiB of scores and block maxima, a grid (y = kv heads) within HIP's limit
     const int64_t M = (int64_t)(a.Hq / a.Hkv) * a.Sq;
-    const int64_t tc = scratch_columns(a);
-    const int64_t max_keys = (int64_t)kMaxSplits * kI8BN * (tc == 4 ? TCfg<4>::MAX_TILES : TCfg<32>::MAX_TILES);
-    return M <= 32 && (int64_t)a.B * a.Hkv <= kMaxGridY && a.Sk <= max_keys &&
-           (int64_t)a.B * a.Hkv * a.Sk * tc * (int64_t)sizeof(float) <= (1 << 30);
+    const int64_t max_blocks =
+        (int64_t)kMaxSplits * (scratch_columns(a) == 4 ? TCfg<4>::MAX_TILES : TCfg<32>::MAX_TILES);
+    return M <= 32 && (int64_t)a.B * a.Hkv <= kMaxGridY && visible_blocks(a) <= max_blocks &&
+           score_bytes(a) <= (int64_t)1 << 30;
 }
 
 int int8_decode_plan(const AttnArgs& a, CallPlan& plan, std::string& err) {
-    plan = CallPlan{CallForm::kDecode, 0, 0};
+    plan = CallPlan{CallForm::kDecode, 0, (size_t)score_bytes(a)};
     SplitKPlan splits;
     if ((a.D == 64 ? decode_splits_as<64>(a, splits, err) : decode_splits_as<128>(a, splits, err)) != 0) {
         return -1;
     }
     plan.splits = splits.splits;
-    plan.scratch = splitk_partial_bytes(a, splits.splits) + (size_t)score_bytes(a, splits);
+    plan.scratch += splitk_partial_bytes(a, splits.splits);
     return 0;
 }
 

@@ -13,3 +13,26 @@ def test_decode_grid_limit(int8, hkv, sk, d):
     for b in (65536 // hkv, 100000 // hkv):
         form, splits, scratch = call_plan(int8, b, 4 * hkv, hkv, 1, sk, d)
         assert form != DECODE and splits == 1 and scratch == 0
+
+
+# b, hkv, rows per kv head, sk, d, causal, window
+INT8_SCRATCH = [(4096, 8, 8, 64, 64, False, -1), (8191, 8, 32, 120, 128, False, -1), (512, 8, 1, 1, 64, False, -1),
+                (1024, 8, 4, 700, 128, True, -1), (64, 8, 16, 9001, 128, False, -1), (16, 8, 2, 4000, 64, True, 300),
+                (128, 8, 32, 8192, 64, False, -1), (8, 8, 1, 300000, 128, False, -1)]
+
+
+@pytest.mark.parametrize("case", INT8_SCRATCH, ids=["b{}kv{}m{}k{}d{}c{:d}w{}".format(*c) for c in INT8_SCRATCH])
+def test_int8_decode_scratch(case):
+    """Scores and block maxima are taken for the 64-key blocks that some row sees,
+    whatever the splits, and never above 1 GiB."""
+    b, hkv, m, sk, d, causal, window = case
+    ratio = m // 2 if causal else m
+    form, splits, scratch = call_plan(True, b, ratio * hkv, hkv, m // ratio, sk, d, causal, window)
+    if form != DECODE:
+        return
+    lo = max(0, sk - m // ratio - window + 1) if window > 0 else 0
+    blocks = (sk - 1) // 64 + 1 - lo // 64
+    scores = b * hkv * blocks * 65 * (4 if m <= 4 else 32) * 4
+    assert scores <= 1 << 30
+    partials = splits * b * hkv * m * (d + 2) * 4 if splits > 1 else 0  # with a device
+    assert scratch == scores + partials
