@@ -436,8 +436,8 @@ int splitk_begin(const AttnArgs& a, int splits, StreamScratch& ws, hipStream_t s
     r.splits = splits;
     // every partial is written by its split's workgroup before the combine
     // reads it, so the buffer needs no clearing
-    if (ws.alloc(splitk_partial_bytes(a, splits), stream, err) != 0) {
-        return -1;
+    if (const int rc = ws.alloc(splitk_partial_bytes(a, splits), stream, err)) {
+        return rc;
     }
     r.part_o = static_cast<float*>(ws.ptr);
     r.part_ml = splits > 1 ? r.part_o + (size_t)splits * r.n_rows * a.D : nullptr;
@@ -494,10 +494,14 @@ int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::stri
     if (splitk_plan(a, room, plan, err) != 0) {
         return -1;
     }
+    StreamScratch ws(ScratchUse::SplitKPartials, region);
+    int rc = splitk_begin(a, plan.splits, ws, stream, p.out, err);
+    if (rc == kScratchFull && splitk_plan(a, 0, plan, err) == 0) { // one split
+        rc = splitk_begin(a, plan.splits, ws, stream, p.out, err);
+    }
     p.keys_per_split = plan.keys_per_split;
     p.key0 = plan.key0;
-    StreamScratch ws(ScratchUse::SplitKPartials, region);
-    if (splitk_begin(a, plan.splits, ws, stream, p.out, err) != 0 ||
+    if (rc != 0 ||
         for_dim(a.D, [&](auto d) { return launch_decode<decltype(d)::value>(p, a.B * a.Hkv, stream, err); }) != 0) {
         return -1;
     }

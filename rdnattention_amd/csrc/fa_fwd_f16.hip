@@ -999,6 +999,17 @@ static CallPlan f16_prefill_plan(const AttnArgs& a, size_t max_partials) {
 }
 
 int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err, ScratchRegion* region) {
+    CallPlan plan = f16_prefill_plan(a, region != nullptr ? region->bytes - region->used : SIZE_MAX);
+    SplitRows out{};
+    StreamScratch ws(ScratchUse::SplitKPartials, region);
+    int rc = splitk_begin(a, plan.splits, ws, stream, out, err);
+    if (rc == kScratchFull) {
+        plan = f16_prefill_plan(a, 0); // keys not split
+        rc = splitk_begin(a, plan.splits, ws, stream, out, err);
+    }
+    if (rc != 0) {
+        return -1;
+    }
     PrefillParams p{};
     p.q = static_cast<const _Float16*>(a.q);
     p.k = static_cast<const _Float16*>(a.k);
@@ -1031,7 +1042,6 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
     p.groups_per_kv = p.ratio / p.G;
     p.n_head_groups = a.B * a.Hkv * p.groups_per_kv;
     p.hg_chunk = f16_hg_chunk(a);
-    const CallPlan plan = f16_prefill_plan(a, region != nullptr ? region->bytes - region->used : SIZE_MAX);
     p.splits = plan.splits;
     p.alternate = plan.form == CallForm::kAlternate;
     if (p.alternate) {
@@ -1054,15 +1064,10 @@ int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::str
         err = "launch grid too large";
         return -1;
     }
-    SplitRows out{};
-    StreamScratch ws(ScratchUse::SplitKPartials, region);
-    if (splitk_begin(a, p.splits, ws, stream, out, err) != 0) {
-        return -1;
-    }
     p.part_o = out.part_o;
     p.part_ml = out.part_ml;
     p.n_rows = out.n_rows;
-    int rc = -1;
+    rc = -1;
     switch (a.D) {
     case 32: rc = launch_pp<32>(p, n_wg, stream, err); break;
     case 64: rc = launch_pp<64>(p, n_wg, stream, err); break;

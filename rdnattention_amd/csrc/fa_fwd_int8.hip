@@ -856,7 +856,7 @@ static int64_t int8_row_max_bytes(const AttnArgs& a, int splits) {
     return (int64_t)splits * a.B * a.Hq * a.Sq * (int64_t)sizeof(float);
 }
 
-static CallPlan int8_prefill_plan(const AttnArgs& a, int hg_chunk) {
+static CallPlan int8_prefill_plan(const AttnArgs& a, int hg_chunk, size_t max_partials) {
     // too few workgroups for the CUs: split the keys (a 64-key tile takes
     // about 1.5 us at D = 64, 1.9 us at D = 128, and half as much again in the
     // launch that finds the row maxima).  Measured, us a call: B1 Hq32 Hkv8
@@ -864,7 +864,7 @@ static CallPlan int8_prefill_plan(const AttnArgs& a, int hg_chunk) {
     // 382 and 69
     const double tile_us = a.D == 64 ? 1.5 : 1.9;
     CallPlan plan;
-    plan.splits = prefill_splits(a, 32 * kI8Waves, tile_us, 1.3 * tile_us, 1.5 * tile_us, 2, SIZE_MAX);
+    plan.splits = prefill_splits(a, 32 * kI8Waves, tile_us, 1.3 * tile_us, 1.5 * tile_us, 2, max_partials);
     if (plan.splits > 1) {
         plan.form = CallForm::kSplit;
         plan.scratch = splitk_partial_bytes(a, plan.splits) + int8_row_max_bytes(a, plan.splits);
@@ -887,7 +887,7 @@ int int8_call_plan(const AttnArgs& a, CallPlan& plan, std::string& err) {
         return int8_decode_plan(a, plan, err);
     }
     const int64_t head_groups = (int64_t)a.B * (a.Hq / int8_group(a));
-    plan = int8_prefill_plan(a, xcd_head_group_chunk((int)head_groups, 2 * (int64_t)a.Sk * a.D));
+    plan = int8_prefill_plan(a, xcd_head_group_chunk((int)head_groups, 2 * (int64_t)a.Sk * a.D), SIZE_MAX);
     return 0;
 }
 
@@ -904,18 +904,33 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
     // few query rows per kv head (one MFMA column block): split-K, at every key
     // count; the prefill kernels put 256 rows in a workgroup (B8 Hq32 Hkv8
     // Sq1 Sk8192 D128: 43 us a call against 205)
+    // (without memory for the scratch: the prefill kernels, keys not split)
+    size_t max_partials = SIZE_MAX;
     if (int8_splitk_supported(a)) {
-        return fwd_int8_splitk(a, p, stream, err);
+        const int rc = fwd_int8_splitk(a, p, stream, err);
+        if (rc != kScratchFull) {
+            return rc;
+        }
+        max_partials = 0;
     }
-    const CallPlan plan = int8_prefill_plan(a, p.hg_chunk);
+    CallPlan plan = int8_prefill_plan(a, p.hg_chunk, max_partials);
+    SplitRows out{};
+    StreamScratch ws(ScratchUse::SplitKPartials), maxima(ScratchUse::Int8Scores);
+    int rc = splitk_begin(a, plan.splits, ws, stream, out, err);
+    if (rc == 0 && plan.splits > 1) {
+        rc = maxima.alloc((size_t)int8_row_max_bytes(a, plan.splits), stream, err);
+    }
+    if (rc == kScratchFull) {
+        plan = int8_prefill_plan(a, p.hg_chunk, 0);
+        rc = 0;
+    }
+    if (rc != 0) {
+        return -1;
+    }
+    p.row_max = static_cast<float*>(maxima.ptr);
     p.splits = plan.splits;
     n_wg *= p.splits;
     p.n_items = (int32_t)n_wg;
-    SplitRows out{};
-    StreamScratch ws(ScratchUse::SplitKPartials);
-    if (splitk_begin(a, p.splits, ws, stream, out, err) != 0) {
-        return -1;
-    }
     p.part_o = out.part_o;
     p.part_ml = out.part_ml;
     p.n_rows = out.n_rows;
@@ -936,11 +951,6 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
         p.n_items = (int32_t)n_wg;
         return launch(Int8Mode::kAlternate);
     }
-    StreamScratch maxima(ScratchUse::Int8Scores);
-    if (maxima.alloc((size_t)int8_row_max_bytes(a, p.splits), stream, err) != 0) {
-        return -1;
-    }
-    p.row_max = static_cast<float*>(maxima.ptr);
     if (launch(Int8Mode::kRowMax) != 0 || launch(Int8Mode::kSplit) != 0) {
         return -1;
     }

@@ -499,9 +499,12 @@ int launch_int8_decode(const AttnArgs& a, const Int8Params& ip, hipStream_t stre
     p.blocks = (int32_t)visible_blocks(a); // key0 begins the first of them
     const size_t blocks = (size_t)a.B * a.Hkv * p.blocks;
     StreamScratch ws(ScratchUse::SplitKPartials), scores(ScratchUse::Int8Scores);
-    if (splitk_begin(a, plan.splits, ws, stream, p.out, err) != 0 ||
-        scores.alloc((size_t)score_bytes(a), stream, err) != 0) {
-        return -1;
+    int rc = splitk_begin(a, plan.splits, ws, stream, p.out, err);
+    if (rc == 0) {
+        rc = scores.alloc((size_t)score_bytes(a), stream, err);
+    }
+    if (rc != 0) {
+        return rc;
     }
     p.t = static_cast<float*>(scores.ptr);
     p.bmax = p.t + blocks * TCfg<TC>::BLOCK_FLOATS;

@@ -44,6 +44,9 @@ enum class ScratchUse : int { RotatedK = 0, SplitKPartials = 1, QuantPartials = 
 // (hipMallocAsync / hipFreeAsync).  No path here waits on the host.
 // With a region: carved from it, nothing allocated or freed (the caller has
 // checked that it fits).
+// alloc: 0, or with `err` kScratchFull when the device has no memory left (a
+// call whose keys need not be split then runs without), else -1.
+constexpr int kScratchFull = -2;
 struct StreamScratch {
     void* ptr = nullptr;
     hipStream_t stream = nullptr;
@@ -156,7 +159,8 @@ int f16_call_plan(const AttnArgs& a, size_t max_partials, CallPlan& plan, std::s
 int int8_call_plan(const AttnArgs& a, CallPlan& plan, std::string& err);
 
 // Before and after a launch of `splits` key splits: `r` from the arguments, with
-// the partials taken from `ws`; and the combine launch.  0, or -1 with `err`.
+// the partials taken from `ws` (0, or what its alloc returns); and the combine
+// launch (0, or -1 with `err`).
 struct SplitRows;
 int splitk_begin(const AttnArgs& a, int splits, StreamScratch& ws, hipStream_t stream, SplitRows& r,
                  std::string& err);

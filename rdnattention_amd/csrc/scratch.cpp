@@ -59,6 +59,15 @@ std::string hip_err(const char* what, hipError_t e) {
     return std::string(what) + ": " + hipGetErrorString(e);
 }
 
+// A failed hipMallocAsync: `err` and what alloc returns.  The error does not
+// stay behind for the check after the next launch, which a caller that can do
+// with less makes.
+int alloc_failed(hipError_t e, std::string& err) {
+    (void)hipGetLastError();
+    err = hip_err("scratch allocation failed", e);
+    return e == hipErrorOutOfMemory ? kScratchFull : -1;
+}
+
 // Releases e's buffer in the order of stream s: after the work recorded in
 // its last_use event (a GPU-side wait), then hipFreeAsync on s.  Nothing here
 // waits on the host.
@@ -157,8 +166,7 @@ int StreamScratch::alloc(size_t bytes, hipStream_t s, std::string& err) {
                     }
                     if (e != hipSuccess) {
                         ent.ptr = nullptr;
-                        err = hip_err("scratch allocation failed", e);
-                        return -1;
+                        return alloc_failed(e, err);
                     }
                     ent.bytes = want;
                     dc.bytes += want;
@@ -196,8 +204,7 @@ int StreamScratch::alloc(size_t bytes, hipStream_t s, std::string& err) {
     }
     if (e != hipSuccess) {
         ptr = nullptr;
-        err = hip_err("scratch allocation failed", e);
-        return -1;
+        return alloc_failed(e, err);
     }
     pooled = true;
     return 0;

@@ -8,13 +8,15 @@ tests drive the C ABI on three streams with preallocated tensors, so that the
 only device allocations in the measured regions are the library's own, and
 read its counters through rdna_scratch_stats.
 """
+import contextlib
+import ctypes
 import time
 
 import pytest
 import torch
 
 import oracle
-from tests.gpu_util import forward_raw, log
+from tests.gpu_util import DECODE, SPLIT, call_plan, forward_raw, log
 
 pytestmark = pytest.mark.gpu
 
@@ -185,3 +187,81 @@ def test_cap_bounds_cached_bytes_over_streams(gpu):
         assert torch.equal(o.view(torch.int16), want.view(torch.int16))
     rdnattention.trim_scratch()
     assert _stats()["cached_bytes"] == 0
+
+
+class _MemLocation(ctypes.Structure):
+    _fields_ = [("type", ctypes.c_int), ("id", ctypes.c_int)]
+
+
+class _MemPoolProps(ctypes.Structure):  # hipMemPoolProps
+    _fields_ = [("allocType", ctypes.c_int), ("handleTypes", ctypes.c_int), ("location", _MemLocation),
+                ("win32SecurityAttributes", ctypes.c_void_p), ("maxSize", ctypes.c_size_t),
+                ("reserved", ctypes.c_ubyte * 56)]
+
+
+@contextlib.contextmanager
+def _small_pool(nbytes):
+    """Stream-ordered allocations of the current device from a pool of at most
+    `nbytes`, as on a device whose memory is taken."""
+    import rdnattention
+
+    hip = ctypes.CDLL("libamdhip64.so")
+    dev = torch.cuda.current_device()
+    props = _MemPoolProps(allocType=1, location=_MemLocation(1, dev), maxSize=nbytes)
+    pool, before = ctypes.c_void_p(), ctypes.c_void_p()
+    torch.cuda.synchronize()
+    rdnattention.trim_scratch()
+    assert hip.hipMemPoolCreate(ctypes.byref(pool), ctypes.byref(props)) == 0
+    assert hip.hipDeviceGetMemPool(ctypes.byref(before), dev) == 0
+    assert hip.hipDeviceSetMemPool(dev, pool) == 0
+    try:
+        yield
+    finally:
+        torch.cuda.synchronize()
+        rdnattention.trim_scratch()
+        assert hip.hipDeviceSetMemPool(dev, before) == 0
+        assert hip.hipMemPoolDestroy(pool) == 0
+
+
+# int8, b, hq, hkv, sq, sk, d: decode (partials, and scores for INT8) and prefill
+# with split keys, each with more scratch than 2 MiB
+NO_MEMORY_CASES = [(False, 1, 32, 8, 100, 6000, 128), (False, 1, 16, 8, 60, 6000, 256), (False, 8, 32, 2, 2, 9000, 96),
+                   (False, 8, 32, 2, 2, 9000, 128), (True, 8, 32, 8, 1, 4000, 128), (True, 2, 32, 8, 4, 4000, 64),
+                   (True, 1, 32, 8, 100, 6000, 64), (True, 1, 32, 8, 100, 6000, 128)]
+
+
+@pytest.mark.parametrize("case", NO_MEMORY_CASES, ids=["i{:d}b{}h{}kv{}q{}k{}d{}".format(*c) for c in NO_MEMORY_CASES])
+def test_calls_without_memory_for_scratch(gpu, case):
+    """Where the device has no memory left for the scratch of split keys, the call
+    runs without splitting them, to the same result within the bars of another
+    order of the sums (INT8: the same P), and leaves no error behind."""
+    import rdnattention as ra
+
+    int8, b, hq, hkv, sq, sk, d = case
+    log(f"[no memory] {case}")
+    form, _, scratch = call_plan(int8, b, hq, hkv, sq, sk, d)
+    assert form in (SPLIT, DECODE) and scratch > 2 << 20, (form, scratch)
+    g = torch.Generator(device=gpu).manual_seed(330)
+    if int8:
+        q, k, v = (torch.randint(-127, 128, (b, h, s, d), generator=g, device=gpu, dtype=torch.int8)
+                   for h, s in ((hq, sq), (hkv, sk), (hkv, sk)))
+    else:
+        q, k, v = (torch.randn(b, h, s, d, generator=g, device=gpu).half()
+                   for h, s in ((hq, sq), (hkv, sk), (hkv, sk)))
+
+    def run():
+        out = torch.full((b, hq, sq, d), float("nan"), dtype=torch.float16, device=gpu)
+        if int8:
+            ra.attention_int8_forward_into(q, k, v, out, 0.01, 0.01, 1 / 127)
+        else:
+            ra.attention_forward_into(q, k, v, out)
+        torch.cuda.synchronize()
+        return out
+
+    want = run()
+    with _small_pool(2 << 20):
+        got = run()
+        again = run()
+    assert torch.equal(got, again)
+    assert (got.float() - want.float()).abs().max().item() <= 2e-3
+    assert torch.equal(run(), want)
