@@ -883,7 +883,7 @@ static CallPlan int8_prefill_plan(const AttnArgs& a, int hg_chunk, size_t max_pa
 }
 
 int int8_call_plan(const AttnArgs& a, CallPlan& plan, std::string& err) {
-    if (int8_splitk_supported(a)) {
+    if (int8_prefer_splitk(a)) {
         return int8_decode_plan(a, plan, err);
     }
     const int64_t head_groups = (int64_t)a.B * (a.Hq / int8_group(a));
@@ -901,12 +901,12 @@ int fwd_int8(const AttnArgs& a, hipStream_t stream, std::string& err) {
         err = "unsupported head_dim (only 64 and 128 are compiled in for the int8 kernel)";
         return -1;
     }
-    // few query rows per kv head (one MFMA column block): split-K, at every key
-    // count; the prefill kernels put 256 rows in a workgroup (B8 Hq32 Hkv8
-    // Sq1 Sk8192 D128: 43 us a call against 205)
-    // (without memory for the scratch: the prefill kernels, keys not split)
+    // few query rows per kv head (one MFMA column block): split-K; the prefill
+    // kernels put 256 rows in a workgroup (B8 Hq32 Hkv8 Sq1 Sk8192 D128: 43 us a
+    // call against 205).  Without memory for the scratch: the prefill kernels,
+    // keys not split.
     size_t max_partials = SIZE_MAX;
-    if (int8_splitk_supported(a)) {
+    if (int8_prefer_splitk(a)) {
         const int rc = fwd_int8_splitk(a, p, stream, err);
         if (rc != kScratchFull) {
             return rc;

@@ -546,6 +546,59 @@ bool int8_splitk_supported(const AttnArgs& a) {
            score_bytes(a) <= (int64_t)1 << 30;
 }
 
+// The decode kernels or, where they are supported too, the prefill kernels (whose
+// workgroup holds all rows of up to four query heads of a kv head, and of up to
+// 512 workgroups may alternate).  Time prefill / decode, each over caches that
+// together exceed the last-level cache, by prefill workgroups:
+//   * up to 256 the two launches and the merge cost about 5 us (a cache of 64 keys
+//     9.2 / 12.9 us): even at about 576 keys at D = 64 (8 kv heads of 512 keys
+//     0.95 to 1.03, of 640 1.03 to 1.16), 448 at D = 128 (1.07 to 1.15)
+//   * beyond, prefill runs in rounds: up to 512 from 192 keys (512 kv heads with
+//     one row 1.15, of 128 keys 0.9 to 0.98), from 128 at D = 128 (384 heads 0.99 to
+//     1.04) or with several workgroups per kv head (1.0 to 1.25); above from 128
+//     (768 heads 1.09 to 1.14), and always with several workgroups per kv head
+//     (320 heads of eight rows, 1 key 1.08) or from 1024 workgroups on (4096 heads
+//     of one key 1.2)
+//   * rows of one workgroup that take the 32-column scratch, whose scores are
+//     more bytes than K: prefill that fills its rounds is quicker (256 kv heads
+//     with 8 to 32 rows, 512 to 8192 keys 0.82 to 1.03, 512 of them 0.84 to 0.98;
+//     but 128 1.0 to 1.8, and 320 and 384 from 256 keys 1.07 to 1.17 at D = 64), and
+//     more often so with 32 rows of one head, in one wave, at D = 128 (192 heads
+//     0.94 to 0.97, of 8192 keys 1.12, 384 0.92 to 1.0); and where its one round leaves CUs idle but
+//     the scores leave the last-level cache (192 heads of 16384 keys, 408 MB: 0.8;
+//     128 heads, 272 MB: 1.5).  Above 512 workgroups they do not alternate
+//     (1024 heads with 16 rows, 192 keys 1.07 at D = 64; at D = 128 4096 of 320 1.05,
+//     768, whole rounds, of 384 to 576 0.93 to 0.96; with 32 rows of one head 1.06
+//     from 256 and 1.1 from 1024)
+bool int8_prefer_splitk(const AttnArgs& a) {
+    if (!int8_splitk_supported(a)) {
+        return false;
+    }
+    const int ratio = a.Hq / a.Hkv;
+    const int groups = ratio % 4 == 0 ? ratio / 4 : ratio % 2 == 0 ? ratio / 2 : ratio; // per kv head
+    const bool one_wave = ratio == groups;
+    const int64_t n_wg = (int64_t)a.B * a.Hkv * groups;
+    const int64_t keys = visible_blocks(a) * kI8BN;
+    const bool d64 = a.D == 64;
+    const int64_t even = d64 ? 576 : 448;
+    if (groups > 1 || scratch_columns(a) == 4) {
+        if (n_wg > 512) {
+            return n_wg >= 1024 || groups > 1 || keys >= 128;
+        }
+        return keys >= (n_wg <= 256 ? even : groups > 1 || !d64 ? 128 : 192);
+    }
+    const int64_t rounds = (n_wg + 255) / 256;
+    const bool filled = 10 * n_wg > (one_wave && !d64 && keys < 4096 ? 7 : 9) * 256 * rounds;
+    if (n_wg > 512) {
+        const int64_t d128 = one_wave ? 1024 : n_wg >= 2048 ? 256 : filled && n_wg < 1024 ? 768 : 384;
+        return keys >= (d64 ? (one_wave ? 256 : 192) : d128);
+    }
+    if (filled) {
+        return false;
+    }
+    return rounds > 1 ? keys >= (d64 ? 256 : 320) : keys >= even && score_bytes(a) <= (int64_t)320 << 20;
+}
+
 int int8_decode_plan(const AttnArgs& a, CallPlan& plan, std::string& err) {
     plan = CallPlan{CallForm::kDecode, 0, (size_t)score_bytes(a)};
     SplitKPlan splits;

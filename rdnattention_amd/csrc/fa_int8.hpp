@@ -96,8 +96,9 @@ int launch_int8_f16pv(const Int8Params& p, int head_dim, bool scores, Int8Mode m
                       hipStream_t stream, std::string& err);
 
 // Split-K decode (fa_fwd_int8_decode.hip): (Hq / Hkv) * Sq <= 32, head_dim 64
-// or 128.
+// or 128; and whether a call takes it.
 bool int8_splitk_supported(const AttnArgs& a);
+bool int8_prefer_splitk(const AttnArgs& a);
 int fwd_int8_splitk(const AttnArgs& a, const Int8Params& p, hipStream_t stream, std::string& err);
 struct CallPlan;
 int int8_decode_plan(const AttnArgs& a, CallPlan& plan, std::string& err);

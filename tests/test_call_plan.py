@@ -36,3 +36,23 @@ def test_int8_decode_scratch(case):
     assert scores <= 1 << 30
     partials = splits * b * hkv * m * (d + 2) * 4 if splits > 1 else 0  # with a device
     assert scratch == scores + partials
+
+
+# b, hkv, query heads per kv head, rows, sk, d: the calls that were slower on the
+# decode kernels than on the prefill kernels, and their neighbours that are not
+@pytest.mark.parametrize("b,hkv,ratio,sq,sk,d,decode", [
+    (1, 8, 1, 1, 64, 64, False), (1, 8, 4, 1, 384, 128, False), (1, 8, 4, 1, 600, 64, True), (1, 8, 4, 1, 512, 128, True),
+    (64, 8, 1, 1, 64, 128, False), (64, 8, 1, 1, 256, 128, True), (512, 8, 1, 1, 1, 64, True),
+    (128, 8, 4, 2, 1, 128, False), (128, 8, 4, 4, 64, 64, False), (128, 8, 4, 4, 256, 64, True),
+    (32, 8, 4, 8, 512, 128, False), (32, 8, 1, 32, 2048, 64, False), (16, 8, 4, 8, 2048, 128, True),
+    (40, 8, 4, 2, 448, 64, True), (24, 8, 4, 4, 16384, 64, False), (16, 8, 4, 4, 16384, 64, True),
+    (128, 8, 1, 32, 512, 128, False), (512, 8, 1, 32, 1024, 128, True), (24, 8, 8, 1, 1, 128, False),
+    (80, 8, 8, 1, 1, 128, True)])
+def test_int8_decode_line(b, hkv, ratio, sq, sk, d, decode):
+    assert (call_plan(True, b, ratio * hkv, hkv, sq, sk, d)[0] == DECODE) == decode
+
+
+def test_int8_decode_line_counts_visible_keys():
+    """A window that leaves few keys of a long cache."""
+    assert call_plan(True, 1, 32, 8, 1, 100000, 128, True, 200)[0] != DECODE
+    assert call_plan(True, 1, 32, 8, 1, 100000, 128, True, 2000)[0] == DECODE
