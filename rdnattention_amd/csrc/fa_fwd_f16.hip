@@ -957,17 +957,22 @@ static double longest_walk(const AttnArgs& a, int rows, int tiles_per_step, doub
     return longest;
 }
 
-bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us, int chunk) {
+bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us, int chunk, int max_half_wg,
+                       double half_margin) {
     // Twice as many row tiles of half as many steps, where the longest row
     // tile of a launch sets its time: up to two row tiles per CU.  A row tile
     // takes about 5 us beside its steps.
     const int rows = 32 * kPPWaves / prefill_group(a);
     const int head_groups = a.B * (a.Hq / prefill_group(a));
-    if (a.Sk <= 2 * kBN || (int64_t)((a.Sq + rows - 1) / rows) * head_groups > 512) {
+    const int64_t n_wg = (int64_t)((a.Sq + rows - 1) / rows) * head_groups;
+    // Rows that fill at most half a row tile: as many workgroups as without, whose
+    // second group had no rows and left each step shorter than the model's.
+    const bool half = a.Sq <= rows / 2;
+    if (a.Sk <= 2 * kBN || n_wg > (half ? max_half_wg : 512)) {
         return false;
     }
     return step_us * longest_walk(a, rows / 2, 2, 5.0 / step_us, chunk) <
-           0.97 * tile_us * longest_walk(a, rows, 1, 5.0 / tile_us, chunk);
+           (half ? half_margin : 0.97) * tile_us * longest_walk(a, rows, 1, 5.0 / tile_us, chunk);
 }
 
 // Whether the two groups of a workgroup take the key tiles in turn (D <= 128).
@@ -975,10 +980,15 @@ bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us, int ch
 // one.  Measured, us a call, whole against alternating (Hq 32 Hkv 8, causal): B1
 // S1024 D128 29.0 / 20.6, D64 22.5 / 15.8; B1 S2048 D128 55 / 45; B2 S1024 D128
 // 31.8 / 30.5; and where the rule keeps whole row tiles: B1 S2048 D128 not
-// causal 71 / 79, B2 S1500 49 / 58, B2 S2048 78 / 92.
+// causal 71 / 79, B2 S1500 49 / 58, B2 S2048 78 / 92.  Of rows that fill
+// half a tile it does not pay at D = 32, where two workgroups share a CU, with more
+// than 256 (512 kv heads of 33 to 128 rows, Sk 400 13.6 / 16.6), nor at D = 128 with
+// more than 128, which stream their own K and V (256 kv heads of 64 rows, Sk 2048
+// 52 / 57, Sk 512 18.7 / 20.1).
 static bool f16_prefill_alternate(const AttnArgs& a, int chunk) {
     const double tile_us = 0.4 + a.D / 128.0;
-    return a.D <= 128 && prefill_alternate(a, tile_us, 1.4 * tile_us, chunk);
+    const int max_half_wg = a.D == 32 ? 256 : a.D == 128 ? 128 : 512;
+    return a.D <= 128 && prefill_alternate(a, tile_us, 1.4 * tile_us, chunk, max_half_wg, 0.95);
 }
 
 static int f16_hg_chunk(const AttnArgs& a) {

@@ -875,8 +875,9 @@ static CallPlan int8_prefill_plan(const AttnArgs& a, int hg_chunk, size_t max_pa
     // against alternating (Hq 32 Hkv 8): B1 S1024 causal D64 31.5 / 21.5, D128
     // 37.0 / 25.8; B1 S2048 causal D64 56 / 40, D128 67 / 51; B2 S512 D128 22.3
     // / 17.4; and where the rule keeps whole row tiles: B1 S2048 D128 not causal
-    // 69 / 83, B2 S2048 causal 79 / 98
-    if (prefill_alternate(a, tile_us, 1.3 * tile_us, hg_chunk)) {
+    // 69 / 83, B2 S2048 causal 79 / 98, 512 kv heads of 33 rows Sk 130 D128 19.3 /
+    // 20.1
+    if (prefill_alternate(a, tile_us, 1.3 * tile_us, hg_chunk, 512, 0.9)) {
         plan.form = CallForm::kAlternate;
     }
     return plan;

@@ -139,8 +139,11 @@ int prefill_splits(const AttnArgs& a, int wg_rows, double tile_us, double altern
 
 // Whether a prefill launch of the ping-pong kernels (256 rows of G heads per
 // workgroup, tile_us per 64-key tile, hg_chunk = chunk) ends sooner with 128
-// rows and two tiles per step of step_us.
-bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us, int chunk);
+// rows and two tiles per step of step_us.  Where the rows fill at most half a row
+// tile: of up to max_half_wg workgroups, when its modelled time is less than
+// half_margin of the other's.
+bool prefill_alternate(const AttnArgs& a, double tile_us, double step_us, int chunk, int max_half_wg,
+                       double half_margin);
 
 // The kernels a call takes: prefill by whole row tiles, with split keys, with the
 // wave groups taking the key tiles in turn, or split-K decode; the key splits,

@@ -56,3 +56,15 @@ def test_int8_decode_line_counts_visible_keys():
     """A window that leaves few keys of a long cache."""
     assert call_plan(True, 1, 32, 8, 1, 100000, 128, True, 200)[0] != DECODE
     assert call_plan(True, 1, 32, 8, 1, 100000, 128, True, 2000)[0] == DECODE
+
+
+# int8, b, hq, hkv, sq, sk, d
+@pytest.mark.parametrize("case,form", [
+    ((False, 64, 8, 8, 64, 400, 32), WHOLE), ((False, 32, 8, 8, 64, 400, 32), ALTERNATE),
+    ((False, 32, 8, 8, 64, 512, 128), WHOLE), ((False, 16, 8, 8, 64, 512, 128), ALTERNATE),
+    ((False, 32, 32, 8, 9, 400, 128), WHOLE), ((False, 64, 8, 8, 64, 1024, 64), ALTERNATE),
+    ((True, 64, 8, 8, 33, 130, 128), WHOLE), ((True, 64, 8, 8, 33, 400, 128), ALTERNATE)])
+def test_alternate_line(case, form):
+    """Rows that fill at most half a row tile, and D = 32, whose workgroups share a
+    CU: where alternating groups were slower than whole row tiles, and not."""
+    assert call_plan(*case)[0] == form
