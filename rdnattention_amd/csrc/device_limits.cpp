@@ -1,4 +1,4 @@
-// Device occupancy queries for the persistent kernels.
+// Device queries for the persistent kernels and the split-K plans.
 #include "fa_internal.hpp"
 
 #include <hip/hip_runtime.h>
@@ -9,9 +9,9 @@
 
 namespace rdna_amd {
 
-int64_t resident_workgroups(const void* kernel, int threads, std::string& err) {
+int64_t resident_workgroups(const void* kernel, int threads, std::string& err, int* compute_units) {
     static std::mutex mu;
-    static std::map<std::pair<int, const void*>, int64_t> cache; // guarded by mu
+    static std::map<std::pair<int, const void*>, std::pair<int, int>> cache; // CUs, workgroups each; guarded by mu
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) {
@@ -22,7 +22,10 @@ int64_t resident_workgroups(const void* kernel, int threads, std::string& err) {
         std::lock_guard<std::mutex> lock(mu);
         auto it = cache.find({dev, kernel});
         if (it != cache.end()) {
-            return it->second;
+            if (compute_units != nullptr) {
+                *compute_units = it->second.first;
+            }
+            return (int64_t)it->second.first * it->second.second;
         }
     }
     int cus = 0, per_cu = 0;
@@ -38,10 +41,12 @@ int64_t resident_workgroups(const void* kernel, int threads, std::string& err) {
         err = "kernel does not fit on a compute unit";
         return -1;
     }
-    const int64_t n = (int64_t)cus * per_cu;
+    if (compute_units != nullptr) {
+        *compute_units = cus;
+    }
     std::lock_guard<std::mutex> lock(mu);
-    cache[{dev, kernel}] = n;
-    return n;
+    cache[{dev, kernel}] = {cus, per_cu};
+    return (int64_t)cus * per_cu;
 }
 
 } // namespace rdna_amd

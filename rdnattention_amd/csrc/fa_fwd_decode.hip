@@ -359,8 +359,8 @@ size_t splitk_partial_bytes(const AttnArgs& a, int splits) {
     return splits <= 1 ? 0 : (size_t)a.B * a.Hq * a.Sq * splits * (a.D + 2) * sizeof(float);
 }
 
-SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
-                           size_t max_partials, int64_t max_keys) {
+SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t max_keys, size_t max_partials,
+                           const std::function<double(int, int64_t)>& time_us) {
     // The keys that some row sees, from a tile boundary on, are dealt to the
     // splits in multiples of `round` keys.
     const MaskSpec mask{a.Sk, a.Sk - a.Sq, a.causal ? 1 : 0, a.window > 0 ? a.window : 0};
@@ -372,36 +372,26 @@ SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_b
         return plan; // one split, which writes zeros
     }
     plan.key0 = lo / tile * tile;
-    const int64_t keys = (int64_t)hi + 1 - plan.key0;
-    const int64_t n_bkv = (int64_t)a.B * a.Hkv;
-    // Splits: the least modelled time over 1 .. 256.  A launch runs in rounds
-    // of `resident` workgroups (one per CU at D = 128); a workgroup takes
-    // about 2 us beside its keys and streams at most 40 KB/us (measured: 40
-    // with 128 workgroups, 48 to 50 with 8 to 64, D = 128 to 256), all
-    // together 6.8 TB/s; the merge, a second launch, adds about 5 us.  So a
-    // count just above a whole round (264 workgroups for 24 kv heads) is never
-    // taken, which rounding resident / n_bkv up did.  Measured, us a call,
-    // against the count chosen: n_bkv 8, Sk 512: 10.8 (1, chosen), 13.9 (2);
-    // D = 64, 8, 768: 8.4 (1, chosen), 12.4 (3); n_bkv 128, Sk 32768: 420 (1), 317 (2, chosen), 349 (3);
-    // 32, 4096: 23 (4), 19.2 (8, chosen), 25.7 (16); 8, 32768: 37 (16),
-    // 29.7 (32, chosen), 33.7 (64); D = 64, 256, 2048: 27.6 (1, chosen), 33 (2).
-    const int64_t rounds_of_keys = (keys + round - 1) / round;
+    const int keys = hi + 1 - plan.key0;
+    const int units = (keys + round - 1) / round;
     double best = INFINITY;
-    for (int64_t s = 1; s <= std::min<int64_t>(rounds_of_keys, kMaxSplits); s++) {
-        const int64_t kps = (rounds_of_keys + s - 1) / s * round;
-        if (kps > max_keys || kps * (s - 1) >= keys || region_bytes(splitk_partial_bytes(a, (int)s)) > max_partials) {
-            continue; // too many keys for a split, the last one empty, or the partials too large
+    // over 1 .. kMaxSplits, the smallest count of each size (another one has an
+    // empty split)
+    for (int s = 1; s <= std::min(units, kMaxSplits);) {
+        const int per = (units + s - 1) / s;
+        const int64_t kps = (int64_t)per * round;
+        if (kps <= max_keys && region_bytes(splitk_partial_bytes(a, s)) <= max_partials) {
+            const double t = time_us(s, std::min<int64_t>(kps, keys));
+            if (t < best) {
+                best = t;
+                plan.splits = s;
+                plan.keys_per_split = (int)kps;
+            }
         }
-        const int64_t wgs = n_bkv * s;
-        const int64_t waves_of_wgs = (wgs + resident - 1) / resident;
-        const double rate = std::min(40e3, 6.8e6 / (double)std::min(wgs, resident)); // bytes per us
-        const double t = (double)waves_of_wgs * (2.0 + (double)(std::min(kps, keys) * key_bytes) / rate) +
-                         (s > 1 ? 5.0 : 0.0);
-        if (t < best) {
-            best = t;
-            plan.splits = (int)s;
-            plan.keys_per_split = (int)kps;
+        if (per == 1) {
+            break;
         }
+        s = (units + per - 2) / (per - 1);
     }
     return plan;
 }
@@ -409,16 +399,38 @@ SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_b
 int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::string& err) {
     return for_dim(a.D, [&](auto d) {
         using C = DecCfg<decltype(d)::value>;
+        int cus = 0;
         const int64_t resident = resident_workgroups(
-            reinterpret_cast<const void*>(&fa_fwd_f16_decode<decltype(d)::value>), C::THREADS, err);
+            reinterpret_cast<const void*>(&fa_fwd_f16_decode<decltype(d)::value>), C::THREADS, err, &cus);
         if (resident <= 0) {
             return -1;
         }
-        // Half rounds of the waves: whole ones leave the last split short (64
-        // kv heads, Sk 6244, D = 128: 3 x 1792 keys and 868, 39.9 us against
-        // 38.9 of 3 x 1664 and 1252; 128 of 2303: 30.4 / 29.7); single tiles
-        // measure the same as these.
-        plan = splitk_plan_for(a, kDecTile, C::WAVES / 2 * kDecTile, 2 * C::RB, resident, max_partials);
+        // A launch runs in rounds of `resident` workgroups, the last with what is
+        // left.  A round takes 3 us and its bytes: those of the CU with the most
+        // workgroups at 34 KB/us (24 at D = 32, 30 at 64, 36 above 192), and of all at 6.8
+        // TB/s.  So 192 workgroups (64 heads of 8198 keys, D = 128, 3 splits: 54.3 us)
+        // are no match for 256 (4: 50.8), and at D = 64, where two share a CU, 160
+        // heads of 7166 keys take 66 us with one split, 77 with two, 55 with three
+        // and 65 with four.  The merge, a second launch, adds about 9 us, 15 ns per
+        // split and the partials, written and read, at 2.5 MB/us.  Fitted to 520
+        // calls (8 to 512 kv heads, 512 to 16384 keys, one and four rows, caches
+        // beyond the last-level cache) over all splits: 1.1 % above the best of them
+        // on average with a head's rows in one block (36 KB/us would fit best), 2.6
+        // % with the rows apart, as in a [B, S, 2, H, D] cache (26 to 31); the bits do
+        // not depend on the strides.  A rate of 40 KB/us per workgroup and no CUs: 2.3
+        // and 4.8 %.  Splits of single tiles: rounds of the waves leave the last one
+        // short.
+        const double cu_rate = a.D <= 32 ? 24e3 : a.D <= 64 ? 30e3 : a.D <= 192 ? 34e3 : 36e3;
+        const int64_t n_bkv = (int64_t)a.B * a.Hkv;
+        plan = splitk_plan_for(a, kDecTile, kDecTile, INT32_MAX, max_partials, [&](int s, int64_t keys) {
+            const double bytes = (double)(keys * 2 * C::RB);
+            auto round_us = [&](int64_t n) {
+                return 3.0 + std::max((double)((n + cus - 1) / cus) * bytes / cu_rate, (double)n * bytes / 6.8e6);
+            };
+            const int64_t rounds = n_bkv * s / resident, rest = n_bkv * s % resident;
+            return (double)rounds * round_us(resident) + (rest > 0 ? round_us(rest) : 0.0) +
+                   (s > 1 ? 9.0 + 0.015 * s + 2.0 * (double)splitk_partial_bytes(a, s) / 2.5e6 : 0.0);
+        });
         return 0;
     });
 }

@@ -482,7 +482,16 @@ int int8_decode_splits(const AttnArgs& a, SplitKPlan& plan, std::string& err) {
     if (resident <= 0) {
         return -1;
     }
-    plan = splitk_plan_for(a, kI8BN, kI8DecWaves * kI8BN, 2 * D, resident, SIZE_MAX, TCfg<TC>::MAX_TILES * kI8BN);
+    // rounds of `resident` workgroups, each 2 us and its keys at 40 KB/us, all
+    // together 6.8 TB/s; 5 us for the merge
+    const int64_t n_bkv = (int64_t)a.B * a.Hkv;
+    plan = splitk_plan_for(
+        a, kI8BN, kI8DecWaves * kI8BN, TCfg<TC>::MAX_TILES * kI8BN, SIZE_MAX, [&](int s, int64_t keys) {
+            const int64_t wgs = n_bkv * s;
+            const double rate = std::min(40e3, 6.8e6 / (double)std::min(wgs, resident));
+            return (double)((wgs + resident - 1) / resident) * (2.0 + (double)(keys * 2 * D) / rate) +
+                   (s > 1 ? 5.0 : 0.0);
+        });
     return 0;
 }
 

@@ -7,6 +7,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <functional>
 #include <string>
 
 namespace rdna_amd {
@@ -105,7 +106,7 @@ class KernelTimerGuard {
 // Workgroups of `kernel` (launched with `threads` threads and no dynamic LDS)
 // that the current device holds at once: compute units x workgroups per
 // compute unit. Cached per device and kernel; <= 0 with `err` set on failure.
-int64_t resident_workgroups(const void* kernel, int threads, std::string& err);
+int64_t resident_workgroups(const void* kernel, int threads, std::string& err, int* compute_units = nullptr);
 
 // Launchers.  `region`, when given, supplies every scratch buffer.
 int fwd_f16_prefill(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err,
@@ -124,10 +125,10 @@ struct SplitKPlan {
 int splitk_plan(const AttnArgs& a, size_t max_partials, SplitKPlan& plan, std::string& err);
 
 // The same for any split-K kernel: `tile` keys per wave tile, the splits
-// multiples of `round` keys, key_bytes of K and V per key, `resident` workgroups
-// on the device, at most max_keys keys per split.
-SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t key_bytes, int64_t resident,
-                           size_t max_partials, int64_t max_keys = INT32_MAX);
+// multiples of `round` keys and at most max_keys of them, the least time_us(splits,
+// keys of the largest).
+SplitKPlan splitk_plan_for(const AttnArgs& a, int tile, int round, int64_t max_keys, size_t max_partials,
+                           const std::function<double(int, int64_t)>& time_us);
 
 // Key splits of a prefill call whose workgroups hold wg_rows rows (of G heads)
 // and take tile_us per 64-key tile (split_tile_us over `launches` launches where

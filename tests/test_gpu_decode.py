@@ -11,7 +11,7 @@ import pytest
 import torch
 
 import oracle
-from tests.gpu_util import assert_f16_parity, forward_raw, log, reference_f16, seeded_inputs
+from tests.gpu_util import DECODE, assert_f16_parity, call_plan, forward_raw, log, reference_f16, seeded_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -267,3 +267,15 @@ def test_more_kv_heads_than_a_grid_dimension(gpu, int8, d, sk):
     assert torch.equal(outs[1], outs[1][:1].expand_as(outs[1]))
     diff = (outs[1][0].float() - outs[0][0].float()).abs().max().item()
     assert diff <= 2e-3, diff  # another order of the sums; the same INT8 P
+
+
+@pytest.mark.parametrize("d,b,sk,lo,hi", [
+    (128, 8, 8198, 4, 4), (128, 16, 2082, 1, 2), (128, 16, 32768, 2, 2), (128, 1, 512, 1, 1), (64, 20, 7166, 3, 3),
+    (64, 12, 7447, 5, 5), (128, 3, 4000, 8, 10), (256, 8, 6001, 3, 4)])
+def test_decode_splits(gpu, d, b, sk, lo, hi):
+    """Eight kv heads per batch entry on 256 CUs: as many splits as fill whole rounds
+    of workgroups, or every CU alike."""
+    form, splits, scratch = call_plan(False, b, 64 if d > 192 else 8, 8, 1, sk, d)
+    log(f"[decode splits] d{d} b{b} sk{sk}: {splits}")
+    assert form == DECODE and lo <= splits <= hi
+    assert scratch == (splits * b * (64 if d > 192 else 8) * (d + 2) * 4 if splits > 1 else 0)
