@@ -476,10 +476,6 @@ int splitk_finish(const AttnArgs& a, const SplitRows& r, hipStream_t stream, std
 }
 
 int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::string& err, ScratchRegion* region) {
-    if (!splitk_built(a)) {
-        err = "split-K path needs head_dim in {32, 64, 128} and (num_heads / num_kv_heads) * seq_len <= 32";
-        return -1;
-    }
     DecodeParams p{};
     p.q = static_cast<const _Float16*>(a.q);
     p.k = static_cast<const _Float16*>(a.k);

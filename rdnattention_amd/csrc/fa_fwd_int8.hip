@@ -67,7 +67,6 @@ namespace rdna_amd {
 
 namespace {
 
-typedef int i2 __attribute__((ext_vector_type(2)));
 
 constexpr int kI8Slots = 4;                  // K/V tile slots in LDS (DMAs run two tiles ahead)
 constexpr int kI8OpDepth = 4;                // LDS operands in flight in the MFMA phase
@@ -103,18 +102,6 @@ struct I8Cfg {
 // The swizzle depends only on row bits 2-3, so rows 16 and 32 apart share it.
 __host__ __device__ constexpr int i8_swz(int r) {
     return (r >> 2) & 3;
-}
-
-// ds_read_b64_tr_b8 (gfx950 LDS transpose read).  Within each 16-lane group,
-// lane i receives as byte k the byte (i % 8) of the 8-byte word whose address
-// lane 2k + i / 8 supplies: if lane j points at row j / 2, bytes 8 (j % 2) ..
-// +7 of an 8-row x 16-byte block, lane i gets column i of the block, the
-// eight rows' bytes in order.
-__device__ __forceinline__ i2 lds_read_tr8(const int8_t* p) {
-    typedef __attribute__((address_space(3))) i2 lds_i2;
-    const auto* lp = reinterpret_cast<const __attribute__((address_space(3))) char*>(
-        (uint32_t)reinterpret_cast<uintptr_t>(p));
-    return __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i2*)lp);
 }
 
 __device__ __forceinline__ i32x4_t uniform_rsrc(i32x4_t r) {

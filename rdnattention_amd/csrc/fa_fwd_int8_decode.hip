@@ -117,32 +117,6 @@ struct TileOffsets {
     }
 };
 
-// ds_read_b64_tr_b8: within each 16-lane group, lane i receives as byte k
-// byte i % 8 of the 8-byte word that lane 2k + i / 8 addresses; with lane j at
-// row j / 2, columns 8 (j % 2) .. +7 of an 8 x 16 block, lane i gets column i.
-typedef int i2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ i2 lds_read_tr8(uint32_t lds_byte_addr) {
-    typedef int i2_raw __attribute__((__vector_size__(2 * sizeof(int))));
-    typedef __attribute__((address_space(3))) i2_raw lds_i2;
-    i2_raw r = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-        (lds_i2*)reinterpret_cast<const __attribute__((address_space(3))) char*>(lds_byte_addr));
-    return __builtin_bit_cast(i2, r);
-}
-
-// 8 signed bytes -> fp16 (exact): flipping the sign bit gives u = v + 128, a
-// byte permute against 0x64 makes the fp16 number 1024 + u, minus 1152 is v
-__device__ __forceinline__ h8 widen8(i2 w) {
-    const h2 off = {(_Float16)1152.0f, (_Float16)1152.0f};
-    h2 r[4];
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-        const uint32_t u = (uint32_t)w[c] ^ 0x80808080u;
-        r[2 * c] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) - off;
-        r[2 * c + 1] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) - off;
-    }
-    return h8{r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]};
-}
-
 // 8 signed bytes of 8 keys with the scales lo (keys 0..3) and hi (4..7):
 // fp16(sat(v * vs)), as the prefill kernel stages a per-token-scaled V row
 __device__ __forceinline__ h8 widen8_scaled(i2 w, f4 lo, f4 hi) {

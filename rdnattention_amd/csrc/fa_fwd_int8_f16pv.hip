@@ -80,7 +80,6 @@ namespace rdna_amd {
 namespace {
 
 typedef int8_t i8x8 __attribute__((ext_vector_type(8)));
-typedef int i2 __attribute__((ext_vector_type(2)));
 
 template <int D>
 struct I8Cfg {
@@ -114,25 +113,10 @@ __device__ __forceinline__ i4 buffer_load_i4(__amdgpu_buffer_rsrc_t r, uint32_t 
     return __builtin_bit_cast(i4, x);
 }
 
-// 16 signed bytes -> two h8 (exact: every int8 is an fp16 integer).  Flipping
-// the sign bit gives u = v + 128 as an unsigned byte; a byte permute pairs each
-// u with the high byte 0x64, i.e. the fp16 value 1024 + u (exact: the ulp in
-// [1024, 2048) is 1), and one packed subtract of 1152 leaves v.  Five VALU
-// instructions per 4 values.
+// 16 signed bytes -> two h8
 __device__ __forceinline__ void i8x16_to_h8x2(i4 w, h8& lo, h8& hi) {
-    const h2 off = {(_Float16)1152.0f, (_Float16)1152.0f};
-    h2 r[8];
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const uint32_t u = (uint32_t)w[c] ^ 0x80808080u;
-        // byte selects: 0-3 pick bytes of u, 4 picks byte 0 of 0x64646464
-        const uint32_t p01 = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u);
-        const uint32_t p23 = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
-        r[2 * c] = __builtin_bit_cast(h2, p01) - off;
-        r[2 * c + 1] = __builtin_bit_cast(h2, p23) - off;
-    }
-    lo = {r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]};
-    hi = {r[4][0], r[4][1], r[5][0], r[5][1], r[6][0], r[6][1], r[7][0], r[7][1]};
+    lo = widen8(i2{w[0], w[1]});
+    hi = widen8(i2{w[2], w[3]});
 }
 
 // 16 signed bytes of one V row -> two h8 of fp16(sat(v * vs)): the product in

@@ -35,6 +35,41 @@ __device__ __forceinline__ float int8_exp_offset(float m) {
     return (kLog2Of127 - mc) - (a >= 32768.0f ? a * 0x1p-21f : 0.0f);
 }
 
+typedef int i2 __attribute__((ext_vector_type(2)));
+
+// ds_read_b64_tr_b8 (gfx950 LDS transpose read).  Within each 16-lane group,
+// lane i receives as byte k the byte (i % 8) of the 8-byte word whose address
+// lane 2k + i / 8 supplies: if lane j points at row j / 2, bytes 8 (j % 2) ..
+// +7 of an 8-row x 16-byte block, lane i gets column i of the block, the
+// eight rows' bytes in order.
+__device__ __forceinline__ i2 lds_read_tr8(uint32_t lds_byte_addr) {
+    typedef __attribute__((address_space(3))) i2 lds_i2;
+    const auto* lp = reinterpret_cast<const __attribute__((address_space(3))) char*>(
+        lds_byte_addr);
+    return __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i2*)lp);
+}
+__device__ __forceinline__ i2 lds_read_tr8(const int8_t* p) {
+    return lds_read_tr8((uint32_t)reinterpret_cast<uintptr_t>(p));
+}
+
+// 8 signed bytes -> fp16 (exact: every int8 is an fp16 integer).  Flipping the
+// sign bit gives u = v + 128 as an unsigned byte; a byte permute pairs each u with
+// the high byte 0x64, i.e. the fp16 value 1024 + u (exact: the ulp in [1024, 2048)
+// is 1), and one packed subtract of 1152 leaves v.  Five VALU instructions per 4
+// values.
+__device__ __forceinline__ h8 widen8(i2 w) {
+    const h2 off = {(_Float16)1152.0f, (_Float16)1152.0f};
+    h2 r[4];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const uint32_t u = (uint32_t)w[c] ^ 0x80808080u;
+        // byte selects: 0-3 pick bytes of u, 4 picks byte 0 of 0x64646464
+        r[2 * c] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) - off;
+        r[2 * c + 1] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) - off;
+    }
+    return h8{r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]};
+}
+
 struct Int8Params {
     const int8_t* q;
     const int8_t* k;
