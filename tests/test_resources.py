@@ -28,8 +28,17 @@ WAVES_PER_SIMD = {
     "fa_fwd_int8_f16pv": 2,
     "fa_fwd_f16_kpair": 2,
     "fa_fwd_f16_dpair": 2,
-    "fa_fwd_f16_decode": 1,
+    "fa_fwd_f16_decode": 1,  # head dims 224 and 256; see DECODE_WAVES_PER_SIMD
+    "fa_fwd_f16_pp_split": 2,
+    "fa_fwd_f16_pp_alt": 2,
+    "fa_fwd_f16_kpair_split": 2,
+    "fa_fwd_int8_split": 2,
+    "fa_fwd_int8_f16pv_split": 2,
+    "fa_int8_decode_scores": 2,
+    "fa_int8_decode_pv": 2,
 }
+# eight waves (six at 192) per workgroup; two workgroups to a CU at 64, three at 32
+DECODE_WAVES_PER_SIMD = {32: 6, 64: 4, 96: 2, 128: 2, 160: 2, 192: 2, 224: 1, 256: 1}
 
 
 @pytest.fixture(scope="module")
@@ -59,12 +68,20 @@ def test_lds_within_gfx950_limit(kernels):
 def test_occupancy_fits_the_workgroup(kernels):
     checked = 0
     for k in kernels:
-        need = WAVES_PER_SIMD.get(_demangled_base(k["kernel"]))
+        base = _demangled_base(k["kernel"])
+        need = WAVES_PER_SIMD.get(base)
+        if base == "fa_fwd_f16_decode":
+            need = DECODE_WAVES_PER_SIMD[int(re.search(r"decodeILi(\d+)E", k["kernel"]).group(1))]
+        if base in ("fa_int8_decode_scores", "fa_int8_decode_pv") and "ELi4E" in k["kernel"]:
+            # two workgroups to a CU, but for the per-token V scale at head_dim 128
+            need = 2 if "pvILi128ELb1E" in k["kernel"] else 4
         if need is not None:
             assert k["waves_per_simd"] >= need, (k["kernel"], k["waves_per_simd"], need)
             checked += 1
     # pp 4, kpair 4, dpair 8, decode 3, int8 3 + int8_f16pv 3 (+ 2 score-export instantiations)
     assert checked >= 4 + 4 + 3 + 5 + 3 + 4
+    # every attention kernel is held to one of the lines above
+    assert checked == sum("fa_" in _demangled_base(k["kernel"]) and "combine" not in k["kernel"] for k in kernels)
 
 
 def test_every_dispatched_head_dim_is_compiled(kernels):
@@ -79,20 +96,27 @@ def test_every_dispatched_head_dim_is_compiled(kernels):
         assert has("fa_fwd_f16_kpair", d), d
     for d in range(288, 513, 32):
         assert has("fa_fwd_f16_dpair", d), d
-    for d in (32, 64, 128):
+    for d in range(32, 257, 32):
         assert has("fa_fwd_f16_decode", d), d
+    for d in (32, 64, 96, 128):
+        assert has("fa_fwd_f16_pp_split", d) and has("fa_fwd_f16_pp_alt", d), d
+    for d in (160, 192, 224, 256):
+        assert has("fa_fwd_f16_kpair_split", d), d
     # INT8: head_dim 64 with both GEMMs on int8 MFMA, 128 (and the per-token V
     # scale) with P V on fp16 MFMA
     assert has("fa_fwd_int8", 64)
+    assert has("fa_fwd_int8_split", 64)
     for d in (64, 128):
         assert has("fa_fwd_int8_f16pv", d), d
+        assert has("fa_fwd_int8_f16pv_split", d), d
+        assert has("fa_int8_decode_scores", d) and has("fa_int8_decode_pv", d), d
     for frag in ("rope_rotate_rows", "fa_decode_combine", "quant_rows_kernel", "col_max_kernel",
                  "quant_cols_kernel"):
         assert any(frag in n for n in names), frag
 
 
 ATTENTION_SOURCES = ["fa_fwd_f16.hip", "fa_fwd_f16_kpair.hip", "fa_fwd_f16_dpair.hip", "fa_fwd_int8.hip",
-                     "fa_fwd_int8_f16pv.hip", "fa_fwd_decode.hip"]
+                     "fa_fwd_int8_f16pv.hip", "fa_fwd_decode.hip", "fa_fwd_int8_decode.hip"]
 
 
 def test_no_waterfall_loops(tmp_path):
