@@ -157,8 +157,9 @@ def test_auto_decode_vs_oracle(gpu, oracle_lib, case):
 
 
 # d, b, hq, hkv, sq, sk, causal, window, rope: prefill launches too small for
-# the CUs, whose keys are split (every head dim; one and several row tiles,
-# rows without keys, splits that end short or empty, a window)
+# the CUs, whose keys are split (every head dim; one and several row tiles, splits
+# that end short or empty, a window) or, of two, whose groups alternate (a window,
+# rows without keys; those under split keys: test_gpu_forms.py)
 SPLIT_PREFILL_CASES = [(d, 1, 8, 2, 70, 1500, True, -1, False) for d in range(32, 257, 32)] + [
     (128, 1, 8, 2, 257, 5000, True, -1, True),
     (128, 1, 4, 4, 33, 2049, False, -1, False),

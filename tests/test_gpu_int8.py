@@ -423,8 +423,10 @@ def test_int8_quantised_p_against_oracle_integers(gpu, oracle_lib, d, per_token)
     assert n_diff <= 2e-5 * diff.size
 
 
-# b, hq, hkv, sq, sk, d, causal, window, scales: the split-K decode kernel at
-# the edges of its 64-key tiles, its rounds of eight of them and its 32 columns
+# b, hq, hkv, sq, sk, d, causal, window, scales: few rows per kv head, at the edges
+# of the decode kernel's 64-key tiles, its rounds of eight of them and its 32
+# columns (so few kv heads go to the prefill kernels below about 500 keys; the
+# decode kernel's shortest caches: test_gpu_forms.py)
 DECODE_CASES = [(1, 8, 2, 1, sk, d, False, -1, sc) for d in (64, 128)
                 for sk, sc in ((1, "tensor"), (63, "token"), (65, "channel"), (512, "vtoken"), (513, "token"))] + [
     (2, 8, 8, 1, 3000, 128, False, -1, "channel"),
@@ -437,7 +439,8 @@ DECODE_CASES = [(1, 8, 2, 1, sk, d, False, -1, sc) for d in (64, 128)
 
 
 # more rows than one column block, too few workgroups for the CUs: the keys of
-# the prefill kernels are split
+# the prefill kernels are split (in the last two the groups alternate; a window
+# and rows without keys under split keys: test_gpu_forms.py)
 SPLIT_CASES = [(1, 8, 2, 70, 3000, d, True, -1, sc) for d in (64, 128)
                for sc in ("tensor", "token", "channel", "vtoken")] + [
     (1, 4, 4, 257, 2049, 128, False, -1, "token"),

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import oracle
-from tests.gpu_util import assert_f16_parity, lib, log, reference_f16, stream_ptr
+from tests.gpu_util import assert_f16_parity, call_plan, lib, log, reference_f16, stream_ptr
 
 pytestmark = pytest.mark.gpu
 
@@ -125,3 +125,32 @@ def test_noalloc_makes_no_allocation(gpu):
     cached = rdnattention.scratch_stats(dev)
     assert cached["entries"] == 2 and cached["allocations"] == before["allocations"] + 2, cached
     rdnattention.trim_scratch()
+
+
+# b, hq, hkv, sq, sk, d: RoPE calls whose rotated K leaves less of the array than
+# the partials of as many splits as the allocating entry point takes
+REDUCED = [(1, 32, 8, 1, 32640, 128), (1, 8, 2, 2, 131000, 128), (1, 32, 8, 256, 32000, 128),
+           (1, 16, 4, 130, 29000, 256), (1, 16, 2, 60, 65536, 256)]
+
+
+@pytest.mark.parametrize("case", REDUCED, ids=["b{}h{}kv{}q{}k{}d{}".format(*c) for c in REDUCED])
+def test_noalloc_takes_fewer_splits(gpu, case):
+    """Fewer splits, down to none, where their partials would not fit beside the K
+    copy: the allocating entry point's result within 1e-3 (another order of the
+    fp32 sums, one rounding to fp16), the same bits again."""
+    b, hq, hkv, sq, sk, d = case
+    copy = b * hkv * sk * d * 2
+    left = LIMIT - copy
+    full = call_plan(False, b, hq, hkv, sq, sk, d, True)
+    reduced = call_plan(False, b, hq, hkv, sq, sk, d, True, max_partials=left)
+    log(f"[noalloc] {case}: splits {full[1]} -> {reduced[1]}, {left} bytes left of the array")
+    assert 0 <= left and full[2] > left >= reduced[2] and reduced[1] < full[1]
+    q, k, v, cos, sin = _inputs(gpu, 98, b, hq, hkv, sq, sk, d, True, True)
+    outs = [torch.full_like(q, float("nan")) for _ in range(3)]
+    L = lib()
+    assert _call(L.rdna_attention_forward, q, k, v, outs[0], True, -1, cos, sin) == 0, L.rdna_get_error()
+    for o in outs[1:]:
+        assert _call(L.rdna_attention_forward_noalloc, q, k, v, o, True, -1, cos, sin) == 0, L.rdna_get_error()
+    torch.cuda.synchronize()
+    assert torch.equal(outs[1], outs[2])
+    assert (outs[0].float() - outs[1].float()).abs().max().item() <= 1e-3
