@@ -21,9 +21,10 @@
 // an eighth for 4 rows at D = 128).  Grid (splits, B * Hkv), the M = ratio *
 // Sq <= 32 rows of a kv head as the 32 columns of the MFMAs, eight waves on
 // interleaved 64-key tiles, one slot each, filled by non-temporal HBM -> LDS
-// DMA; two workgroups share a CU, so that some waves' tiles are in flight while
-// others compute.  V stays int8 in LDS; its operands come from
-// ds_read_b64_tr_b8 transpose reads and are widened to fp16 in registers.
+// DMA; two workgroups fit a CU (of TC = 4), and where a launch has as many some
+// waves' tiles are in flight while others compute.  V stays int8 in LDS; its
+// operands come from ds_read_b64_tr_b8 transpose reads and are widened to fp16 in
+// registers.
 //
 // B = 8 Hq = 32 Hkv = 8 Sk = 8192 D = 128 (136 MB): 16.9 us (scores),
 // 18.6 us (P V) and 4.2 us (merge), 43 us a call; on the prefill kernel 205.  One
