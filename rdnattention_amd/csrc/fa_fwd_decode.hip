@@ -59,6 +59,7 @@ struct DecodeParams {
     float q_sign;
     MaskSpec mask;
     int32_t rope_q;
+    int32_t pair_heads; // pairs of kv heads to one XCD (D % 64 == 32)
 };
 
 template <int D>
@@ -107,8 +108,20 @@ __global__ __launch_bounds__(DecCfg<D>::THREADS, DecCfg<D>::WAVES_PER_SIMD) void
     const int lane = tid & 63;
     const int l32 = lane & 31;
     const int g = lane >> 5;
-    const int split = blockIdx.x;
-    const int bkv = blockIdx.y;
+    int split = blockIdx.x;
+    int bkv = blockIdx.y;
+    if constexpr (D % 64 == 32) {
+        // Rows of 64, 192, ... bytes: in a [B, S, 2, H, D] cache two heads share every
+        // (or every third, ...) 128-byte line.  Pairs of heads go to one XCD, whose
+        // L2 then fetches it once: workgroup `id` runs on XCD id % 8, and its slot
+        // there is one head of pair slot / 2.
+        if (p.pair_heads != 0) {
+            const int id = bkv * (int)gridDim.x + split;
+            const int pair = (id & 7) + 8 * (id >> 4);
+            split = pair % (int)gridDim.x;
+            bkv = 2 * (pair / (int)gridDim.x) + ((id >> 3) & 1);
+        }
+    }
     const int b = bkv / p.Hkv;
     const int kvh = bkv - b * p.Hkv;
 
@@ -509,6 +522,12 @@ int fwd_f16_splitk(const AttnArgs& a, bool rope_q, hipStream_t stream, std::stri
     }
     p.keys_per_split = plan.keys_per_split;
     p.key0 = plan.key0;
+    // rows of neighbouring heads next to each other, an even number of heads, whole
+    // rounds of pairs over the 8 XCDs.  us a call without / with, one row per head:
+    // D = 32, 128 heads of 9027 keys 54.7 / 37.9, 64 of 13925 45.5 / 31.3; D = 96, 512
+    // of 4122 172 / 161; D = 160, 128 of 3000 51.8 / 47.9
+    p.pair_heads = (a.ks[1] == a.D || a.vs[1] == a.D) && a.Hkv % 2 == 0 &&
+                   (int64_t)a.B * a.Hkv * plan.splits % 16 == 0;
     if (rc != 0 ||
         for_dim(a.D, [&](auto d) { return launch_decode<decltype(d)::value>(p, a.B * a.Hkv, stream, err); }) != 0) {
         return -1;

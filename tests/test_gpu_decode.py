@@ -280,3 +280,28 @@ def test_decode_splits(gpu, d, b, sk, lo, hi):
     log(f"[decode splits] d{d} b{b} sk{sk}: {splits}")
     assert form == DECODE and lo <= splits <= hi
     assert scratch == (splits * b * (64 if d > 192 else 8) * (d + 2) * 4 if splits > 1 else 0)
+
+
+# d, b, hq, hkv, sk: rows that end inside a 128-byte line, whose heads go to the XCDs
+# in pairs where those fill whole rounds (the first two of each head dim) or not
+@pytest.mark.parametrize("case", [(d, *c) for d in (32, 96, 160, 224)
+                                  for c in ((2, 64, 8, 700), (4, 64, 4, 3000), (1, 64, 6, 900), (3, 20, 2, 2500))],
+                         ids=lambda c: "d{}b{}h{}kv{}k{}".format(*c))
+def test_decode_cache_views_every_head_dim(gpu, case):
+    """K/V as views of one [B, S, 2, Hkv, D] cache: the bits of contiguous tensors."""
+    d, b, hq, hkv, sk = case
+    hq = hq // hkv * hkv
+    assert call_plan(False, b, hq, hkv, 1, sk, d)[0] == DECODE
+    g = torch.Generator(device=gpu).manual_seed(91)
+    cache = torch.randn(b, sk, 2, hkv, d, generator=g, device=gpu).half()
+    q = torch.randn(b, hq, 1, d, generator=g, device=gpu).half()
+    k, v = cache[:, :, 0].transpose(1, 2), cache[:, :, 1].transpose(1, 2)
+    outs = [torch.full_like(q, float("nan")) for _ in range(2)]
+    assert forward_raw(q, k, v, outs[0]) == 0
+    assert forward_raw(q, k.contiguous(), v.contiguous(), outs[1]) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    kr = k.float().repeat_interleave(hq // hkv, dim=1).transpose(2, 3).contiguous()
+    vr = v.float().repeat_interleave(hq // hkv, dim=1)
+    ref = torch.matmul(torch.softmax(torch.matmul(q.float(), kr) * d ** -0.5, dim=-1), vr)
+    assert_f16_parity(outs[0].float().cpu().numpy(), ref.cpu().numpy(), "cache views")
